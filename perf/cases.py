@@ -1,0 +1,557 @@
+"""Performance cases: the work a user of this framework has it do, through its
+public Python entry points (how-mhd-kokkos_amd/howmhd.py), with the inputs, the
+compulsory work and, in plain torch float64, the exact results of each.
+
+Four kinds of case:
+
+  steps    the hydro loop between an initial state and an output: upload_q0,
+           init_faces, then (tstep, ssprk) a few times, and the download of
+           q(0).  Every precision form, 1-D to 3-D, both boundary conditions.
+  train    one optimiser step of the smoothness indicator: gradient of one
+           minibatch and Adam.
+  infer    the indicator's logits of a held-out set.
+  samples  the indicator's features and labels from every interface of a state.
+  restart  a run picked up from a checkpoint and written out again: upload of
+           q(0) and the faces, dt, diagnostics, download of both.
+"""
+from __future__ import annotations
+
+import math
+import sys
+from pathlib import Path
+
+import numpy as np
+import torch
+
+PKG = Path(__file__).resolve().parent.parent / "how-mhd-kokkos_amd"
+sys.path.insert(0, str(PKG))
+import howmhd as H  # noqa: E402
+
+WEIGHTS = PKG / "weights" / "indicator_mlp.txt"
+F64 = torch.float64
+
+
+# ------------------------------------------------------------------ the cases
+def _steps(name, problem, nx, ny, nz, form, steps, bc="periodic", cour=0.4):
+    return {"name": name, "kind": "steps", "problem": problem, "nx": nx, "ny": ny, "nz": nz, "form": form,
+            "steps": steps, "bc": bc, "cour": cour}
+
+
+def listed():
+    return [
+        # the reference's shock tube: 1-D, no CT, a grid that leaves most of the chip idle
+        _steps("brio_wu_800_fp64", "brio_wu", 800, 1, 1, "fp64", 20, bc="open", cour=0.8),
+        # the reference's example configuration (2-D, CT)
+        _steps("orszag_tang_128_fp64", "orszag_tang", 128, 128, 1, "fp64", 20, cour=0.8),
+        # the smallest grid of the convergence study (3-D, smooth)
+        _steps("cpaw_32_fp64", "cpaw3d", 32, 32, 32, "fp64", 20),
+        # the rotor of the indicator's evaluation: 2-D, FP32 with routing
+        _steps("rotor_512_fp32_indicator", "mhd_rotor", 512, 512, 1, "fp32+indicator", 20, bc="open"),
+        # a box that divides into no tile, open on every side
+        _steps("blast_97x75x61_fp64fast", "blast3d", 97, 75, 61, "fp64fast", 10, bc="open"),
+        # a production-sized turbulence box of one GPU's share, FP32
+        _steps("turbulence_128_fp32", "turbulence3d", 128, 128, 128, "fp32", 10),
+        # the headline workload, plain FP64 and FP32 with the indicator
+        _steps("blast_256_fp64", "mhd_blast3d", 256, 256, 256, "fp64", 10),
+        _steps("blast_256_fp32_indicator", "mhd_blast3d", 256, 256, 256, "fp32+indicator", 10),
+        # the training script's minibatch
+        {"name": "train_16384", "kind": "train", "batch": 16384},
+        # a held-out set of its size, not a multiple of any tile
+        {"name": "infer_1500001", "kind": "infer", "batch": 1500001},
+        # one snapshot of the training script's turbulence run
+        {"name": "samples_64", "kind": "samples", "problem": "turbulence3d", "nx": 64, "ny": 64, "nz": 64},
+        # a checkpoint read back and written out
+        {"name": "restart_144", "kind": "restart", "problem": "turbulence3d", "nx": 144, "ny": 144, "nz": 144},
+    ]
+
+
+def _logint(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["steps"] * 6 + ["train", "infer", "samples", "restart"])
+    if kind == "train":
+        return {"kind": kind, "batch": _logint(rng, 1000, 200000)}
+    if kind == "infer":
+        return {"kind": kind, "batch": _logint(rng, 1000, 4000000)}
+    if kind in ("samples", "restart"):
+        n = [_logint(rng, 12, 100 if kind == "samples" else 180) for _ in range(3)]
+        return {"kind": kind, "problem": rng.choice(["turbulence3d", "mhd_blast3d"]), "nx": n[0], "ny": n[1], "nz": n[2]}
+    dim = rng.choice([1, 2, 2, 3, 3, 3])
+    form = rng.choice(["fp64", "fp64", "fp32", "fp64fast", "fp32+indicator"])
+    bc = rng.choice(["periodic", "open"])
+    if dim == 1:
+        n = [_logint(rng, 64, 8192), 1, 1]
+        problem, form = "brio_wu", form.replace("+indicator", "")
+    elif dim == 2:
+        n = [_logint(rng, 32, 1200), _logint(rng, 32, 1200), 1]
+        problem = "mhd_rotor" if form.endswith("indicator") else rng.choice(["orszag_tang", "mhd_rotor"])
+    else:
+        n = [_logint(rng, 16, 200) for _ in range(3)]
+        problem = rng.choice(["mhd_blast3d", "blast3d"] if form.endswith("indicator") else
+                             ["mhd_blast3d", "turbulence3d", "cpaw3d", "mpi_smooth3d"])
+    cells = n[0] * n[1] * n[2]
+    steps = max(4, min(20, int(4e7 / cells)))
+    c = _steps("", problem, n[0], n[1], n[2], form, steps, bc=bc)
+    del c["name"]
+    return c
+
+
+# ----------------------------------------------------------------- the inputs
+def _run_of(case, seed):
+    size = dict(xsize=3.0, ysize=1.5, zsize=1.5) if case["problem"] == "cpaw3d" else {}
+    bc = case.get("bc", "periodic")
+    return H.parse(H.make_input(problem=case["problem"], nx=case["nx"], ny=case["ny"], nz=case["nz"], nt=1, tend=100.0,
+                                cour=case.get("cour", 0.4), x1bc=bc, x2bc=bc, x3bc=bc, seed=seed + 1, **size))
+
+
+def _initial(case, seed):
+    """(run, q0): the problem's initial state with a smooth density wave of 2%
+    whose wave vector and phase come from the seed (velocity, field and
+    pressure as the problem sets them)."""
+    run = _run_of(case, seed)
+    q0 = H.init_problem(run)
+    rng = np.random.default_rng(seed)
+    a = [2.0 * math.pi * int(rng.integers(1, 4)) * (np.arange(n) + 0.5) / n if n > 1 else np.zeros(1)
+         for n in (run.nx, run.ny, run.nz)]
+    ph = rng.uniform(0.0, 2.0 * math.pi)
+    f = (1.0 + 0.02 * np.sin(a[0] + ph))[:, None, None] * (1.0 + 0.02 * np.sin(a[1] - ph))[None, :, None]
+    f = f * (1.0 + 0.02 * np.sin(a[2] + 2.0 * ph))[None, None, :]
+    q = q0[:, 3:-3, 3:-3, 3:-3]
+    kin = 0.5 * (q[1] ** 2 + q[2] ** 2 + q[3] ** 2) / q[0]
+    q[7] += (f - 1.0) * kin
+    for m in range(4):
+        q[m] *= f
+    return run, q0
+
+
+def _params(run, form):
+    p = H.gpu_params(run)
+    p.precision = H.PREC[form.split("+")[0]]
+    p.indicator = H.INDICATOR["mlp" if form.endswith("+indicator") else "off"]
+    return p
+
+
+def _features(n, seed, device):
+    """n indicator samples: 6-cell stencils of three quantities (a wave, on
+    two thirds of them a jump), each mapped to [0, 1] by its min and max, as
+    the solver's features are; the label is 1 where there is a jump, but for 5%
+    of them."""
+    g = torch.Generator(device=device).manual_seed(seed)
+    r = lambda *s: torch.rand(*s, generator=g, device=device)  # noqa: E731
+    k = torch.arange(6, device=device, dtype=torch.float32)
+    jump = (r(n) < 0.65).float()
+    at = (r(n) * 5.0).floor()[:, None, None]
+    x = torch.sin(k * (0.2 + r(n, 3, 1)) + 6.3 * r(n, 3, 1)) + 0.02 * r(n, 3, 6)
+    x += jump[:, None, None] * 4.0 * (r(n, 3, 1) - 0.5) * (k > at)
+    lo, hi = x.amin(dim=2, keepdim=True), x.amax(dim=2, keepdim=True)
+    x = ((x - lo) / (hi - lo)).reshape(n, 18).contiguous()
+    y = torch.where(r(n) < 0.05, 1.0 - jump, jump)
+    return x, y
+
+
+def _network(seed, device):
+    """The trained network with seeded noise, and Adam moments of a training
+    under way."""
+    P, _ = H.load_indicator(WEIGHTS)
+    g = torch.Generator(device=device).manual_seed(seed + 77)
+    P = torch.from_numpy(P).to(device)
+    P = P + 0.05 * torch.randn(P.shape, generator=g, device=device)
+    M = 1e-3 * torch.randn(P.shape, generator=g, device=device)
+    V = 1e-5 * (0.1 + torch.rand(P.shape, generator=g, device=device))
+    return P, M, V
+
+
+ADAM_T, LR, POS_WEIGHT = 200, 2e-3, 4.0
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "steps":
+        run, q0 = _initial(case, seed)
+        solver = H.GpuSolver(_params(run, case["form"]))
+        if case["form"].endswith("+indicator"):
+            P, thr = H.load_indicator(WEIGHTS)
+            solver.set_indicator(P, thr, enable=1)
+        return {"case": case, "q0": q0, "solver": solver}
+    if kind in ("train", "infer"):
+        x, y = _features(case["batch"], seed, "cuda")
+        P, M, V = _network(seed, "cuda")
+        return {"case": case, "x": x, "y": y, "P": P, "M": M, "V": V, "G": torch.zeros_like(P),
+                "loss": torch.zeros(1, device="cuda"), "t": ADAM_T}
+    run, q0 = _initial(case, seed)
+    solver = H.GpuSolver(_params(run, "fp64"))
+    solver.upload_q0(q0)
+    solver.init_faces()
+    if kind == "samples":
+        n = [solver.n_samples(d) for d in range(3)]
+        bufs = [(torch.empty((m, H.MLP_NFEAT), dtype=torch.float32, device="cuda"),
+                 torch.empty(m, dtype=torch.float32, device="cuda")) for m in n]
+        return {"case": case, "solver": solver, "bufs": bufs}
+    return {"case": case, "solver": solver, "q0": q0, "faces": solver.faces()}
+
+
+# ------------------------------------------------------------------- one pass
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "steps":
+        s = state["solver"]
+        s.upload_q0(state["q0"])
+        s.init_faces()
+        t = 0.0
+        for _ in range(case["steps"]):
+            dt = s.tstep()
+            s.ssprk(dt)
+            t += dt
+        return {"q": s.q0(), "t": t}
+    if kind == "train":
+        state["t"] += 1
+        G, loss = state["G"].zero_(), state["loss"].zero_()
+        H.mlp_grad(state["x"], state["y"], state["P"], pos_weight=POS_WEIGHT, scale=1.0 / case["batch"], G=G, loss=loss)
+        H.mlp_adam(state["P"], state["M"], state["V"], G, state["t"], LR)
+        return {"grad": G, "loss": loss, "P": state["P"], "M": state["M"], "V": state["V"]}
+    if kind == "infer":
+        return H.mlp_infer(state["x"], state["P"])
+    s = state["solver"]
+    if kind == "samples":
+        for d, (x, y) in enumerate(state["bufs"]):
+            s.collect_samples(d, x, y)
+        return [list(b) for b in state["bufs"]]
+    s.upload_q0(state["q0"])
+    s.upload_faces(state["faces"])
+    dt = s.tstep()
+    d = s.diag()
+    return {"dt": dt, "q": s.q0(), "faces": s.faces(), "sums": np.array(list(d.sum_cons)),
+            "divb_cell": d.max_divb_cell, "min": np.array([d.min_rho, d.min_p])}
+
+
+def work(case):
+    """Bytes and operations one pass cannot do without."""
+    kind = case["kind"]
+    if kind == "train":     # samples in, five parameter-sized arrays in and out; forward and backward products
+        return {"bytes": 76.0 * case["batch"] + 40.0 * H.MLP_NPARAM, "flops": 3.0 * 2.0 * 1632 * case["batch"]}
+    if kind == "infer":
+        return {"bytes": 76.0 * case["batch"] + 4.0 * H.MLP_NPARAM, "flops": 2.0 * 1632 * case["batch"]}
+    cells = float(case["nx"] * case["ny"] * case["nz"])
+    cells6 = float((case["nx"] + 6) * (case["ny"] + 6) * (case["nz"] + 6))
+    axes = sum(n > 1 for n in (case["nx"], case["ny"], case["nz"]))
+    if kind == "samples":   # q in; 18 features and a label per interface out
+        return {"bytes": 64.0 * cells + axes * 76.0 * cells, "flops": axes * 2850.0 * cells}
+    if kind == "restart":   # q(0) and faces in and out, read once more for dt and the diagnostics
+        return {"bytes": 2.0 * 88.0 * cells6 + 2.0 * 88.0 * cells, "flops": 100.0 * cells}
+    # a stage reads q and the faces of the stages it combines and writes its
+    # own (1,472 B per zone and step in 3-D); 2,850 operations per interface
+    # and sweep, 250 per cell and stage besides
+    per_zone = 1472.0 if axes > 1 else 5 * 3 * 64.0
+    return {"bytes": 64.0 * 2.0 * cells6 + case["steps"] * per_zone * cells,
+            "flops": case["steps"] * 5.0 * (axes * 2850.0 + 250.0) * cells}
+
+
+# ------------------------------------------------- the same in plain float64
+def _index(n, off, per, device):
+    """Stored index of cell i + off for i = 0..n-1 (wrap or clamp)."""
+    i = torch.arange(n, device=device) + off
+    return i % n if per else i.clamp(0, n - 1)
+
+
+def _at(a, axis, off, per):
+    n = a.shape[axis]
+    return a if n == 1 or off == 0 else a.index_select(axis, _index(n, off, per, a.device))
+
+
+def _with_ghosts(a, axis, per, g=3):
+    n = a.shape[axis]
+    i = torch.arange(-g, n + g, device=a.device)
+    return a.index_select(axis, i % n if per else i.clamp(0, n - 1))
+
+
+def _perm(d, m):
+    return m if m in (0, 7) else (1 + (m - 1 + d) % 3 if m < 4 else 4 + (m - 4 + d) % 3)
+
+
+def _weno_phi(a, b, c, d):
+    eps = 1.0e-10
+    a0 = 1.0 / (eps + 13.0 * (a - b) ** 2 + 3.0 * (a - 3.0 * b) ** 2) ** 2
+    a1 = 6.0 / (eps + 13.0 * (b - c) ** 2 + 3.0 * (b + c) ** 2) ** 2
+    a2 = 3.0 / (eps + 13.0 * (c - d) ** 2 + 3.0 * (3.0 * c - d) ** 2) ** 2
+    s = a0 + a1 + a2
+    return (a0 / s) * (a - 2.0 * b + c) / 3.0 + (a2 / s - 0.5) * (b - 2.0 * c + d) / 6.0
+
+
+def _sweep64(q, d, per, p):
+    """Interface fluxes (7, n+1 along axis d) and the two CT flux terms (at
+    right faces) of the characteristic LLF-WENO5 sweep along axis d."""
+    gam = p.gam
+    u = _with_ghosts(torch.stack([q[_perm(d, m)] for m in range(8)]), d + 1, per).movedim(d + 1, -1).contiguous()
+    n = q.shape[d + 1]
+    rho, mom, B, E = u[0], u[1:4], u[4:7], u[7]
+    v = mom / rho
+    vv, BB = (v * v).sum(0), (B * B).sum(0)
+    pg = (gam - 1.0) * (E - 0.5 * (rho * vv + BB))
+    low = (rho < p.rhomin) | (pg < p.pgmin)
+    rho = torch.where(low, rho.clamp(min=p.rhomin), rho)
+    pg = torch.where(low, pg.clamp(min=p.pgmin), pg)
+    E = torch.where(low, pg / (gam - 1.0) + 0.5 * (rho * vv + BB), E)
+    Hh = (E + pg) / rho
+    pt, vB = pg + 0.5 * BB, (v * B).sum(0)
+    U = torch.stack([rho, mom[0], mom[1], mom[2], B[1], B[2], E])
+    F = torch.stack([rho * v[0], mom[0] * v[0] + pt - B[0] * B[0], mom[1] * v[0] - B[0] * B[1],
+                     mom[2] * v[0] - B[0] * B[2], B[1] * v[0] - B[0] * v[1], B[2] * v[0] - B[0] * v[2],
+                     (E + pt) * v[0] - B[0] * vB])
+    bb, bn = BB / rho, B[0] * B[0] / rho
+    c2 = (gam * (pg / rho).abs()).clamp(min=0.0)
+    root = ((bb + c2) ** 2 - 4.0 * bn * c2).clamp(min=0.0).sqrt()
+    lf = (0.5 * (bb + c2 + root)).clamp(min=0.0).sqrt()
+    ls = (0.5 * (bb + c2 - root)).clamp(min=0.0).sqrt()
+    la = bn.clamp(min=0.0).sqrt()
+    speed = torch.stack([v[0] - lf, v[0] - la, v[0] - ls, v[0], v[0] + ls, v[0] + la, v[0] + lf]).abs()
+    S = lambda a, k: a[..., k:k + n + 1]  # noqa: E731
+    avg = lambda a: 0.5 * (S(a, 2) + S(a, 3))  # noqa: E731
+    amx = S(speed, 0)
+    for k in range(1, 6):
+        amx = torch.maximum(amx, S(speed, k))
+    # interface eigensystem
+    r, vx, vy, vz = avg(rho), avg(v[0]), avg(v[1]), avg(v[2])
+    Bx, By, Bz, HH = avg(B[0]), avg(B[1]), avg(B[2]), avg(Hh)
+    v2 = vx * vx + vy * vy + vz * vz
+    b2, bx2 = (Bx * Bx + By * By + Bz * Bz) / r, Bx * Bx / r
+    cs2 = (gam - 1.0) * (HH - 0.5 * (v2 + b2))
+    cs = cs2.clamp(min=0.0).sqrt()
+    root = ((b2 + cs2) ** 2 - 4.0 * bx2 * cs2).clamp(min=0.0).sqrt()
+    f = (0.5 * (b2 + cs2 + root)).clamp(min=0.0).sqrt()
+    s = (0.5 * (b2 + cs2 - root)).clamp(min=0.0).sqrt()
+    one = torch.ones_like(f)
+    gap = f * f - s * s
+    sg = gap.clamp(min=1.0e-30).sqrt()
+    af = torch.where(gap >= 1.0e-30, (cs2 - s * s).clamp(min=0.0).sqrt() / sg, one)
+    as_ = torch.where(gap >= 1.0e-30, (f * f - cs2).clamp(min=0.0).sqrt() / sg, one)
+    bt2 = By * By + Bz * Bz
+    sb = bt2.clamp(min=1.0e-30).sqrt()
+    ty = torch.where(bt2 >= 1.0e-30, By / sb, one / math.sqrt(2.0))
+    tz = torch.where(bt2 >= 1.0e-30, Bz / sb, one / math.sqrt(2.0))
+    sgn = torch.where(Bx >= 0.0, one, -one)
+    sr = r.sqrt()
+    g0, g1, g2 = 1.0 - gam, 0.5 * (gam - 1.0), (gam - 2.0) / (gam - 1.0)
+    tv, zero = ty * vy + tz * vz, torch.zeros_like(f)
+
+    def fast_l(sig):     # -1: wave 0, +1: wave 6
+        return [af * (g1 * v2 - sig * f * vx) + sig * as_ * s * tv * sgn, af * (g0 * vx + sig * f),
+                g0 * af * vy - sig * as_ * s * ty * sgn, g0 * af * vz - sig * as_ * s * tz * sgn,
+                g0 * af * By + cs * as_ * ty * sr, g0 * af * Bz + cs * as_ * tz * sr, -g0 * af]
+
+    def slow_l(sig):     # -1: wave 2, +1: wave 4
+        return [as_ * (g1 * v2 - sig * s * vx) - sig * af * f * tv * sgn, as_ * (g0 * vx + sig * s),
+                g0 * as_ * vy + sig * af * f * ty * sgn, g0 * as_ * vz + sig * af * f * tz * sgn,
+                g0 * as_ * By - cs * af * ty * sr, g0 * as_ * Bz - cs * af * tz * sr, -g0 * as_]
+
+    def alf_l(sig):      # -1: wave 1, +1: wave 5
+        return [tz * vy - ty * vz, zero, -tz, ty, sig * tz * sgn * sr, -sig * ty * sgn * sr, zero]
+
+    ent = [-cs2 / g0 - 0.5 * v2, vx, vy, vz, By, Bz, -one]
+    sc = 0.5 / cs2
+    L = torch.stack([torch.stack(x) for x in (
+        [a * sc for a in fast_l(-1)], [0.5 * a for a in alf_l(-1)], [a * sc for a in slow_l(-1)],
+        [-g0 * a / cs2 for a in ent],
+        [a * sc for a in slow_l(1)], [0.5 * a for a in alf_l(1)], [a * sc for a in fast_l(1)])])
+
+    def fast_r(sig):
+        return [af, af * (vx + sig * f), af * vy - sig * as_ * s * ty * sgn, af * vz - sig * as_ * s * tz * sgn,
+                cs * as_ * ty / sr, cs * as_ * tz / sr,
+                af * (f * f + sig * f * vx + 0.5 * v2 - g2 * cs2) - sig * as_ * s * tv * sgn]
+
+    def slow_r(sig):
+        return [as_, as_ * (vx + sig * s), as_ * vy + sig * af * f * ty * sgn, as_ * vz + sig * af * f * tz * sgn,
+                -cs * af * ty / sr, -cs * af * tz / sr,
+                as_ * (s * s + sig * s * vx + 0.5 * v2 - g2 * cs2) + sig * af * f * tv * sgn]
+
+    def alf_r(sig):
+        return [zero, zero, -tz, ty, sig * tz * sgn / sr, -sig * ty * sgn / sr, ty * vz - tz * vy]
+
+    ent_r = [one, vx, vy, vz, zero, zero, 0.5 * v2]
+    Fk = [sum(L[:, j] * S(F[j], k) for j in range(7)) for k in range(6)]
+    qk = [sum(L[:, j] * S(U[j], k) for j in range(7)) for k in range(6)]
+    dF = [Fk[k + 1] - Fk[k] for k in range(5)]
+    dq = [amx * (qk[k + 1] - qk[k]) for k in range(5)]
+    pl = [0.5 * (dF[k] + dq[k]) for k in range(5)]
+    mi = [0.5 * (dF[k] - dq[k]) for k in range(5)]
+    Fs = (-Fk[1] + 7.0 * Fk[2] + 7.0 * Fk[3] - Fk[4]) / 12.0 - _weno_phi(*pl[:4]) + _weno_phi(*mi[4:0:-1])
+    R = [fast_r(-1), alf_r(-1), slow_r(-1), ent_r, slow_r(1), alf_r(1), fast_r(1)]
+    flux = torch.stack([sum(R[m][c] * Fs[m] for m in range(7)) for c in range(7)])
+    cta = (flux[4] + avg(B[0] * v[1]))[..., 1:]
+    ctb = (flux[5] + avg(B[0] * v[2]))[..., 1:]
+    return flux.movedim(-1, d + 1), cta.movedim(-1, d), ctb.movedim(-1, d)
+
+
+def _four(a, axis, per):
+    return (-_at(a, axis, -1, per) + 9.0 * a + 9.0 * _at(a, axis, 1, per) - _at(a, axis, 2, per)) / 16.0
+
+
+def _lap(a, axis, per):
+    return (_at(a, axis, -1, per) - 2.0 * a + _at(a, axis, 1, per)) / 24.0
+
+
+def _d4(a, axis, per):
+    return 9.0 / 8.0 * (a - _at(a, axis, -1, per)) - (_at(a, axis, 1, per) - _at(a, axis, -2, per)) / 24.0
+
+
+def _centre(a, axis, per):
+    s = lambda o: _at(a, axis, o, per)  # noqa: E731
+    return (3.0 * (s(-3) + s(2)) - 25.0 * (s(-2) + s(1)) + 150.0 * (s(-1) + a)) / 256.0
+
+
+RK = {1: (1.0, 0.39175222700392, 0.0, 0.0, 0.0),
+      2: (0.44437049406734, 0.36841059262959, 0.55562950593266, 0.0, 0.0),
+      3: (0.62010185138540, 0.25189177424738, 0.37989814861460, 0.0, 0.0),
+      4: (0.17807995410773, 0.54497475021237, 0.82192004589227, 0.0, 0.0),
+      5: (-2.081261929715610e-02, 0.22600748319395, 5.03580947213895e-1, 0.51723167208978, -6.518979800418380e-12)}
+PERMS = [[_perm(d, m) for m in range(8)] for d in range(3)]
+
+
+def _step64(q, b, dt, p, per):
+    n = q.shape[1:]
+    use = [m > 1 for m in n]
+    delta = (p.dx, p.dy, p.dz)
+    Q, Bf = {0: q}, {0: b}
+    for iw in range(1, 6):
+        k1, k2, k3, k4, k5 = RK[iw]
+        mix = lambda X: X[0] + k4 / k1 * X[2] + k5 / k1 * X[3] if iw == 5 else X[0]  # noqa: E731
+        qi, bi, qp, bp = mix(Q), mix(Bf), Q[iw - 1], Bf[iw - 1]
+        new, ct = k1 * qi + k3 * qp, {}
+        for d in range(3):
+            if not use[d]:
+                continue
+            flux, ct[2 * d], ct[2 * d + 1] = _sweep64(qp, d, per[d], p)
+            diff = -(k2 * dt / delta[d]) * torch.diff(flux, dim=d + 1)
+            for slot, m in enumerate((0, 1, 2, 3, 5, 6, 7)):
+                new[PERMS[d][m]] += diff[slot]
+        c = [k2 * dt / x for x in delta]
+        ox, oy, oz = use[0] and use[1], use[1] and use[2], use[0] and use[2]
+        bo = bi.clone()
+        # x: fsy, fsz; y: gsz, gsx; z: hsx, hsy
+        if ox:
+            o = _four(ct[3], 0, per[0]) - _four(ct[0], 1, per[1])
+            Ox = o + _lap(o, 0, per[0]) + _lap(o, 1, per[1])
+        if oy:
+            o = _four(ct[5], 1, per[1]) - _four(ct[2], 2, per[2])
+            Oy = o + _lap(o, 1, per[1]) + _lap(o, 2, per[2])
+        if oz:
+            o = _four(ct[1], 2, per[2]) - _four(ct[4], 0, per[0])
+            Oz = o + _lap(o, 0, per[0]) + _lap(o, 2, per[2])
+        if ox or oz:
+            bo[0] = k1 * bi[0] + k3 * bp[0]
+            bo[0] += (-c[1] * _d4(Ox, 1, per[1]) if ox else 0.0) + (c[2] * _d4(Oz, 2, per[2]) if oz else 0.0)
+        if oy or ox:
+            bo[1] = k1 * bi[1] + k3 * bp[1]
+            bo[1] += (-c[2] * _d4(Oy, 2, per[2]) if oy else 0.0) + (c[0] * _d4(Ox, 0, per[0]) if ox else 0.0)
+        if oz or oy:
+            bo[2] = k1 * bi[2] + k3 * bp[2]
+            bo[2] += (-c[0] * _d4(Oz, 0, per[0]) if oz else 0.0) + (c[1] * _d4(Oy, 1, per[1]) if oy else 0.0)
+        if ox or oy or oz:
+            for d in range(3):
+                new[4 + d] = _centre(bo[d], d, per[d]) if use[d] else bo[d]
+        rho = new[0].clamp(min=p.rhomin)
+        kin, mag = 0.5 * (new[1:4] ** 2).sum(0) / rho, 0.5 * (new[4:7] ** 2).sum(0)
+        pg = ((p.gam - 1.0) * (new[7] - kin - mag)).clamp(min=p.pgmin)
+        new[0], new[7] = rho, pg / (p.gam - 1.0) + kin + mag
+        Q[iw], Bf[iw] = new, bo
+    return Q[5], Bf[5]
+
+
+def _dt64(q, p):
+    rho = q[0].clamp(min=p.rhomin)
+    v = q[1:4] / rho
+    BB = (q[4:7] ** 2).sum(0)
+    pg = ((p.gam - 1.0) * (q[7] - 0.5 * (rho * (v * v).sum(0) + BB))).clamp(min=p.pgmin)
+    b, c = BB / rho, p.gam * pg / rho
+    inv = 0.0
+    for d, dx in enumerate((p.dx, p.dy, p.dz)):
+        if q.shape[d + 1] > 1:
+            root = ((b + c) ** 2 - 4.0 * q[4 + d] ** 2 / rho * c).clamp(min=0.0).sqrt()
+            inv += float((v[d].abs() + (0.5 * (b + c + root)).sqrt()).max()) / dx
+    return p.cour / inv
+
+
+def _ref_layout(a, per):
+    for d in range(3):
+        a = _with_ghosts(a, a.dim() - 3 + d, per[d])
+    return a
+
+
+def _net64(x, P, y, scale):
+    """Forward pass, and (y given) loss and gradient, of the indicator network
+    with bf16 operands and 64-bit sums."""
+    bf = lambda a: a.to(torch.bfloat16).double()  # noqa: E731
+    W1, b1 = bf(P[0:576].reshape(32, 18)), P[576:608].double()
+    W2, b2 = bf(P[608:1632].reshape(32, 32)), P[1632:1664].double()
+    w3, b3 = bf(P[1664:1696]), P[1696].double()
+    x = bf(x)
+    a1 = bf((x @ W1.T + b1).clamp(min=0.0).float())
+    a2 = bf((a1 @ W2.T + b2).clamp(min=0.0).float())
+    z = a2 @ w3 + b3
+    if y is None:
+        return z
+    y = y.double()
+    w = torch.where(y > 0.5, POS_WEIGHT, 1.0).double()
+    loss = (w * (torch.nn.functional.softplus(z) - y * z)).sum() * scale
+    dz = w * (torch.sigmoid(z) - y) * scale
+    d2 = bf((dz[:, None] * w3 * (a2 != 0.0)).float())
+    d1 = bf(((d2 @ W2) * (a1 != 0.0)).float())
+    G = torch.cat([(d1.T @ x).reshape(-1), d1.sum(0), (d2.T @ a1).reshape(-1), d2.sum(0), a2.T @ dz, dz.sum()[None]])
+    return G, loss
+
+
+def _features64(q, d, per, gam):
+    """Indicator features of every interface along axis d, in the solver's
+    sample order."""
+    v2 = (q[1:4] ** 2).sum(0) / q[0]
+    B2 = (q[4:7] ** 2).sum(0)
+    out = []
+    n = q.shape[d + 1]
+    for a in (q[0], (gam - 1.0) * (q[7] - 0.5 * (v2 + B2)), B2.sqrt()):
+        g = _with_ghosts(a, d, per).movedim(d, -1)
+        x = g.unfold(-1, 6, 1)[..., (1 if per else 0):n + 1, :]
+        lo, hi = x.amin(-1, keepdim=True), x.amax(-1, keepdim=True)
+        span = hi - lo
+        flat = span <= 1e-5 * torch.maximum(hi.abs(), lo.abs()) + 1e-30
+        out.append(torch.where(flat, torch.zeros_like(x), (x - lo) / torch.where(flat, torch.ones_like(span), span)))
+    x = torch.cat(out, dim=-1).movedim(-2, d)          # x, y, z, feature
+    return x.permute(2, 1, 0, 3).reshape(-1, 18)       # x fastest, as stored
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    if kind in ("train", "infer"):
+        x, y = _features(case["batch"], seed, dev)
+        P, M, V = _network(seed, dev)
+        if kind == "infer":
+            return torch.cat([_net64(c, P, None, 0.0) for c in x.split(1 << 18)])
+        G, loss = _net64(x, P, y, 1.0 / case["batch"])
+        b1, b2, t = 0.9, 0.999, ADAM_T + 1
+        M = b1 * M.double() + (1.0 - b1) * G
+        V = b2 * V.double() + (1.0 - b2) * G * G
+        P = P.double() - LR * (M / (1.0 - b1 ** t)) / ((V / (1.0 - b2 ** t)).sqrt() + 1e-8)
+        return {"grad": G, "loss": loss[None], "P": P, "M": M, "V": V}
+    cells = case["nx"] * case["ny"] * case["nz"]
+    if kind == "steps" and cells * case["steps"] > 6e7:
+        return None
+    run_, q0 = _initial(case, seed)
+    p = H.gpu_params(run_)
+    per = [p.bc[d] == H.BC["periodic"] for d in range(3)]
+    q = torch.from_numpy(np.ascontiguousarray(H.active(q0))).to(dev)
+    if kind == "samples":
+        return [[_features64(q, d, per[d], p.gam), None] for d in range(3)]
+    b = torch.stack([_four(q[4 + d], d, per[d]) for d in range(3)])
+    if kind == "restart":
+        v2 = (q[1:4] ** 2).sum(0) / q[0]
+        pg = (p.gam - 1.0) * (q[7] - 0.5 * v2 - 0.5 * (q[4:7] ** 2).sum(0))
+        return {"dt": _dt64(q, p), "q": _ref_layout(q, per).cpu(), "faces": _ref_layout(b, per).cpu(),
+                "sums": None, "divb_cell": None, "min": torch.stack([q[0].min(), pg.min()]).cpu()}
+    t = 0.0
+    for _ in range(case["steps"]):
+        dt = _dt64(q, p)
+        q, b = _step64(q, b, dt, p, per)
+        t += dt
+    return {"q": _ref_layout(q, per).cpu(), "t": t}
