@@ -107,18 +107,26 @@ def _run_of(case, seed):
 
 
 def _initial(case, seed):
-    """(run, q0): the problem's initial state with a smooth density wave of 2%
-    whose wave vector and phase come from the seed (velocity, field and
-    pressure as the problem sets them)."""
+    """(run, q0): the problem's initial state with another density from the
+    seed (velocity, field and pressure as the problem sets them).  Blasts and
+    rotors keep their uniform surroundings, on which the indicator's routing
+    depends: their density is scaled by one factor within 10% and the whole
+    state moved by up to an eighth of the box.  The others get a smooth wave
+    of 2% with the seed's wave vector and phase."""
     run = _run_of(case, seed)
     q0 = H.init_problem(run)
     rng = np.random.default_rng(seed)
-    a = [2.0 * math.pi * int(rng.integers(1, 4)) * (np.arange(n) + 0.5) / n if n > 1 else np.zeros(1)
-         for n in (run.nx, run.ny, run.nz)]
-    ph = rng.uniform(0.0, 2.0 * math.pi)
-    f = (1.0 + 0.02 * np.sin(a[0] + ph))[:, None, None] * (1.0 + 0.02 * np.sin(a[1] - ph))[None, :, None]
-    f = f * (1.0 + 0.02 * np.sin(a[2] + 2.0 * ph))[None, None, :]
     q = q0[:, 3:-3, 3:-3, 3:-3]
+    n = (run.nx, run.ny, run.nz)
+    if "blast" in case["problem"] or case["problem"] in ("mhd_rotor", "brio_wu"):
+        f = rng.uniform(0.9, 1.1)
+        if case["problem"] != "brio_wu":
+            q[...] = np.roll(q, [int(rng.integers(-(m // 8), m // 8 + 1)) for m in n], axis=(1, 2, 3))
+    else:
+        a = [2.0 * math.pi * int(rng.integers(1, 4)) * (np.arange(m) + 0.5) / m if m > 1 else np.zeros(1) for m in n]
+        ph = rng.uniform(0.0, 2.0 * math.pi)
+        f = (1.0 + 0.02 * np.sin(a[0] + ph))[:, None, None] * (1.0 + 0.02 * np.sin(a[1] - ph))[None, :, None]
+        f = f * (1.0 + 0.02 * np.sin(a[2] + 2.0 * ph))[None, None, :]
     kin = 0.5 * (q[1] ** 2 + q[2] ** 2 + q[3] ** 2) / q[0]
     q[7] += (f - 1.0) * kin
     for m in range(4):
