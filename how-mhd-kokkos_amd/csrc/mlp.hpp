@@ -65,49 +65,6 @@ __host__ __device__ constexpr int mlp_acc_row(int r, int h) { return 8 * (r / 4)
 // the lane (rows 8s..8s+7).
 __host__ __device__ constexpr int mlp_hidden_slot(int s, int v, int h) { return mlp_acc_row(8 * s + v, h); }
 
-// B-operand fragments of one 32x32 bf16 matrix Wt[k][n]: [k-step s][n-tile u]
-struct BFrag {
-    bf16x4 f[2][2];
-};
-
-// Scratch rows of one wavefront: 64 rows x 32 bf16 (+2 pad to stagger banks).
-constexpr int MLP_ROW = MLP_H + 2;
-
-// One dense layer on the 64 rows of a wavefront: dst <- relu(src * Wt + b),
-// bf16 rows of MLP_ROW, four 16-row tiles.  src may equal dst: every lane
-// reads its fragments of a tile before any lane writes that tile.
-__device__ __forceinline__ void layer_relu(const uint16_t* src, uint16_t* dst, const BFrag& W, const float* bias) {
-    const int l = threadIdx.x & 63;
-    const int r16 = l % 16, kq = 4 * (l / 16);
-    const float bl0 = bias[r16], bl1 = bias[16 + r16];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        bf16x4 a[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) a[s][v] = (short)src[(16 * t + r16) * MLP_ROW + 16 * s + kq + v];
-        f32x4 d[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const float b = u ? bl1 : bl0;
-            f32x4 c = {b, b, b, b};
-            c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[0], W.f[0][u], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[1], W.f[1][u], c, 0, 0, 0);
-            d[u] = c;
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float z = d[u][v];
-                dst[(16 * t + kq + v) * MLP_ROW + 16 * u + r16] = f2bf(z > 0.f ? z : 0.f);
-            }
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
 // Features of one interface from its 6-cell stencils of rho, p and |B|: each
 // mapped to [0, 1] by its min and max, or all 0 when max - min <= MLP_FLAT
 // max(|min|, |max|).  The relative floor keeps round-off-level wiggles of
