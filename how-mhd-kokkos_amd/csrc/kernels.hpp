@@ -911,7 +911,7 @@ __global__ __launch_bounds__(256) void k_emf(SmoothArgs<R> A) {
 // set): the corner EMFs O2 of src/fluxct.cpp:809-821 and their smoothing,
 // 828-840, without the O2 round trip through memory.  A block of 512
 // threads holds a 64 x 8 tile of columns (EMF_OX x EMF_OY owned columns and a
-// one-column halo) and marches through EMF_CZ planes.  Per plane z:
+// one-column halo) and marches through cz planes (stage.hpp).  Per plane z:
 //  * the in-plane CT fluxes of plane z + 1 (gsx, hsx with a 1|2-column halo
 //    for their x stencils, fsy, hsy with a 1|2-row halo) were loaded one
 //    plane ahead and go to LDS; gsz and fsz come from per-column registers
@@ -933,10 +933,7 @@ __global__ __launch_bounds__(256) void k_emf(SmoothArgs<R> A) {
 #ifndef HOWMHD_EMF_WY
 #define HOWMHD_EMF_WY 8
 #endif
-#ifndef HOWMHD_EMF_CZ
-#define HOWMHD_EMF_CZ 32
-#endif
-constexpr int EMF_WX = HOWMHD_EMF_WX, EMF_WY = HOWMHD_EMF_WY, EMF_CZ = HOWMHD_EMF_CZ;
+constexpr int EMF_WX = HOWMHD_EMF_WX, EMF_WY = HOWMHD_EMF_WY;
 constexpr int EMF_OX = EMF_WX - 2, EMF_OY = EMF_WY - 2;
 constexpr int EMF_THREADS = EMF_WX * EMF_WY;
 static_assert(6 * (EMF_WX + EMF_WY) <= EMF_THREADS, "one stencil-halo cell per thread at most");
@@ -946,6 +943,7 @@ struct EmfMarchArgs {
     const R *fsy, *fsz, *gsx, *gsz, *hsx, *hsy;
     R *Ox, *Oy, *Oz;
     Geom g;
+    int cz;  // planes per block
 };
 
 template <typename R, int EX>
@@ -960,7 +958,7 @@ __global__ __launch_bounds__(EMF_THREADS) void k_emf_march(EmfMarchArgs<R> A) {
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
     const int px = g.per[0], py = g.per[1], pz = g.per[2];
     const int x0 = blockIdx.x * EMF_OX, y0 = blockIdx.y * EMF_OY;
-    const int zs = blockIdx.z * EMF_CZ, ze = min(zs + EMF_CZ, nz);
+    const int zs = blockIdx.z * A.cz, ze = min(zs + A.cz, nz);
     const int tid = threadIdx.x;
     const int ex = tid % WX, ey = tid / WX;
     // image of tile position p (x: column, y: row); positions beyond the
@@ -1106,6 +1104,7 @@ struct FaceArgs {
     Geom g;
     CtFlags f;
     StageCoef s;
+    int cz;  // k_faces_march: planes per block
 };
 
 // Staggered 4th-order difference aa*(o0-om1) + bb*(op1-om2) + cc*(op2-om3),
@@ -1207,15 +1206,11 @@ __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
 }
 
 // k_faces for three-dimensional grids (every CT flag set), marching a
-// FACE_TX x FACE_TY column tile through FACE_CZ planes: the in-plane EMF
+// FACE_TX x FACE_TY column tile through cz planes (stage.hpp): the in-plane EMF
 // tiles of each plane (the LDS tiles of k_faces) and the face values of the
 // next plane are loaded one plane ahead, and each column keeps Oy and Oz of
 // planes z - 3 .. z + 2 (images through bmap) in registers for the z
 // differences.  The arithmetic is k_faces', term for term.
-#ifndef HOWMHD_FACE_CZ
-#define HOWMHD_FACE_CZ 32
-#endif
-constexpr int FACE_CZ = HOWMHD_FACE_CZ;
 // 3 wavefronts per SIMD (136 VGPRs, no scratch in FP64; 4 spills 4 values and
 // runs 4% slower)
 #ifndef HOWMHD_FACE_WAVES
@@ -1237,7 +1232,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_FACE
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
     const int px = g.per[0], py = g.per[1], pz = g.per[2];
     const int x0 = blockIdx.x * FACE_TX, y0 = blockIdx.y * FACE_TY;
-    const int zs = blockIdx.z * FACE_CZ, ze = min(zs + FACE_CZ, nz);
+    const int zs = blockIdx.z * A.cz, ze = min(zs + A.cz, nz);
     const int tid = threadIdx.x;
     const long long plane = (long long)nx * ny;
     auto hx = [&](int c) { const int a = x0 - 3 + c; return bmap(a > nx + 2 ? nx + 2 : a, nx, px); };

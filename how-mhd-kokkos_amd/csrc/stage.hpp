@@ -58,6 +58,25 @@ inline int march_steps(const dim3& tiles) {
     return s < 1 ? 1 : (int)s;
 }
 
+// Planes per block of the kernels that march through z (k_emf_march,
+// k_faces_march).  A block's time is a start (the EMF's first two planes come
+// from memory with 24 loads a cell) plus about 1.2 us per plane, so a grid
+// that cannot fill the chip with long marches takes as many planes as leave
+// kPlaneMarchBlocks blocks, two per CU.  Measured in FP64 against 32 planes
+// everywhere: 32^3 EMF 47 -> 10 us and faces 44 -> 7 us (1 plane), 64^3
+// 49 -> 20 and 46 -> 11 (3 and 2), 97x75x61 50 -> 24 and 52 -> 23 (4 and 5),
+// 128^3 85 -> 74 and 59 -> 53 (17 and 6).  Longer marches than the maxima gain
+// nothing: EMF 354 us with 32 or 64 planes at 256^3 (370 with 12); faces
+// 333 us with 6 or 32 there, but 147 against 169 us at 192^3, where 32 planes
+// make 864 blocks, one more than a round of the 768 the chip holds.
+constexpr unsigned kPlaneMarchBlocks = 512;
+constexpr int kEmfMaxPlanes = 32, kFaceMaxPlanes = 6;
+inline int march_planes(const dim3& tiles, int nz, int most) {
+    const unsigned long long n = (unsigned long long)tiles.x * tiles.y * (unsigned)nz;
+    const unsigned long long cz = (n + kPlaneMarchBlocks - 1) / kPlaneMarchBlocks;
+    return (int)std::min<unsigned long long>(cz, (unsigned long long)most);
+}
+
 // The sweep along d.  Reference rounding: the sweep with unscaled WENO
 // divisions, then the IEEE-division launch for the tiles it queued (it exits
 // at once when there are none; no counting there).
@@ -170,7 +189,9 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
         e.hsx = (const R*)c->ct[4]; e.hsy = (const R*)c->ct[5];
         e.Ox = (R*)c->O[0]; e.Oy = (R*)c->O[1]; e.Oz = (R*)c->O[2];
         e.g = c->g;
-        const dim3 grid(blocks_for(c->g.n[0], EMF_OX), blocks_for(c->g.n[1], EMF_OY), blocks_for(c->g.n[2], EMF_CZ));
+        dim3 grid(blocks_for(c->g.n[0], EMF_OX), blocks_for(c->g.n[1], EMF_OY));
+        e.cz = march_planes(grid, c->g.n[2], kEmfMaxPlanes);
+        grid.z = blocks_for(c->g.n[2], e.cz);
         {
             TimedLaunch tl(c, HOWMHD_K_EMF);
             hipLaunchKernelGGL((k_emf_march<R, EX>), grid, dim3(EMF_THREADS), 0, c->stream, e);
@@ -213,8 +234,9 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
     {
         TimedLaunch tl(c, HOWMHD_K_FACES);
         if (c->ctf.use_x && c->ctf.use_y && c->ctf.use_z) {
-            const dim3 fgrid(blocks_for(c->g.n[0], FACE_TX), blocks_for(c->g.n[1], FACE_TY),
-                             blocks_for(c->g.n[2], FACE_CZ));
+            dim3 fgrid(blocks_for(c->g.n[0], FACE_TX), blocks_for(c->g.n[1], FACE_TY));
+            fa.cz = march_planes(fgrid, c->g.n[2], kFaceMaxPlanes);
+            fgrid.z = blocks_for(c->g.n[2], fa.cz);
             hipLaunchKernelGGL((k_faces_march<R, EX>), fgrid, dim3(256), 0, c->stream, fa);
         } else {
             const dim3 fgrid(blocks_for(c->g.n[0], FACE_TX), blocks_for(c->g.n[1], FACE_TY), c->g.n[2]);

@@ -1,0 +1,41 @@
+"""Launch rules that depend on the grid size, against the CPU restatement bit
+for bit (needs a GPU; plain FP64, one step, q and faces).
+
+z-marching EMF and face kernels: planes per block from one (a grid far too
+small for the chip) over a few, with and without a remainder, to a last chunk
+of one plane; periodic and open edges.
+"""
+import numpy as np
+import pytest
+
+import howmhd as H
+import oracle_ctypes as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _step_matches(problem, n, bc, steps=1):
+    run = H.parse(H.make_input(problem=problem, nx=n[0], ny=n[1], nz=n[2], nt=1, tend=1.0, x1bc=bc, x2bc=bc, x3bc=bc))
+    print(f"[launch rules] {problem} {n} {bc}", flush=True)
+    p, q0 = H.gpu_params(run), H.init_problem(run)
+    ref, gpu = O.RefSolver(p), H.GpuSolver(p)
+    for s in (ref, gpu):
+        s.upload_q0(q0)
+        s.init_faces()
+    for _ in range(steps):
+        dt = ref.tstep()
+        assert gpu.tstep() == dt
+        ref.ssprk(dt)
+        gpu.ssprk(dt)
+    for a, b in ((gpu.q0(), ref.q0()), (gpu.faces(), ref.faces())):
+        assert np.array_equal(H.active(a).view(np.int64), H.active(b).view(np.int64))
+    gpu.close()
+    ref.close()
+
+
+# (EMF planes per block, face planes): (1, 1) with 5 planes; (2, 2) with an odd
+# depth; (3, 2), last EMF chunk one plane; (5, 5), last chunks 4 and 4; (1, 6)
+@pytest.mark.parametrize("n,bc", [((33, 30, 5), "open"), ((70, 64, 41), "periodic"), ((64, 50, 67), "open"),
+                                  ((130, 61, 64), "periodic"), ((9, 8, 400), "open")])
+def test_planes_per_block(n, bc, require_gpu):
+    _step_matches("mpi_smooth3d", n, bc)
