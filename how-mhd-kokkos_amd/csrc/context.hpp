@@ -51,9 +51,12 @@ struct howmhd_gpu_ctx {
     // diagnostics: per-block partials of k_diag and the folded values
     double* diagpart = nullptr;
     double* diagout = nullptr;
-    // host transfers: one variable in the reference layout
-    // ((nx+6)(ny+6)(nz+6) doubles), allocated with the context
-    double* stage_ref = nullptr;
+    // host transfers (transfer.hpp): pinned slots of xfer_slot values each,
+    // with an event per slot, allocated with the context
+    double* xfer = nullptr;
+    size_t xfer_slot = 0;
+    int xfer_n = 0;
+    std::vector<hipEvent_t> xfer_ev;
     // learned indicator: device weights, routing mode (0 off, 1 on with the
     // plain-WENO fallback, 2 on for every step), the routed sweeps' counters
     // per wavefront slot (nwave slots, cleared by each fold) and their

@@ -16,6 +16,7 @@
 #include "howmhd_mlp.h"
 #include "context.hpp"
 #include "tstep_kernels.hpp"
+#include "transfer.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -99,46 +100,6 @@ uint16_t bf16_bits(float f) {
     uint32_t u;
     std::memcpy(&u, &r, 4);
     return (uint16_t)(u >> 16);
-}
-
-// Transfers between the caller's arrays in the reference layout
-// (m, i, j, k), three ghost layers per side, and the device layout
-// (m, z, y, x) of active cells.  One variable at a time goes through the
-// context's staging buffer of one variable's reference-layout size: the copy
-// reads or writes the caller's (pageable) memory directly and the transpose
-// runs on the device (k_ref_to_dev, k_dev_to_ref).
-size_t ref_size(const howmhd_gpu_ctx* c) {
-    return ((size_t)c->g.n[0] + 6) * ((size_t)c->g.n[1] + 6) * ((size_t)c->g.n[2] + 6);
-}
-
-unsigned lay_planes(int n) { return (unsigned)std::min(n, 65535); }
-
-int upload_ref(howmhd_gpu_ctx* c, const double* ref, double* dev, int nvar) {
-    const size_t n6 = ref_size(c);
-    const dim3 grid(blocks_for(c->g.n[2], LAY_T), blocks_for(c->g.n[0], LAY_T), lay_planes(c->g.n[1]));
-    for (int m = 0; m < nvar; ++m) {
-        HCHECK(c, hipMemcpyAsync(c->stage_ref, ref + (size_t)m * n6, n6 * sizeof(double), hipMemcpyHostToDevice,
-                                 c->stream));
-        hipLaunchKernelGGL(k_ref_to_dev, grid, dim3(LAY_T, 8), 0, c->stream, (const double*)c->stage_ref,
-                           dev + (size_t)m * c->ncell, c->g);
-        HCHECK(c, hipGetLastError());
-    }
-    HCHECK(c, hipStreamSynchronize(c->stream));
-    return HOWMHD_OK;
-}
-
-int download_ref(howmhd_gpu_ctx* c, const double* dev, double* ref, int nvar) {
-    const size_t n6 = ref_size(c);
-    const dim3 grid(blocks_for(c->g.n[2] + 6, LAY_T), blocks_for(c->g.n[0] + 6, LAY_T), lay_planes(c->g.n[1] + 6));
-    for (int m = 0; m < nvar; ++m) {
-        hipLaunchKernelGGL(k_dev_to_ref, grid, dim3(LAY_T, 8), 0, c->stream, dev + (size_t)m * c->ncell,
-                           c->stage_ref, c->g);
-        HCHECK(c, hipGetLastError());
-        HCHECK(c, hipMemcpyAsync(ref + (size_t)m * n6, c->stage_ref, n6 * sizeof(double), hipMemcpyDeviceToHost,
-                                 c->stream));
-    }
-    HCHECK(c, hipStreamSynchronize(c->stream));
-    return HOWMHD_OK;
 }
 
 // dt of src/tstep.cpp:123-135 from the per-direction maxima
@@ -289,7 +250,15 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
     ok = ok && alloc((void**)&c->floorpart, 2 * (size_t)blocks_for(c->ncell, 256) * sizeof(unsigned));
     ok = ok && alloc((void**)&c->diagpart, (size_t)DIAG_BLOCKS * DIAG_NV * sizeof(double));
     ok = ok && alloc((void**)&c->diagout, DIAG_NV * sizeof(double));
-    ok = ok && alloc((void**)&c->stage_ref, ref_size(c) * sizeof(double));
+    c->xfer_slot = xfer_slot(c->ncell, n[2]);
+    c->xfer_n = xfer_slots(c->ncell, c->xfer_slot);
+    ok = ok && hipHostMalloc((void**)&c->xfer, c->xfer_n * c->xfer_slot * sizeof(double), hipHostMallocDefault) ==
+                   hipSuccess;
+    for (int s = 0; s < c->xfer_n && ok; ++s) {
+        hipEvent_t ev = nullptr;
+        ok = hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+        if (ok) c->xfer_ev.push_back(ev);
+    }
     ok = ok && alloc((void**)&c->mlp, sizeof(MlpDev));
     // one counter slot per wavefront of the largest sweep grid
     for (int d = 0; d < 3; ++d) {
@@ -331,7 +300,8 @@ int howmhd_gpu_destroy(howmhd_gpu_ctx* c) {
     if (c->floorpart) (void)hipFree(c->floorpart);
     if (c->diagpart) (void)hipFree(c->diagpart);
     if (c->diagout) (void)hipFree(c->diagout);
-    if (c->stage_ref) (void)hipFree(c->stage_ref);
+    if (c->xfer) (void)hipHostFree(c->xfer);
+    for (hipEvent_t ev : c->xfer_ev) (void)hipEventDestroy(ev);
     if (c->ilast) (void)hipFree(c->ilast);
     if (c->mlp) (void)hipFree(c->mlp);
     if (c->istats) (void)hipFree(c->istats);

@@ -43,7 +43,7 @@ struct Geom {
 };
 
 // Active index a in [-3, n+2] -> stored index, following src/bound.cpp.
-__device__ __forceinline__ int bmap(int a, int n, int per) {
+__host__ __device__ __forceinline__ int bmap(int a, int n, int per) {
     if (n == 1) return 0;
     if (per) return a < 0 ? a + n : (a >= n ? a - n : a);
     return a < 0 ? 0 : (a >= n ? n - 1 : a);

@@ -277,62 +277,60 @@ __global__ __launch_bounds__(256) void k_init_faces(const double* q, double* b, 
 }
 
 // ------------------------------------------- host layout <-> device layout
-// One variable in the reference's host layout: (nx+6) x (ny+6) x (nz+6)
-// values, three ghost layers per side, z fastest (the q(m, i, j, k) view of
-// src/bound.cpp:19-95 for one m); on the device: active cells only, x
-// fastest.  Both directions transpose (x, z) tiles of 32 x 32 through LDS at
-// fixed y, so that global reads and writes are contiguous along a wavefront
-// on both sides.  Block 32 x 8; grid (z tiles, x tiles, y planes), the
-// planes strided by gridDim.z.
+// One chunk of a host transfer (transfer.hpp): per variable ni rows (x from
+// i0) of ncol values, row-contiguous in pinned host memory, column (j, k) =
+// (col / nz, col % nz) from y plane j0; on the device x is fastest.  Blocks
+// transpose 32 x 32 tiles through LDS, so that reads and writes are
+// contiguous along a wavefront on both sides; a tile of w < 32 columns is
+// read from (written to) the host side as one run of 32 w values where the
+// rows are that short.  Grid (column tiles, x tiles, variables).
 constexpr int LAY_T = 32;
 
-// host -> device: active cells of the reference layout
-__global__ __launch_bounds__(256) void k_ref_to_dev(const double* __restrict__ ref, double* __restrict__ dev, Geom g) {
+struct LayTile {
+    int x0, c0, w, rows;
+};
+__device__ __forceinline__ LayTile lay_tile(int ni, int ncol) {
+    LayTile t;
+    t.c0 = blockIdx.x * LAY_T;
+    t.x0 = blockIdx.y * LAY_T;
+    t.w = min(LAY_T, ncol - t.c0);
+    t.rows = min(LAY_T, ni - t.x0);
+    return t;
+}
+// device index of (x, column c)
+__device__ __forceinline__ size_t lay_dev(const Geom& g, int x, int j0, int c) {
+    const int j = c / g.n[2], k = c - j * g.n[2];
+    return ((size_t)k * g.n[1] + j0 + j) * g.n[0] + x;
+}
+
+__global__ __launch_bounds__(256) void k_ref_to_dev(const double* __restrict__ pin, double* __restrict__ dev, Geom g,
+                                                    int i0, int ni, int j0, int ncol) {
     __shared__ double t[LAY_T][LAY_T + 1];
-    const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    const size_t n6y = (size_t)ny + 6, n6z = (size_t)nz + 6;
-    const int z0 = blockIdx.x * LAY_T, x0 = blockIdx.y * LAY_T;
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    for (int y = blockIdx.z; y < ny; y += gridDim.z) {
-#pragma unroll
-        for (int r = 0; r < LAY_T; r += 8) {
-            const int x = x0 + ty + r, z = z0 + tx;
-            if (x < nx && z < nz) t[ty + r][tx] = ref[(((size_t)x + 3) * n6y + (size_t)y + 3) * n6z + (size_t)z + 3];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < LAY_T; r += 8) {
-            const int z = z0 + ty + r, x = x0 + tx;
-            if (x < nx && z < nz) dev[((size_t)z * ny + y) * nx + x] = t[tx][ty + r];
-        }
-        __syncthreads();
+    const LayTile T = lay_tile(ni, ncol);
+    pin += (size_t)blockIdx.z * ni * ncol;
+    dev += (size_t)blockIdx.z * g.ncell;
+    for (int e = threadIdx.x; e < T.rows * T.w; e += 256)
+        t[e / T.w][e % T.w] = pin[(size_t)(T.x0 + e / T.w) * ncol + T.c0 + e % T.w];
+    __syncthreads();
+    for (int e = threadIdx.x; e < T.w * LAY_T; e += 256) {
+        const int x = e % LAY_T, c = e / LAY_T;
+        if (x < T.rows) dev[lay_dev(g, i0 + T.x0 + x, j0, T.c0 + c)] = t[x][c];
     }
 }
 
-// device -> host: every cell of the reference layout, the ghost layers filled
-// with the active cells the boundary conditions map them to (src/bound.cpp)
-__global__ __launch_bounds__(256) void k_dev_to_ref(const double* __restrict__ dev, double* __restrict__ ref, Geom g) {
+__global__ __launch_bounds__(256) void k_dev_to_ref(const double* __restrict__ dev, double* __restrict__ pin, Geom g,
+                                                    int i0, int ni, int j0, int ncol) {
     __shared__ double t[LAY_T][LAY_T + 1];
-    const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    const int n6x = nx + 6, n6y = ny + 6, n6z = nz + 6;
-    const int k0 = blockIdx.x * LAY_T, i0 = blockIdx.y * LAY_T;
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    for (int j = blockIdx.z; j < n6y; j += gridDim.z) {
-        const size_t yo = (size_t)bmap(j - 3, ny, g.per[1]) * nx;
-#pragma unroll
-        for (int r = 0; r < LAY_T; r += 8) {
-            const int k = k0 + ty + r, i = i0 + tx;
-            if (i < n6x && k < n6z)
-                t[ty + r][tx] = dev[(size_t)bmap(k - 3, nz, g.per[2]) * ny * nx + yo + bmap(i - 3, nx, g.per[0])];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < LAY_T; r += 8) {
-            const int i = i0 + ty + r, k = k0 + tx;
-            if (i < n6x && k < n6z) ref[((size_t)i * n6y + j) * n6z + k] = t[tx][ty + r];
-        }
-        __syncthreads();
+    const LayTile T = lay_tile(ni, ncol);
+    pin += (size_t)blockIdx.z * ni * ncol;
+    dev += (size_t)blockIdx.z * g.ncell;
+    for (int e = threadIdx.x; e < T.w * LAY_T; e += 256) {
+        const int x = e % LAY_T, c = e / LAY_T;
+        if (x < T.rows) t[x][c] = dev[lay_dev(g, i0 + T.x0 + x, j0, T.c0 + c)];
     }
+    __syncthreads();
+    for (int e = threadIdx.x; e < T.rows * T.w; e += 256)
+        pin[(size_t)(T.x0 + e / T.w) * ncol + T.c0 + e % T.w] = t[e / T.w][e % T.w];
 }
 
 }  // namespace howmhd

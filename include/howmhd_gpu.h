@@ -101,8 +101,8 @@ typedef struct howmhd_timing {
 typedef struct howmhd_gpu_ctx howmhd_gpu_ctx;
 
 /* Allocates q (5 stage buffers), faces (5 stage buffers), the sweep / CT
- * scratch and a staging buffer for host transfers on the current HIP device;
- * no later call allocates device memory.  Replaces the allocation of q
+ * scratch on the current HIP device, and pinned host memory for host
+ * transfers; no later call allocates device memory.  Replaces the allocation of q
  * (src/main.cpp:114-120) and allocate_bfield_ct (src/fluxct.cpp:27-35).
  * Axes must have n == 1 (degenerate) or n >= 3; ny and nz at most 65535
  * (launch grid limit), at most 2^40 cells.  Bad parameters return
@@ -115,10 +115,11 @@ HOWMHD_API int howmhd_gpu_destroy(howmhd_gpu_ctx* ctx);
 /* Copies stage-0 q from the host (reference layout, ghosts ignored).  The
  * reference's problem initialisers write q(0,...) in place
  * (src/problem.cpp:39-59); this is the device hand-over of that array.
- * Host transfers (this call, upload_faces and the downloads) read or write
- * the caller's memory directly, one variable at a time, through the
- * context's device buffer of one variable's reference-layout size; the
- * layout change runs on the device.  Synchronises. */
+ * Host transfers (this call, upload_faces and the downloads) move the active
+ * cells in chunks through the context's pinned host memory (at most 32 MiB);
+ * up to eight host threads, joined before the call returns, copy between it
+ * and the caller's memory while the layout change runs on the device.
+ * Synchronises. */
 HOWMHD_API int howmhd_gpu_upload_q0(howmhd_gpu_ctx* ctx, const double* q0);
 
 /* bound(q,0) + initialize_bfield_from_q + bound_bfield(0)
