@@ -58,14 +58,16 @@ struct howmhd_gpu_ctx {
     int xfer_n = 0;
     std::vector<hipEvent_t> xfer_ev;
     // learned indicator: device weights, routing mode (0 off, 1 on with the
-    // plain-WENO fallback, 2 on for every step), the routed sweeps' counters
-    // per wavefront slot (nwave slots, cleared by each fold) and their
+    // plain-WENO fallback, 2 on for every step), the routed sweeps' counter
+    // words (per stage nwave words, four per tile of the x, y and z sweeps
+    // from tile slot tile0[d] on) and their
     // totals (flagged, total, wavefronts flagged, wavefronts total)
     howmhd::MlpDev* mlp = nullptr;
     int ind_mode = 0;
     bool route_now = false;              // the running step routes
-    uint4* iwave = nullptr;
+    unsigned* iwave = nullptr;
     long long nwave = 0;
+    long long tile0[3] = {0, 0, 0};
     // reference-rounding sweeps: tiles to recompute with IEEE divisions
     // (nwave / 4 flags and queue entries, kept zero/empty between sweeps;
     // queue length and blocks done)

@@ -260,12 +260,14 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         if (ok) c->xfer_ev.push_back(ev);
     }
     ok = ok && alloc((void**)&c->mlp, sizeof(MlpDev));
-    // one counter slot per wavefront of the largest sweep grid
+    // one slot per tile of the sweeps (x, y, z), four counter words each
     for (int d = 0; d < 3; ++d) {
         const dim3 gr = sweep_grid(c->g, d);
-        c->nwave = std::max(c->nwave, 4LL * gr.x * gr.y * gr.z);
+        c->tile0[d] = c->nwave / 4;
+        if (n[d] > 1) c->nwave += 4LL * gr.x * gr.y * gr.z;
     }
-    ok = ok && alloc((void**)&c->iwave, (size_t)c->nwave * sizeof(uint4));
+    c->nwave = std::max(c->nwave, 4LL);
+    ok = ok && alloc((void**)&c->iwave, 5 * (size_t)c->nwave * sizeof(unsigned));
     ok = ok && alloc((void**)&c->fixflag, (size_t)(c->nwave / 4) * sizeof(unsigned));
     ok = ok && alloc((void**)&c->fixlist, (size_t)(c->nwave / 4) * sizeof(unsigned));
     ok = ok && alloc((void**)&c->fixctl, 2 * sizeof(unsigned));
@@ -454,9 +456,10 @@ int howmhd_gpu_ssprk(howmhd_gpu_ctx* c, double dt) {
         // step's own (flagged, total) (slots cleared)
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->ilast, 2);
         HCHECK(c, hipGetLastError());
-        const unsigned nb = std::min(1024u, blocks_for((size_t)c->nwave, 256));
-        hipLaunchKernelGGL(k_fold_wave_stats, dim3(nb), dim3(256), 0, c->stream, c->iwave, c->nwave, c->istats,
-                           c->ilast);
+        const long long ntile = 5 * c->nwave / 4;
+        const unsigned nb = std::min(1024u, blocks_for((size_t)ntile, 256));
+        hipLaunchKernelGGL(k_fold_wave_stats, dim3(nb), dim3(256), 0, c->stream, (const uint4*)c->iwave, ntile,
+                           c->istats, c->ilast);
         HCHECK(c, hipGetLastError());
         c->any_routed = true;
     }
@@ -636,7 +639,7 @@ int howmhd_gpu_set_indicator(howmhd_gpu_ctx* c, const float* params, float thres
     HCHECK(c, hipMemsetAsync(c->istats, 0, 4 * sizeof(unsigned long long), c->stream));
     HCHECK(c, hipMemsetAsync(c->ilast, 0, 2 * sizeof(unsigned long long), c->stream));
     c->any_routed = false;
-    HCHECK(c, hipMemsetAsync(c->iwave, 0, (size_t)c->nwave * sizeof(uint4), c->stream));
+    HCHECK(c, hipMemsetAsync(c->iwave, 0, 5 * (size_t)c->nwave * sizeof(unsigned), c->stream));
     HCHECK(c, hipStreamSynchronize(c->stream));
     c->istats_pending = false;
     c->fallback_left = 0;

@@ -88,20 +88,18 @@ struct Phys {
 };
 
 // ------------------------------------------------------------- sweep tiling
-// X sweep: 64 interfaces along x per row, 4 rows (y) per block.
-// Y/Z sweep: HOWMHD_YZ_LANES x-columns, 256/HOWMHD_YZ_LANES interfaces along the
-// sweep axis per block.
-template <int DIR> struct SweepTile;
-template <> struct SweepTile<0> {
+// Two tile shapes.  ALONG_X (x sweep): 64 interfaces along x per row, 4 rows
+// (y) per block.  ACROSS_X (y and z sweeps): HOWMHD_YZ_LANES x-columns,
+// 256/HOWMHD_YZ_LANES interfaces along the sweep axis per block.
+enum TileShape { ALONG_X = 0, ACROSS_X = 1 };
+template <int TS> struct SweepTile;
+template <> struct SweepTile<ALONG_X> {
     static constexpr int LANES = 64, ROWS = 4, CELLS = (64 + 5) * 4;
 };
 #ifndef HOWMHD_YZ_LANES
 #define HOWMHD_YZ_LANES 32
 #endif
-template <> struct SweepTile<1> {
-    static constexpr int LANES = HOWMHD_YZ_LANES, ROWS = 256 / HOWMHD_YZ_LANES, CELLS = LANES * (ROWS + 5);
-};
-template <> struct SweepTile<2> {
+template <> struct SweepTile<ACROSS_X> {
     static constexpr int LANES = HOWMHD_YZ_LANES, ROWS = 256 / HOWMHD_YZ_LANES, CELLS = LANES * (ROWS + 5);
 };
 
@@ -121,12 +119,14 @@ template <> struct SweepTile<2> {
 
 __host__ __device__ inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// Launch grid of the sweep along axis d (256-thread blocks; SweepTile).
+// Tiles of the sweep along axis d: (x tiles, tiles along the second axis,
+// planes).
 __host__ __device__ inline dim3 sweep_grid(const Geom& g, int d) {
     const int nif = g.per[d] ? g.n[d] : g.n[d] + 1;
-    if (d == 0) return dim3(blocks_for(nif, SweepTile<0>::LANES), blocks_for(g.n[1], SweepTile<0>::ROWS), g.n[2]);
-    if (d == 1) return dim3(blocks_for(g.n[0], SweepTile<1>::LANES), blocks_for(nif, SweepTile<1>::ROWS), g.n[2]);
-    return dim3(blocks_for(g.n[0], SweepTile<2>::LANES), blocks_for(nif, SweepTile<2>::ROWS), g.n[1]);
+    using X = SweepTile<ALONG_X>;
+    using T = SweepTile<ACROSS_X>;
+    if (d == 0) return dim3(blocks_for(nif, X::LANES), blocks_for(g.n[1], X::ROWS), g.n[2]);
+    return dim3(blocks_for(g.n[0], T::LANES), blocks_for(nif, T::ROWS), d == 1 ? g.n[2] : g.n[1]);
 }
 
 // Sweep variants: plain characteristic WENO5; the same plus indicator
@@ -135,41 +135,83 @@ __host__ __device__ inline dim3 sweep_grid(const Geom& g, int d) {
 // upwind-5 on the components).
 enum SweepMode { SW_PLAIN = 0, SW_COLLECT = 1, SW_ROUTED = 2 };
 
+// Division of n < 2^31 by a constant of the launch: q = n m >> sh with
+// m = ceil(2^sh / d), sh = 31 + ceil(log2 d); exact, because m d - 2^sh < d
+// <= 2^(sh - 31).  Three scalar instructions, where an unsigned division
+// takes some 25 vector ones of every wavefront (two of them were 1.5% of an
+// FP32 routed step).
+struct LaunchDiv {
+    unsigned d, m, sh;
+};
+inline LaunchDiv launch_div(unsigned d) {
+    unsigned l = 0;
+    while ((1ull << l) < d) ++l;
+    return LaunchDiv{d, (unsigned)(((1ull << (31 + l)) + d - 1) / d), 31 + l};
+}
+__host__ __device__ __forceinline__ unsigned div(unsigned n, const LaunchDiv& v) {
+    return (unsigned)(((unsigned long long)n * v.m) >> v.sh);
+}
+
+// What one axis of a launch needs: its arrays, the strides that make the y
+// and z sweeps one code (cells, interfaces t = 0..n of dF and samples lie on
+// lines along the sweep axis; `other` is the axis that is neither x nor the
+// sweep axis), and its place in the launch.
+template <typename R>
+struct SweepAxis {
+    R* dF;              // 7 components, cF apart
+    R* ct_a;            // CT term "bsy": fsy (x), gsz (y), hsx (z)
+    R* ct_b;            // CT term "bsz": fsz (x), gsx (y), hsy (z)
+    long long qoff[8];  // offset of the variable in sweep slot m (sweep_perm)
+    int n, per, nother; // cells along the axis; periodic; cells of `other`
+    // cell and interface indices fit 32 bits: a context of 2^32 / 2 cells
+    // would need more than four times the 288 GB of the device
+    unsigned sA, sB;    // cell strides along the axis and along `other`
+    unsigned tF, oF;    // dF strides: interface, other (components: cF)
+    long long cF;
+    unsigned sS, oS;    // sample strides: interface, other
+    unsigned gx, gy, gz;   // tiles (sweep_grid)
+    LaunchDiv by_gx, by_gy; // by gx, and by the blocks along gy
+    unsigned first;     // first block of the launch on this axis
+    int march;          // consecutive tiles along the axis per block
+    long long tile0;    // first tile slot of the axis (queue, statistics)
+};
+
 template <typename R>
 struct SweepArgs {
     const double* q;    // source stage, 8 arrays of ncell
-    R* dF;              // 7 x n_if planes (see dF_index)
     // constrained transport active: components 4, 5 of dF (the
     // transverse-B fluxes) feed only the CT terms, not k_combine, and are
     // not stored
     int ct_active;
-    R* ct_a;            // CT term "bsy": fsy (x), gsz (y), hsx (z)
-    R* ct_b;            // CT term "bsz": fsz (x), gsx (y), hsy (z)
     Geom g;
     Phys ph;
     GasConst gc;
-    // SW_COLLECT: 18 features and the label per interface (sample_index), and
-    // (when logit is set) the in-sweep network's logit
+    // SW_COLLECT: 18 features and the label per interface (dense: the lines
+    // of the sweep, each with its computed interfaces in order), and (when
+    // logit is set) the in-sweep network's logit
     float* feat;
     float* label;
     float* logit;
-    // SW_ROUTED: device weights; stats (null: not counted): one slot per
-    // wavefront of the launch grid (block-linear index x 4 + wavefront), to
-    // which the wavefront adds (flagged, total, 1 if any flagged, 1): plain
-    // read-modify-writes (every slot has one writer per launch) that
-    // k_fold_wave_stats sums and clears after the step
+    // SW_ROUTED: device weights; stats (null: not counted): one word per
+    // wavefront of every tile (tile slot x 4 + wavefront) of the stage, in
+    // which the wavefront leaves flagged | valid << 8, its lanes of each kind.
+    // Every wavefront writes its word in every routed stage, so nothing is
+    // read or cleared; k_fold_wave_stats sums the words of the five stages
+    // after the step.  (Adding to a slot of four counters, read and written
+    // by each stage, held every wavefront up: routed FP32 sweeps at 256^3
+    // 0.46-0.48 ms, against 0.43-0.44 without counting.)
     const MlpDev* mlp;
-    uint4* stats;
+    unsigned* stats;
     // reference-rounding form: tiles whose WENO weight operands left the
     // range of the unscaled division, for the IEEE-division launch that
-    // follows: a flag per tile (block-linear index, so a tile is queued
-    // once), the queue, and (queue length, blocks done) of that launch
+    // follows: a flag per tile slot (a tile is queued once), the queue, and
+    // (queue length, blocks done) of that launch
     unsigned* fix;
     unsigned* fixlist;
     unsigned* fixctl;
-    // y/z sweeps: consecutive tiles along the sweep axis per block
-    // (sweep_march; 1: single tiles)
-    int march;
+    // the axes of the launch in the order of their blocks: y, z, x (an axis
+    // without blocks starts where the next one does)
+    SweepAxis<R> ax[3];
 };
 
 // dF layout per direction: component-major, interface index t = 0..n along the
@@ -182,17 +224,6 @@ __device__ __forceinline__ long long dF_index(const Geom& g, int c, int t, int x
     if constexpr (DIR == 0) return (((long long)c * g.n[2] + z) * g.n[1] + y) * (g.n[0] + 1) + t;
     else if constexpr (DIR == 1) return (((long long)c * g.n[2] + z) * (g.n[1] + 1) + t) * g.n[0] + x;
     else return (((long long)c * (g.n[2] + 1) + t) * g.n[1] + y) * g.n[0] + x;
-}
-
-// Dense index of a sampled interface: the lines of the sweep, each with its
-// computed interfaces t = tbeg..n (tbeg = 1 periodic, 0 open) in order.
-template <int DIR>
-__device__ __forceinline__ long long sample_index(const Geom& g, int t, int x, int y, int z) {
-    const int tbeg = g.per[DIR] ? 1 : 0;
-    const long long nint = g.n[DIR] + 1 - tbeg, u = t - tbeg;
-    if constexpr (DIR == 0) return ((long long)z * g.n[1] + y) * nint + u;
-    else if constexpr (DIR == 1) return ((long long)z * nint + u) * g.n[0] + x;
-    else return (u * g.n[1] + y) * g.n[0] + x;
 }
 
 template <int B, int E, typename F>
@@ -243,14 +274,14 @@ __device__ __forceinline__ void opaque(Eig<R>& o) {
 // eigensystem, the 7 wave maxima, then the waves in pairs, added to dFo in
 // wave order.  The WENO weights divide in mode DM (DivMode); `bad` collects
 // the lanes whose operands left the range of the unscaled division.
-template <typename R, int DIR, int MODE, int DM>
-__device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<DIR>::CELLS],
-                                               const R (*lo)[SweepTile<DIR>::CELLS], int row, int lane, R gam,
+template <typename R, int TS, int MODE, int DM>
+__device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>::CELLS],
+                                               const R (*lo)[SweepTile<TS>::CELLS], int row, int lane, R gam,
                                                const GasConst& gc, R (&dFo)[7], R& mdev, unsigned long long& bad) {
-    using T = SweepTile<DIR>;
+    using T = SweepTile<TS>;
     (void)mdev;
     auto slot = [&](int k) -> int {
-        if constexpr (DIR == 0) return row * (T::LANES + 5) + lane + k;
+        if constexpr (TS == ALONG_X) return row * (T::LANES + 5) + lane + k;
         else return (row + k) * T::LANES + lane;
     };
     // interface state from cells k = 2, 3: (rho, vn, vt1, vt2, Bn, Bt1, Bt2, p, H)
@@ -418,75 +449,105 @@ constexpr bool sweep_marches() { return sizeof(R) == 8 && MODE != SW_COLLECT; }
 
 // Stored index of slot s of the LDS tile whose first interface is t0 (the
 // tile's cells run from t0 - 3 to t0 + ROWS + 1 along the sweep axis, x
-// sweep: t0 - 3 to t0 + LANES + 1), through the boundary map.
-template <int DIR>
-__device__ __forceinline__ long long tile_cell_index(const Geom& g, int s, int t0, int x0, int y0, int z0) {
-    using T = SweepTile<DIR>;
-    const int nd = g.n[DIR];
-    int cx, cy, cz, along;
-    if constexpr (DIR == 0) {
+// sweep: t0 - 3 to t0 + LANES + 1), through the boundary map.  (x0, o0):
+// first column and other coordinate (ACROSS_X); (y0, z0) of the rows
+// (ALONG_X).
+template <typename R, int TS>
+__device__ __forceinline__ unsigned tile_cell_index(const Geom& g, const SweepAxis<R>& X, int s, int t0, int a0,
+                                                     int b0) {
+    using T = SweepTile<TS>;
+    int along;
+    unsigned base;
+    if constexpr (TS == ALONG_X) {
         const int row = s / (T::LANES + 5), c = s % (T::LANES + 5);
         along = t0 - 3 + c;
-        cy = y0 + row; cz = z0; cx = 0;
+        int cy = a0 + row;
         if (cy >= g.n[1]) cy = g.n[1] - 1;
+        base = ((unsigned)b0 * g.n[1] + cy) * (unsigned)g.n[0];
     } else {
         const int row = s / T::LANES, lane = s % T::LANES;
         along = t0 - 3 + row;
-        cx = x0 + lane;
+        int cx = a0 + lane;
         if (cx >= g.n[0]) cx = g.n[0] - 1;
-        if constexpr (DIR == 1) { cz = z0; cy = 0; }
-        else { cy = y0; cz = 0; }
+        base = cx + (unsigned)b0 * X.sB;
     }
-    if (along > nd + 2) along = nd + 2;
-    const int a = bmap(along, nd, g.per[DIR]);
-    if constexpr (DIR == 0) cx = a;
-    else if constexpr (DIR == 1) cy = a;
-    else cz = a;
-    return ((long long)cz * g.n[1] + cy) * g.n[0] + cx;
+    if (along > X.n + 2) along = X.n + 2;
+    const int a = bmap(along, X.n, X.per);
+    if constexpr (TS == ALONG_X) return base + a;
+    else return base + (unsigned)a * X.sA;
+}
+
+// The LDS of a tile: (U_j, F_j) pairs, the other cell fields, and |B| of each
+// cell for the indicator features (routed and sample sweeps).
+template <typename R, int TS>
+struct TileLds {
+    static constexpr int CELLS = SweepTile<TS>::CELLS;
+    UF<R> (*luf)[CELLS];
+    R (*lo)[CELLS];
+    float* lbmag;
+};
+template <typename R, int MODE, int TS>
+constexpr int tile_lds_bytes() {
+    return SweepTile<TS>::CELLS * (int)(7 * sizeof(UF<R>) + O_COUNT * sizeof(R) + (MODE != SW_PLAIN ? sizeof(float) : 0));
+}
+template <typename R, int TS>
+__device__ __forceinline__ TileLds<R, TS> tile_lds(unsigned char* raw) {
+    TileLds<R, TS> L;
+    L.luf = reinterpret_cast<UF<R>(*)[SweepTile<TS>::CELLS]>(raw);
+    L.lo = reinterpret_cast<R(*)[SweepTile<TS>::CELLS]>(raw + SweepTile<TS>::CELLS * 7 * sizeof(UF<R>));
+    L.lbmag = reinterpret_cast<float*>(raw + SweepTile<TS>::CELLS * (7 * sizeof(UF<R>) + O_COUNT * sizeof(R)));
+    return L;
 }
 
 // Cell values of one cell (its 8 conserved values in sweep order) into LDS
 // slot s.
-template <typename R, int DIR, int MODE, int DM>
-__device__ __forceinline__ void store_cell(const SweepArgs<R>& A, UF<R> (*luf)[SweepTile<DIR>::CELLS],
-                                           R (*lo)[SweepTile<DIR>::CELLS], float* lbmag, int s, const double* q,
+template <typename R, int TS, int MODE, int DM>
+__device__ __forceinline__ void store_cell(const SweepArgs<R>& A, const TileLds<R, TS>& L, int s, const double* q,
                                            bool& cell_bad) {
     R out[C_NFIELD];
     cell_values<R, DM>(q, A.ph.gam, A.ph.rhomin, A.ph.pgmin, out, &cell_bad);
 #pragma unroll
-    for (int j = 0; j < 7; ++j) luf[j][s] = UF<R>{out[C_RHO + j], out[C_F0 + j]};
+    for (int j = 0; j < 7; ++j) L.luf[j][s] = UF<R>{out[C_RHO + j], out[C_F0 + j]};
 #pragma unroll
-    for (int f = 0; f < O_COUNT; ++f) lo[f][s] = out[C_VN + f];
+    for (int f = 0; f < O_COUNT; ++f) L.lo[f][s] = out[C_VN + f];
     if constexpr (MODE != SW_PLAIN)
-        lbmag[s] = sqrtf((float)(out[C_BN] * out[C_BN] + out[C_BT1] * out[C_BT1] + out[C_BT2] * out[C_BT2]));
+        L.lbmag[s] = sqrtf((float)(out[C_BN] * out[C_BN] + out[C_BT1] * out[C_BT1] + out[C_BT2] * out[C_BT2]));
 }
 
 // Phase 2 of a tile whose cell values are in LDS: one interface per thread
-// (t0, x0, y0, z0: the tile origin; blk: its index in the single-tile grid).
-template <typename R, int DIR, int MODE, int EX, int DM>
-__device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF<R> (*luf)[SweepTile<DIR>::CELLS],
-                                                 const R (*lo)[SweepTile<DIR>::CELLS], const float* lbmag, int t0,
-                                                 int x0, int y0, int z0, long long blk) {
-    using T = SweepTile<DIR>;
+// (t0, a0, b0: the tile origin; slot: its tile slot).
+template <typename R, int TS, int MODE, int EX, int DM>
+__device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const SweepAxis<R>& X, const TileLds<R, TS>& L,
+                                                 int t0, int a0, int b0, long long tslot) {
+    using T = SweepTile<TS>;
     const Geom& g = A.g;
-    const int nd = g.n[DIR];
-    const int tid = threadIdx.x;
-    int lane, row, t, x, y, z;
+    const int nd = X.n;
+    // opaque, so that a march computes its addresses in every step instead of
+    // holding them in registers across the interfaces
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const auto luf = const_cast<const UF<R>(*)[T::CELLS]>(L.luf);
+    const auto lo = const_cast<const R(*)[T::CELLS]>(L.lo);
+    const float* lbmag = L.lbmag;
+    const int lane = tid % T::LANES, row = tid / T::LANES;
+    int t, x, o;  // interface; ALONG_X: (y, z) = (x, o), ACROSS_X: column and other coordinate
     bool valid;
-    if constexpr (DIR == 0) {
-        lane = tid % T::LANES; row = tid / T::LANES;
-        t = t0 + lane; x = 0; y = y0 + row; z = z0;
-        valid = (t <= nd && y < g.n[1]);
+    if constexpr (TS == ALONG_X) {
+        t = t0 + lane; x = a0 + row; o = b0;
+        valid = (t <= nd && x < g.n[1]);
     } else {
-        lane = tid % T::LANES; row = tid / T::LANES;
-        t = t0 + row; x = x0 + lane;
-        if constexpr (DIR == 1) { y = 0; z = z0; }
-        else { y = y0; z = 0; }
+        t = t0 + row; x = a0 + lane; o = b0;
         valid = (t <= nd && x < g.n[0]);
     }
     auto slot = [&](int k) -> int {
-        if constexpr (DIR == 0) return row * (T::LANES + 5) + lane + k;
+        if constexpr (TS == ALONG_X) return row * (T::LANES + 5) + lane + k;
         else return (row + k) * T::LANES + lane;
+    };
+    // index of interface u = t - tbeg among the samples
+    auto sample = [&]() -> unsigned {
+        const unsigned u = t - (X.per ? 1 : 0);
+        if constexpr (TS == ALONG_X) return ((unsigned)o * g.n[1] + x) * X.oS + u;
+        else return u * X.sS + (unsigned)o * X.oS + x;
     };
     // indicator features: the 6-cell stencils of rho, p and |B|
     auto features = [&](float* f) {
@@ -506,7 +567,7 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF
             float f[MLP_IN];
             features(f);
             const float zl = mlp_forward_wave(f, *A.mlp);
-            if (valid) A.logit[sample_index<DIR>(g, t, x, y, z)] = zl;
+            if (valid) A.logit[sample()] = zl;
         }
     }
     if constexpr (MODE == SW_ROUTED) {
@@ -516,15 +577,7 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF
         flagged = valid && (zl > A.mlp->logit_threshold);
         if (A.stats) {
             const unsigned long long fb = __ballot(flagged), vb = __ballot(valid);
-            if ((tid & 63) == 0 && vb) {
-                uint4* st = A.stats + 4 * blk + (tid >> 6);
-                uint4 v = *st;
-                v.x += (unsigned)__popcll(fb);
-                v.y += (unsigned)__popcll(vb);
-                v.z += fb ? 1u : 0u;
-                v.w += 1u;
-                *st = v;
-            }
+            if ((tid & 63) == 0) A.stats[4 * tslot + (tid >> 6)] = (unsigned)__popcll(fb) | (unsigned)__popcll(vb) << 8;
         }
     }
     if (!valid) return;
@@ -533,11 +586,11 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF
     R maxdev = R(0);
     if (MODE != SW_ROUTED || flagged) {
         unsigned long long bad = 0ull;
-        weno_interface<R, DIR, MODE, DM>(luf, lo, row, lane, R(A.ph.gam), A.gc, dF, maxdev, bad);
+        weno_interface<R, TS, MODE, DM>(luf, lo, row, lane, R(A.ph.gam), A.gc, dF, maxdev, bad);
         // a WENO weight operand beyond the unscaled-division range: the tile
         // goes (once) on the list of the IEEE-division launch that follows
         if constexpr (EX && DM == DIV_UNSCALED) {
-            if (bad && atomicExch(&A.fix[blk], 1u) == 0u) A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)blk;
+            if (bad && atomicExch(&A.fix[tslot], 1u) == 0u) A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)tslot;
         }
     } else {
         // linear upwind-5 with one LLF speed: the largest |v_n| + c_f over the
@@ -561,9 +614,19 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF
         }
     }
 
+    // dF and (below) the CT terms of the cell left of the interface
+    unsigned fi, ci;
+    if constexpr (TS == ALONG_X) {
+        const unsigned r = (unsigned)o * g.n[1] + x;
+        fi = r * (nd + 1) + t;
+        ci = r * nd + (t - 1);
+    } else {
+        fi = (unsigned)o * X.oF + t * X.tF + x;
+        ci = (unsigned)o * X.sB + (unsigned)(t - 1) * X.sA + x;
+    }
 #pragma unroll
     for (int c = 0; c < 7; ++c)
-        if (!(A.ct_active && (c == 4 || c == 5))) st_nt(&A.dF[dF_index<DIR>(g, c, t, x, y, z)], dF[c]);
+        if (!(A.ct_active && (c == 4 || c == 5))) st_nt(&X.dF[c * X.cF + fi], dF[c]);
 
     // CT flux terms, src/ssprk.cpp:967-994: (-0 a + 9 b + 9 c - 0 d)/18 over
     // cells k = 1..4.  The products with the zero weights are +-0 and are
@@ -580,188 +643,128 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const UF
         }
         const R ftmp1 = div_c<R>(R(9) * bnv1[0] + R(9) * bnv1[1], R(18), R(1.0 / 18.0));
         const R ftmp2 = div_c<R>(R(9) * bnv2[0] + R(9) * bnv2[1], R(18), R(1.0 / 18.0));
-        long long ci;
-        if constexpr (DIR == 0) ci = ((long long)z * g.n[1] + y) * g.n[0] + (t - 1);
-        else if constexpr (DIR == 1) ci = ((long long)z * g.n[1] + (t - 1)) * g.n[0] + x;
-        else ci = ((long long)(t - 1) * g.n[1] + y) * g.n[0] + x;
-        st_nt(&A.ct_a[ci], dF[4] + ftmp1);
-        st_nt(&A.ct_b[ci], dF[5] + ftmp2);
+        st_nt(&X.ct_a[ci], dF[4] + ftmp1);
+        st_nt(&X.ct_b[ci], dF[5] + ftmp2);
     }
     if constexpr (MODE == SW_COLLECT) {
         if (!A.feat) return;
         float f[MLP_IN];
         features(f);
-        const long long si = sample_index<DIR>(g, t, x, y, z);
+        const size_t si = sample();
 #pragma unroll
         for (int j = 0; j < MLP_IN; ++j) A.feat[si * MLP_IN + j] = f[j];
         A.label[si] = (maxdev > R(0.05)) ? 1.f : 0.f;
     }
 }
 
-// One tile (bx, by, bz) of the sweep grid (sweep_grid), block-linear index
-// blk.  DM (DivMode) of the WENO weights: the FMA forms and the
-// reference-rounding recompute launch divide with IEEE divisions; the
+// Up to `nsteps` consecutive tiles (bx, by0 ..) of plane bz along the sweep
+// axis (ALONG_X: one).  DM (DivMode) of the WENO weights: the FMA forms and
+// the reference-rounding recompute launch divide with IEEE divisions; the
 // reference-rounding sweep proper with div_recip/div_with, queueing its tile
 // for the recompute launch where an operand leaves their range.
-template <typename R, int DIR, int MODE, int EX, int DM>
-__device__ __forceinline__ void sweep_tile(const SweepArgs<R>& A, int bx, int by, int bz, long long blk) {
-    using T = SweepTile<DIR>;
-    __shared__ UF<R> luf[7][T::CELLS];
-    __shared__ R lo[O_COUNT][T::CELLS];
-    // |B| of each cell for the indicator features (routed and sample sweeps)
-    __shared__ float lbmag[MODE != SW_PLAIN ? T::CELLS : 1];
-    const Geom& g = A.g;
-    const int tbeg = g.per[DIR] ? 1 : 0;  // periodic: interface 0 is the image of n
-    const int tid = threadIdx.x;
-
-    // block origin
-    int t0, x0 = 0, y0 = 0, z0 = 0;
-    if constexpr (DIR == 0) {
-        t0 = tbeg + bx * T::LANES;
-        y0 = by * T::ROWS;
-        z0 = bz;
-    } else {
-        x0 = bx * T::LANES;
-        t0 = tbeg + by * T::ROWS;
-        if constexpr (DIR == 1) z0 = bz;
-        else y0 = bz;
-    }
-
-    // ---- phase 1: cell values of the tile (stencil halo included) into LDS.
-    // A thread's cells are tid, tid + 256, ...; all their loads are issued
-    // before the first conversion, so a block waits on memory once.
-    auto cell_index = [&](int s) -> long long { return tile_cell_index<DIR>(g, s, t0, x0, y0, z0); };
-    constexpr int NIT = (T::CELLS + 255) / 256;
-    double qs[NIT][8];
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-        const int s = tid + 256 * it;
-        if (s < T::CELLS) {
-            const long long idx = cell_index(s);
-#pragma unroll
-            for (int m = 0; m < 8; ++m) qs[it][m] = A.q[(long long)sweep_perm(DIR, m) * g.ncell + idx];
-        }
-    }
-    bool cell_bad = false;
-#pragma unroll
-    for (int it = 0; it < NIT; ++it) {
-        const int s = tid + 256 * it;
-        if (s < T::CELLS) store_cell<R, DIR, MODE, DM>(A, luf, lo, lbmag, s, qs[it], cell_bad);
-    }
-    // a cell without positive shared reciprocals: the tile goes (once) on the
-    // list of the IEEE-division launch that follows
-    if constexpr (EX && DM == DIV_UNSCALED) {
-        if (__ballot(cell_bad) && atomicExch(&A.fix[blk], 1u) == 0u)
-            A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)blk;
-    }
-    __syncthreads();
-
-    sweep_interfaces<R, DIR, MODE, EX, DM>(A, luf, lo, lbmag, t0, x0, y0, z0, blk);
-}
-
-// The y or z sweep of up to `nsteps` consecutive tiles along the sweep axis
-// (tiles by0, by0 + 1, ... of the single-tile grid) by one block.
-// Consecutive tiles share 5 of their 13 cell rows: each step after the first
-// moves rows 8..12 of the previous tile to rows 0..4 of the LDS tile and
-// converts only its 8 new rows, one cell per thread.  Every value is the one
-// sweep_tile computes for the same tile; queueing and statistics use the
-// tile's single-tile index.
-template <typename R, int DIR, int MODE, int EX, int DM>
-__device__ __forceinline__ void sweep_march(const SweepArgs<R>& A, int bx, int by0, int bz, int nsteps) {
-    static_assert(DIR != 0, "the x sweep takes single tiles");
-    using T = SweepTile<DIR>;
+//
+// Phase 1 puts the cell values of the tile (stencil halo included) into LDS,
+// phase 2 computes one interface per thread.  Consecutive y/z tiles share 5
+// of their 13 cell rows: each step after the first moves rows 8..12 of the
+// previous tile to rows 0..4 of the LDS tile and converts only its 8 new
+// rows, one cell per thread.  Every value is the one a single tile computes;
+// queueing and statistics use the tile's own slot.
+template <typename R, int TS, int MODE, int EX, int DM>
+__device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAxis<R>& X, unsigned char* raw, int bx,
+                                            int by0, int bz, int nsteps) {
+    using T = SweepTile<TS>;
+    constexpr bool MARCH = TS == ACROSS_X && sweep_marches<R, MODE>() && !(EX && DM == DIV_IEEE);
     constexpr int HALO = 5 * T::LANES;        // slots of rows 0..4
     constexpr int NEW = T::CELLS - HALO;      // slots of rows 5..12
     constexpr int KEEP = T::ROWS * T::LANES;  // first slot of rows 8..12
-    static_assert(NEW == 256 && KEEP + HALO == T::CELLS, "one new cell per thread");
-    __shared__ UF<R> luf[7][T::CELLS];
-    __shared__ R lo[O_COUNT][T::CELLS];
-    __shared__ float lbmag[MODE != SW_PLAIN ? T::CELLS : 1];
+    static_assert(!MARCH || (NEW == 256 && KEEP + HALO == T::CELLS), "one new cell per thread");
+    const TileLds<R, TS> L = tile_lds<R, TS>(raw);
     const Geom& g = A.g;
-    const int tbeg = g.per[DIR] ? 1 : 0;
+    const int tbeg = X.per ? 1 : 0;  // periodic: interface 0 is the image of n
     const int tid = threadIdx.x;
-    const dim3 tg = sweep_grid(g, DIR);  // the single-tile grid
-    const int x0 = bx * T::LANES;
-    int y0 = 0, z0 = 0;
-    if constexpr (DIR == 1) z0 = bz;
-    else y0 = bz;
-    static_assert(sweep_marches<R, MODE>(), "a sweep with registers for the march");
+    const int gy = (int)X.gy;
+    // tile origin: first interface, first column (ALONG_X: first row y), plane
+    auto first_if = [&](int by) { return tbeg + (TS == ALONG_X ? bx * T::LANES : by * T::ROWS); };
+    const int a0 = TS == ALONG_X ? by0 * T::ROWS : bx * T::LANES;
+    auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * (by + (long long)gy * bz); };
+    // a cell without positive shared reciprocals: the tile goes (once) on the
+    // list of the IEEE-division launch that follows
+    auto queue = [&](bool bad, long long slot) {
+        if constexpr (EX && DM == DIV_UNSCALED) {
+            if (__ballot(bad) && atomicExch(&A.fix[slot], 1u) == 0u)
+                A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)slot;
+        }
+    };
     // Loads of the next step's cell issued before the interfaces of this
     // step: only where the 16 registers they hold leave the interfaces
     // without spills (the plain sweep of reference rounding); elsewhere each
     // step loads its cell at its start.
-    constexpr bool EARLY = EX && MODE == SW_PLAIN;
+    constexpr bool EARLY = MARCH && EX && MODE == SW_PLAIN;
     double qn[8];            // this thread's new cell of the next step
     bool bad_prev = false;   // this thread converted a cell out of range in the previous step
+    const int by1 = MARCH ? min(by0 + nsteps, gy) : by0 + 1;
     auto load_new = [&](int t0) {  // the new cell of the tile starting at row t0
-        const long long idx = tile_cell_index<DIR>(g, HALO + tid, t0, x0, y0, z0);
+        const unsigned idx = tile_cell_index<R, TS>(g, X, HALO + tid, t0, a0, bz);
 #pragma unroll
-        for (int m = 0; m < 8; ++m) qn[m] = A.q[(long long)sweep_perm(DIR, m) * g.ncell + idx];
+        for (int m = 0; m < 8; ++m) qn[m] = A.q[X.qoff[m] + idx];
     };
-    // queueing of a tile (see sweep_tile) and the early loads
-    auto finish_cells = [&](bool cell_bad, int by, int t0, long long blk) {
-        if constexpr (EX && DM == DIV_UNSCALED) {
-            if (__ballot(cell_bad || bad_prev) && atomicExch(&A.fix[blk], 1u) == 0u)
-                A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)blk;
-        }
+    auto finish = [&](int by, bool cell_bad) {
+        const int t0 = first_if(by);
+        queue(cell_bad || bad_prev, tile_slot(by));
         bad_prev = cell_bad;
         if constexpr (EARLY) {
-            if (by + 1 < by0 + nsteps && by + 1 < (int)tg.y) load_new(t0 + T::ROWS);
+            if (by + 1 < by1) load_new(t0 + T::ROWS);
         }
+        __syncthreads();  // the tile's cells are in LDS
+        sweep_interfaces<R, TS, MODE, EX, DM>(A, X, L, t0, a0, bz, tile_slot(by));
     };
-    if (by0 >= (int)tg.y) return;  // uniform over the block
-    // first tile: every cell, as sweep_tile
     {
-        const int t0 = tbeg + by0 * T::ROWS;
-        const long long blk = bx + (long long)tg.x * (by0 + (long long)tg.y * bz);
-        bool cell_bad = false;
+        // A thread's cells are tid, tid + 256, ...; all their loads are
+        // issued before the first conversion, so a block waits on memory once.
         constexpr int NIT = (T::CELLS + 255) / 256;
         double qs[NIT][8];
+        bool cell_bad = false;
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
             const int s = tid + 256 * it;
             if (s < T::CELLS) {
-                const long long idx = tile_cell_index<DIR>(g, s, t0, x0, y0, z0);
+                const unsigned idx = tile_cell_index<R, TS>(g, X, s, first_if(by0), a0, bz);
 #pragma unroll
-                for (int m = 0; m < 8; ++m) qs[it][m] = A.q[(long long)sweep_perm(DIR, m) * g.ncell + idx];
+                for (int m = 0; m < 8; ++m) qs[it][m] = A.q[X.qoff[m] + idx];
             }
         }
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
             const int s = tid + 256 * it;
-            if (s < T::CELLS) store_cell<R, DIR, MODE, DM>(A, luf, lo, lbmag, s, qs[it], cell_bad);
+            if (s < T::CELLS) store_cell<R, TS, MODE, DM>(A, L, s, qs[it], cell_bad);
         }
-        finish_cells(cell_bad, by0, t0, blk);
-        __syncthreads();  // the tile's cells are in LDS
-        sweep_interfaces<R, DIR, MODE, EX, DM>(A, luf, lo, lbmag, t0, x0, y0, z0, blk);
+        finish(by0, cell_bad);
     }
-    for (int by = by0 + 1; by < by0 + nsteps && by < (int)tg.y; ++by) {  // uniform over the block
-        const int t0 = tbeg + by * T::ROWS;
-        const long long blk = bx + (long long)tg.x * (by + (long long)tg.y * bz);
-        if constexpr (!EARLY) load_new(t0);
-        __syncthreads();  // every interface of the previous tile has read it
-        // rows 8..12 of the previous tile are rows 0..4 of this one (source
-        // and destination slots are disjoint)
-        if (tid < HALO) {
-            const int src = KEEP + tid;
-            UF<R> u[7];
-            R o[O_COUNT];
+    if constexpr (MARCH) {
+        for (int by = by0 + 1; by < by1; ++by) {  // uniform over the block
+            if constexpr (!EARLY) load_new(first_if(by));
+            __syncthreads();  // every interface of the previous tile has read it
+            // rows 8..12 of the previous tile are rows 0..4 of this one (source
+            // and destination slots are disjoint)
+            if (tid < HALO) {
+                const int src = KEEP + tid;
+                UF<R> u[7];
+                R o[O_COUNT];
 #pragma unroll
-            for (int j = 0; j < 7; ++j) u[j] = luf[j][src];
+                for (int j = 0; j < 7; ++j) u[j] = L.luf[j][src];
 #pragma unroll
-            for (int f = 0; f < O_COUNT; ++f) o[f] = lo[f][src];
+                for (int f = 0; f < O_COUNT; ++f) o[f] = L.lo[f][src];
 #pragma unroll
-            for (int j = 0; j < 7; ++j) luf[j][tid] = u[j];
+                for (int j = 0; j < 7; ++j) L.luf[j][tid] = u[j];
 #pragma unroll
-            for (int f = 0; f < O_COUNT; ++f) lo[f][tid] = o[f];
-            if constexpr (MODE != SW_PLAIN) lbmag[tid] = lbmag[src];
+                for (int f = 0; f < O_COUNT; ++f) L.lo[f][tid] = o[f];
+                if constexpr (MODE != SW_PLAIN) L.lbmag[tid] = L.lbmag[src];
+            }
+            __syncthreads();  // rows 8..12 are read before the new rows overwrite them
+            bool cell_bad = false;
+            store_cell<R, TS, MODE, DM>(A, L, HALO + tid, qn, cell_bad);
+            finish(by, cell_bad);
         }
-        __syncthreads();  // rows 8..12 are read before the new rows overwrite them
-        bool cell_bad = false;
-        store_cell<R, DIR, MODE, DM>(A, luf, lo, lbmag, HALO + tid, qn, cell_bad);
-        finish_cells(cell_bad, by, t0, blk);
-        __syncthreads();  // the tile's cells are in LDS
-        sweep_interfaces<R, DIR, MODE, EX, DM>(A, luf, lo, lbmag, t0, x0, y0, z0, blk);
     }
 }
 
@@ -776,33 +779,49 @@ struct CtFlags {
 // the 3-cell stencil halo that it shares with its neighbours (1.5x the row's
 // bytes).  Here workgroups L and L + 8 (the same XCD, dispatched one after
 // the other) take neighbouring x-tiles of one row; rows beyond the last full
-// group of 8 keep the launch order.  A bijection on the grid.
-__device__ __forceinline__ void xcd_row_tiles(int& bx, int& by, int& bz) {
-    const unsigned gx = gridDim.x, gy = gridDim.y, nrow = gy * gridDim.z;
-    const unsigned L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    bx = (int)blockIdx.x; by = (int)blockIdx.y; bz = (int)blockIdx.z;
-    if (gx == 1 || L >= (nrow / 8) * 8 * gx) return;
-    const unsigned a = L / 8, row = (a / gx) * 8 + L % 8;
-    bx = (int)(a % gx); by = (int)(row % gy); bz = (int)(row / gy);
+// group of 8 keep the launch order.  A bijection on the gx x gy x gz tiles.
+template <typename R>
+__device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X, int& bx, int& by, int& bz) {
+    const unsigned gx = X.gx, nrow = X.gy * X.gz;
+    unsigned row;
+    if (gx == 1 || L >= (nrow / 8) * 8 * gx) {
+        row = div(L, X.by_gx);
+        bx = (int)(L - row * gx);
+    } else {
+        const unsigned a = L / 8, r = div(a, X.by_gx);
+        row = r * 8 + L % 8;
+        bx = (int)(a - r * gx);
+    }
+    bz = (int)div(row, X.by_gy);
+    by = (int)(row - bz * X.gy);
 }
 
-// The sweep along DIR.  Reference rounding, DM = DIV_IEEE: the recompute
-// launch (a few blocks) takes the tiles queued by the sweep proper
+// The sweeps of one launch: the blocks of the y axis, of the z axis (marching
+// blocks, the longest, first) and of the x axis (single tiles, which fill the
+// chip while the last marches end).  Reference rounding, DM = DIV_IEEE: the
+// recompute launch (a few blocks) takes the tiles queued by the sweep proper
 // (A.fixlist, A.fixctl[0] of them), clears their flags, and the last block
 // to finish empties the queue; with an empty queue every block exits at once.
-template <typename R, int DIR, int MODE, int EX, int DM>
+template <typename R, int MODE, int EX, int DM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, MODE>()))) void k_sweep(
     SweepArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
     static_assert(EX || DM == DIV_IEEE, "the FMA forms divide with IEEE divisions");
+    __shared__ alignas(16) unsigned char raw[tile_lds_bytes<R, MODE, ACROSS_X>()];
+    static_assert(tile_lds_bytes<R, MODE, ALONG_X>() <= tile_lds_bytes<R, MODE, ACROSS_X>(), "LDS of both shapes");
     if constexpr (EX && DM == DIV_IEEE) {
         const unsigned n = A.fixctl[0];
-        const dim3 gr = sweep_grid(A.g, DIR);
         for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
-            const unsigned b = A.fixlist[i];
+            const unsigned slot = A.fixlist[i];
             __syncthreads();  // the previous tile's LDS is free
-            sweep_tile<R, DIR, MODE, EX, DM>(A, (int)(b % gr.x), (int)((b / gr.x) % gr.y), (int)(b / (gr.x * gr.y)), b);
-            if (threadIdx.x == 0) A.fix[b] = 0u;
+            // slots are ordered x, y, z; an axis without tiles holds none
+            const int k = slot < A.ax[0].tile0 ? 2 : slot < A.ax[1].tile0 ? 0 : 1;
+            const SweepAxis<R>& X = A.ax[k];
+            const unsigned b = slot - (unsigned)X.tile0;
+            const int bx = (int)(b % X.gx), by = (int)((b / X.gx) % X.gy), bz = (int)(b / (X.gx * X.gy));
+            if (k == 2) sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, X, raw, bx, by, bz, 1);
+            else sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by, bz, 1);
+            if (threadIdx.x == 0) A.fix[slot] = 0u;
         }
         __syncthreads();  // every thread of the block has read the count
         if (threadIdx.x == 0 && atomicAdd(&A.fixctl[1], 1u) == gridDim.x - 1) {
@@ -810,13 +829,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             A.fixctl[1] = 0u;
         }
     } else {
-        int bx = (int)blockIdx.x, by = (int)blockIdx.y, bz = (int)blockIdx.z;
-        if constexpr (DIR != 0 && sweep_marches<R, MODE>()) {
-            sweep_march<R, DIR, MODE, EX, DM>(A, bx, by * A.march, bz, A.march);
+        const unsigned b = blockIdx.x;
+        if (b >= A.ax[2].first) {
+            int bx, by, bz;
+            xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by, bz);
+            sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, A.ax[2], raw, bx, by, bz, 1);
         } else {
-            if constexpr (DIR == 0) xcd_row_tiles(bx, by, bz);
-            const long long blk = bx + (long long)gridDim.x * (by + (long long)gridDim.y * bz);
-            sweep_tile<R, DIR, MODE, EX, DM>(A, bx, by, bz, blk);
+            // The y and z sweeps are one code (strides) where it marches:
+            // 31 KB an axis in FP64.  The FP32 forms have it once per axis:
+            // their constants then come straight from the kernel arguments
+            // (routed y/z sweeps at 256^3 444/459 -> 429/445 us).
+            auto across = [&](const SweepAxis<R>& X) {
+                const unsigned L = b - X.first, r = div(L, X.by_gx), bz = div(r, X.by_gy);
+                const int bx = (int)(L - r * X.gx), by = (int)(r - bz * X.by_gy.d);
+                sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by * X.march, (int)bz, X.march);
+            };
+            if constexpr (sizeof(R) == 8) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
+            else if (b >= A.ax[1].first) across(A.ax[1]);
+            else across(A.ax[0]);
         }
     }
 }

@@ -34,13 +34,6 @@ inline RK rk_coeff(int iw) {
     return c;
 }
 
-template <typename R, int MODE, int DM>
-void launch_sweep_dm(howmhd_gpu_ctx* c, int d, const SweepArgs<R>& a, dim3 grid) {
-    if (d == 0) hipLaunchKernelGGL((k_sweep<R, 0, MODE, EX, DM>), grid, dim3(256), 0, c->stream, a);
-    else if (d == 1) hipLaunchKernelGGL((k_sweep<R, 1, MODE, EX, DM>), grid, dim3(256), 0, c->stream, a);
-    else hipLaunchKernelGGL((k_sweep<R, 2, MODE, EX, DM>), grid, dim3(256), 0, c->stream, a);
-}
-
 // Blocks of the IEEE-division recompute launch of the reference-rounding form.
 constexpr unsigned kRecomputeBlocks = 64;
 
@@ -77,47 +70,75 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
     return (int)std::min<unsigned long long>(cz, (unsigned long long)most);
 }
 
-// The sweep along d.  Reference rounding: the sweep with unscaled WENO
-// divisions, then the IEEE-division launch for the tiles it queued (it exits
-// at once when there are none; no counting there).
+// Arguments of stage iw's sweeps of the axes in `mask` (bit d: axis d) from qsrc;
+// *blocks receives the blocks of the launch.
 template <typename R, int MODE>
-void launch_sweep(howmhd_gpu_ctx* c, int d, const SweepArgs<R>& a0) {
-    SweepArgs<R> a = a0;
-    dim3 grid = sweep_grid(c->g, d);
-    a.march = 1;
-    if (d != 0 && sweep_marches<R, MODE>()) {
-        a.march = c->march_force > 0 ? (int)std::min<unsigned>(c->march_force, grid.y) : march_steps(grid);
-        grid.y = (grid.y + a.march - 1) / a.march;
-    }
-    if constexpr (EX) {
-        launch_sweep_dm<R, MODE, DIV_UNSCALED>(c, d, a, grid);
-        SweepArgs<R> b = a;
-        b.stats = nullptr;
-        launch_sweep_dm<R, MODE, DIV_IEEE>(c, d, b, dim3(kRecomputeBlocks));
-    } else {
-        launch_sweep_dm<R, MODE, DIV_IEEE>(c, d, a, grid);
-    }
-}
-
-template <typename R>
-SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int d, const double* qsrc) {
+SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned mask, unsigned* blocks) {
     SweepArgs<R> a{};
     a.q = qsrc;
-    a.dF = (R*)c->dF[d];
-    // x: fsy, fsz; y: gsz, gsx; z: hsx, hsy
-    a.ct_a = (R*)c->ct[2 * d];
-    a.ct_b = (R*)c->ct[2 * d + 1];
-    if (d == 1) { a.ct_a = (R*)c->ct[3]; a.ct_b = (R*)c->ct[2]; }
     a.g = c->g;
     a.ph = c->ph;
     a.gc = c->gc;
     a.ct_active = c->ctf.active;
     a.mlp = c->mlp;
-    a.stats = c->route_now ? c->iwave : nullptr;
+    a.stats = c->route_now ? c->iwave + (size_t)(iw - 1) * c->nwave : nullptr;
     a.fix = c->fixflag;
     a.fixlist = c->fixlist;
     a.fixctl = c->fixctl;
+    const long long nx = c->g.n[0], ny = c->g.n[1], nz = c->g.n[2];
+    const int order[3] = {1, 2, 0};
+    unsigned nb = 0;
+    for (int k = 0; k < 3; ++k) {
+        const int d = order[k];
+        SweepAxis<R>& x = a.ax[k];
+        x.dF = (R*)c->dF[d];
+        // x: fsy, fsz; y: gsz, gsx; z: hsx, hsy
+        x.ct_a = (R*)c->ct[d == 1 ? 3 : 2 * d];
+        x.ct_b = (R*)c->ct[d == 1 ? 2 : 2 * d + 1];
+        for (int m = 0; m < 8; ++m) x.qoff[m] = (long long)sweep_perm(d, m) * c->g.ncell;
+        x.n = c->g.n[d];
+        x.per = c->g.per[d];
+        const long long nif = x.n + 1 - (x.per ? 1 : 0);  // computed interfaces per line
+        x.nother = (int)(d == 2 ? ny : nz);
+        x.sA = (unsigned)(d == 0 ? 1 : d == 1 ? nx : nx * ny);
+        x.sB = (unsigned)(d == 2 ? nx : nx * ny);
+        x.cF = (long long)c->ncell / x.n * (x.n + 1);
+        x.tF = x.sA;
+        x.oF = (unsigned)(d == 2 ? nx : nx * (ny + 1));
+        x.sS = x.sA;
+        x.oS = (unsigned)(d == 0 ? nif : d == 1 ? nx * nif : nx);
+        const dim3 gr = sweep_grid(c->g, d);
+        x.gx = gr.x; x.gy = gr.y; x.gz = gr.z;
+        x.first = nb;
+        x.march = 1;
+        x.tile0 = c->tile0[d];
+        if (d != 0 && sweep_marches<R, MODE>())
+            x.march = c->march_force > 0 ? (int)std::min<unsigned>(c->march_force, gr.y) : march_steps(gr);
+        x.by_gx = launch_div(gr.x);
+        x.by_gy = launch_div((gr.y + x.march - 1) / x.march);
+        if (mask & (1u << d)) nb += gr.x * x.by_gy.d * gr.z;
+    }
+    *blocks = nb;
     return a;
+}
+
+// The sweeps of the axes in `mask`, one launch.  Reference rounding: the
+// sweeps with unscaled WENO divisions, then the IEEE-division launch for the
+// tiles they queued (it exits at once when there are none; no counting there).
+// One launch instead of one per axis: the last round of one axis's blocks,
+// the tail of its marches and its empty recompute launch cost 2% of the
+// sweeps at 256^3, and on a grid that leaves the chip idle the axes run side
+// by side.
+template <typename R, int MODE>
+void launch_sweep(howmhd_gpu_ctx* c, SweepArgs<R>& a, unsigned blocks) {
+    if (blocks == 0) return;
+    if constexpr (EX) {
+        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED>), dim3(blocks), dim3(256), 0, c->stream, a);
+        a.stats = nullptr;
+        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(kRecomputeBlocks), dim3(256), 0, c->stream, a);
+    } else {
+        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(blocks), dim3(256), 0, c->stream, a);
+    }
 }
 
 inline StageCoef stage_coef(const howmhd_gpu_ctx* c, int iw, double dt) {
@@ -157,14 +178,32 @@ CombineArgs<R> combine_args(howmhd_gpu_ctx* c, int iw, double dt) {
     return ca;
 }
 
+// The sweeps of a stage: one launch, or one per axis while the kernels are
+// being timed.
 template <typename R>
-int launch_sweeps(howmhd_gpu_ctx* c, const double* qsrc) {
+int launch_sweeps(howmhd_gpu_ctx* c, int iw, const double* qsrc) {
+    unsigned all = 0;
+    for (int d = 0; d < 3; ++d)
+        if (c->g.n[d] > 1) all |= 1u << d;
+    auto go = [&](unsigned mask) {
+        unsigned nb = 0;
+        if (c->route_now) {
+            SweepArgs<R> a = sweep_args<R, SW_ROUTED>(c, iw, qsrc, mask, &nb);
+            launch_sweep<R, SW_ROUTED>(c, a, nb);
+        } else {
+            SweepArgs<R> a = sweep_args<R, SW_PLAIN>(c, iw, qsrc, mask, &nb);
+            launch_sweep<R, SW_PLAIN>(c, a, nb);
+        }
+    };
+    if (!c->timing) {
+        go(all);
+        HCHECK(c, hipGetLastError());
+        return HOWMHD_OK;
+    }
     for (int d = 0; d < 3; ++d) {
-        if (c->g.n[d] <= 1) continue;
-        const SweepArgs<R> a = sweep_args<R>(c, d, qsrc);
+        if (!(all & (1u << d))) continue;
         TimedLaunch tl(c, HOWMHD_K_SWEEP_X + d);
-        if (c->route_now) launch_sweep<R, SW_ROUTED>(c, d, a);
-        else launch_sweep<R, SW_PLAIN>(c, d, a);
+        go(1u << d);
         HCHECK(c, hipGetLastError());
     }
     return HOWMHD_OK;
@@ -178,7 +217,7 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
     const double* bp = c->fbuf[c->qid[iw - 1]];
     double* bo = c->fbuf[c->qid[iw]];
 
-    int rc = launch_sweeps<R>(c, qp);
+    int rc = launch_sweeps<R>(c, iw, qp);
     if (rc) return rc;
 
     const unsigned nb = blocks_for(c->ncell, 256);

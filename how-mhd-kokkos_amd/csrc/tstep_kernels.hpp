@@ -83,18 +83,25 @@ __global__ void k_zero_u64(unsigned long long* p, int n) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
 }
 
-// Adds the per-wavefront counters of the routed sweeps (n slots of
-// (flagged, total, wavefronts flagged, wavefronts total)) to the four totals
-// and to (flagged, total) of the step in last[0..1] (cleared before the
-// launch), and clears the slots.  Grid-stride loop over the slots; one atomic
-// per total and block.
-__global__ __launch_bounds__(256) void k_fold_wave_stats(uint4* w, long long n, unsigned long long* tot,
+// Adds the wavefront words of a step's routed sweeps (flagged | valid << 8;
+// n tiles of four, over the five stages) to the four totals (flagged, total,
+// wavefronts flagged, wavefronts total) and to (flagged, total) of the step in
+// last[0..1] (cleared before the launch).  Grid-stride loop; one atomic per
+// total and block.
+__global__ __launch_bounds__(256) void k_fold_wave_stats(const uint4* w, long long n, unsigned long long* tot,
                                                          unsigned long long* last) {
     unsigned long long s0 = 0, s1 = 0, s2 = 0, s3 = 0;
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
         const uint4 v = w[i];
-        s0 += v.x; s1 += v.y; s2 += v.z; s3 += v.w;
-        w[i] = make_uint4(0u, 0u, 0u, 0u);
+        const unsigned k[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const unsigned flagged = k[j] & 0xffu;
+            s0 += flagged;
+            s1 += k[j] >> 8;
+            s2 += flagged ? 1u : 0u;
+            s3 += k[j] ? 1u : 0u;
+        }
     }
     for (int o = 32; o > 0; o >>= 1) {
         s0 += __shfl_down(s0, o, 64);

@@ -39,3 +39,30 @@ def _step_matches(problem, n, bc, steps=1):
                                   ((130, 61, 64), "periodic"), ((9, 8, 400), "open")])
 def test_planes_per_block(n, bc, require_gpu):
     _step_matches("mpi_smooth3d", n, bc)
+
+
+# the axes' blocks in one launch: an axis of one cell in each place, ragged
+# tiles on every axis, more rows than a group of 8 in x, marches (the sweeps of
+# the last grid march through 2 tiles)
+@pytest.mark.parametrize("n,bc", [((67, 1, 35), "open"), ((70, 41, 1), "periodic"), ((200, 1, 1), "open"),
+                                  ((65, 35, 9), "open"), ((97, 120, 130), "periodic")])
+def test_axes_in_one_launch(n, bc, require_gpu):
+    _step_matches("mpi_smooth3d", n, bc)
+
+
+def test_timed_launches_change_no_bit(require_gpu):
+    """Timing launches the axes one by one and reports each."""
+    run = H.parse(H.make_input(problem="mhd_blast3d", nx=40, ny=33, nz=20, nt=1, tend=1.0))
+    p, q0 = H.gpu_params(run), H.init_problem(run)
+    out = []
+    for timed in (False, True):
+        with H.GpuSolver(p) as g:
+            g.upload_q0(q0)
+            g.init_faces()
+            g.set_timing(timed)
+            for _ in range(2):
+                g.ssprk(g.tstep())
+            if timed:
+                assert [g.timing()[k][1] for k in ("sweep_x", "sweep_y", "sweep_z")] == [10, 10, 10]
+            out.append(g.q0())
+    assert np.array_equal(out[0].view(np.int64), out[1].view(np.int64))
