@@ -836,15 +836,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, A.ax[2], raw, bx, by, bz, 1);
         } else {
             // The y and z sweeps are one code (strides) where it marches:
-            // 31 KB an axis in FP64.  The FP32 forms have it once per axis:
-            // their constants then come straight from the kernel arguments
-            // (routed y/z sweeps at 256^3 444/459 -> 429/445 us).
+            // 31 KB an axis in FP64.  The single-tile forms have it once per
+            // axis: their constants then come straight from the kernel
+            // arguments (routed FP32 y/z sweeps at 256^3 444/459 -> 429/445 us).
             auto across = [&](const SweepAxis<R>& X) {
                 const unsigned L = b - X.first, r = div(L, X.by_gx), bz = div(r, X.by_gy);
                 const int bx = (int)(L - r * X.gx), by = (int)(r - bz * X.by_gy.d);
                 sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by * X.march, (int)bz, X.march);
             };
-            if constexpr (sizeof(R) == 8) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
+            if constexpr (sweep_marches<R, MODE>()) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
             else if (b >= A.ax[1].first) across(A.ax[1]);
             else across(A.ax[0]);
         }
