@@ -63,14 +63,25 @@ __device__ __forceinline__ R div_by(R a, R b, R y) {
 // exponent(b) < 768; the arithmetic is then div_recip (the refined
 // reciprocal, a function of b alone) and div_with.  So quotients that share a
 // denominator share its refinement and stay bit-for-bit the IEEE quotient.
+// The refinement here is one third-order step, r0 (1 + e + e^2) with
+// e = 1 - b r0 of 2^-24, instead of two Newton steps: three FMAs instead of
+// four, and the same 1/b but for cases within 2^-72 of a rounding boundary
+// (3.4e9 random and edge-case operands for each use: 1/t, 3/t, 6/t, alpha/S
+// and recip_rn, no difference from the IEEE quotient).
 __device__ __forceinline__ double div_recip(double b) {
     const double r0 = __builtin_amdgcn_rcp(b);
-    const double r1 = __builtin_fma(r0, __builtin_fma(-b, r0, 1.0), r0);
-    return __builtin_fma(r1, __builtin_fma(-b, r1, 1.0), r1);
+    const double e = __builtin_fma(-b, r0, 1.0);
+    return __builtin_fma(r0, __builtin_fma(e, e, e), r0);
 }
 __device__ __forceinline__ double div_with(double a, double b, double r) {
     const double q = a * r;
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+}
+// RN(1/b) for b in [2^-900, 2^900] (the division of 1 by b in these parts):
+// six instructions instead of the IEEE division's eleven.
+__device__ __forceinline__ double recip_rn(double b) {
+    const double r = div_recip(b);
+    return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
 }
 
 
@@ -93,7 +104,8 @@ __device__ __forceinline__ float rcp_fast<float>(float x) { return __builtin_amd
 
 // Division form of the reference-rounding WENO weights: IEEE divisions, or
 // div_recip/div_with, which hold for t_k = (eps + IS_k)^2 <= 1e200 (then
-// alpha_k in [1e-200, 6e20] and omega in (5e-222, 1]).  The unscaled form
+// alpha_k in [1e-200, 6e20] and omega in (5e-222, 1]; on doubled arguments,
+// weno_side, t_k is 16 times the reference's).  The unscaled form
 // collects in `bad` (a wavefront mask, kept in scalar registers) the lanes
 // where the high word of a t_k bit pattern reaches kUnscaledHi, the high word
 // of 1e200 (every double with a smaller high word is below 1e200; t_k > 0,
@@ -131,7 +143,9 @@ __device__ __forceinline__ R div_q(R a, R b, R y) {
 // other operand >= 2^-767, and for NaN, the scaling is the identity, so these
 // steps give its bits; an operand in (0, 2^-767) or negative raises `bad`,
 // and the caller recomputes the tile with sqrt().
-__device__ __forceinline__ double sqrt_unscaled(double x, bool& bad) {
+// sqrt_core is the refinement alone, for operands the caller knows to lie in
+// [2^-767, inf).
+__device__ __forceinline__ double sqrt_core(double x) {
     const double r = __builtin_amdgcn_rsq(x);
     double g = x * r;
     double h = r * 0.5;
@@ -141,7 +155,10 @@ __device__ __forceinline__ double sqrt_unscaled(double x, bool& bad) {
     h = __builtin_fma(h, e, h);
     g = __builtin_fma(d0, h, g);
     const double d1 = __builtin_fma(-g, g, x);
-    g = __builtin_fma(d1, h, g);
+    return __builtin_fma(d1, h, g);
+}
+__device__ __forceinline__ double sqrt_unscaled(double x, bool& bad) {
+    const double g = sqrt_core(x);
     const bool special = __builtin_amdgcn_class(x, 0x260);  // -0, +0, +inf
     bad = bad || (x < 0x1p-767 && !special);
     return special ? x : g;
@@ -157,19 +174,19 @@ __device__ __forceinline__ double sqrt_q(double x, bool& bad) {
 }
 
 // x / c for a compile-time constant c > 0 with inv_c = RN(1/c).  Reference
-// rounding: the correctly rounded quotient of div_by without its select:
-// with nr = fma(c, q, -x) = -r exactly, fma(-nr, inv_c, q) equals div_by's
-// (r == 0) ? q : fma(r, inv_c, q) bit for bit when inv_c > 0, signed zeros
-// included (checked on 4e8 pairs for the divisors used, zeros, subnormals and
-// exact multiples among them).  Like div_by it is exact barring underflow
-// (subnormal x).  FMA form: multiplication by the rounded reciprocal (differs
-// by at most one rounding).
+// rounding: with lo = RN(1/c - inv_c), RN(x inv_c + RN(x lo)) is the
+// quotient.  The divisors are 3, 6, 12, 24 and 18, so x/c is a multiple of a
+// third or a ninth of an ulp and lies at least 1/18 ulp from a rounding
+// boundary, while the sum before rounding is within 2^-52 ulp of x/c; the
+// bound holds while RN(x lo) is accurate, for |x| >= 2^-1016, and x = +-0
+// keeps its sign (lo > 0).  For a power of two the product is exact.  Two
+// instructions; q = x inv_c and its FMA remainder are three.  FMA form:
+// multiplication by the rounded reciprocal (differs by at most one rounding).
 template <typename R>
 __device__ __forceinline__ R div_c(R x, R c, R inv_c) {
 #if HOWMHD_EXACT
-    const R q = x * inv_c;
-    const R nr = __builtin_fma(c, q, -x);
-    return __builtin_fma(-nr, inv_c, q);
+    const R lo = __builtin_fma(-c, inv_c, R(1)) / c;  // folded: a constant
+    return lo == R(0) ? x * inv_c : __builtin_fma(x, inv_c, x * lo);
 #else
     (void)c;
     return x * inv_c;
@@ -205,8 +222,13 @@ __device__ __forceinline__ void cell_values(const double* qs, double gam, double
     double rho = DD;
 #if HOWMHD_EXACT
     // correctly rounded quotients from shared reciprocals (div_by)
-    const double iDD = 1.0 / DD;
-    if constexpr (DM == DIV_UNSCALED) *bad = *bad || !(iDD > 0.0);  // rho >= DD > 0 then
+    double iDD;
+    if constexpr (DM == DIV_UNSCALED) {
+        *bad = *bad || !(DD > 0x1p-900 && DD < 0x1p900);  // else recip_rn holds, and rho >= DD > 0
+        iDD = recip_rn(DD);
+    } else {
+        iDD = 1.0 / DD;
+    }
     const double vx = div_q<DM>(Mx, DD, iDD);
     const double vy = div_q<DM>(My, DD, iDD);
     const double vz = div_q<DM>(Mz, DD, iDD);
@@ -383,15 +405,35 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
     const R vv2 = vx * vx + vy * vy + vz * vz;
     const R BB2 = Bx * Bx + By * By + Bz * Bz;
 #if HOWMHD_EXACT
-    const R bbn2 = BB2 / rho;
-    const R bnx2 = Bx * Bx / rho;
+    R bbn2, bnx2;
+    if constexpr (DM == DIV_UNSCALED) {
+        const R ir = recip_rn(rho);
+        bbn2 = div_pos<R>(BB2, rho, ir);
+        bnx2 = div_pos<R>(Bx * Bx, rho, ir);
+    } else {
+        bbn2 = BB2 / rho;
+        bnx2 = Bx * Bx / rho;
+    }
 #else
     const R irho = rcp_fast(rho);
     const R bbn2 = BB2 * irho;
     const R bnx2 = Bx * Bx * irho;
 #endif
     const R cs2 = (gam - R(1)) * (HH - R(0.5) * (vv2 + bbn2));
+#if HOWMHD_EXACT
+    // rho, c_s^2 and the sum in these ranges put every operand of recip_rn,
+    // of sqrt_core and of the divisions by sqrt(c_f^2 - c_slow^2) below in its
+    // range (NaN fails, too)
+    if constexpr (DM == DIV_UNSCALED)
+        sb = !(rho > R(0x1p-760) && rho < R(0x1p900) && cs2 > R(0x1p-760) && bbn2 + cs2 < R(0x1p500));
+    auto sqp = [&](R x) -> R {  // a positive operand in range
+        if constexpr (DM == DIV_UNSCALED) return sqrt_core(x);
+        else return sqrt(x);
+    };
+    const R cs = sqp(DM == DIV_UNSCALED ? cs2 : rmax(R(0), cs2));
+#else
     const R cs = sq(rmax(R(0), cs2));
+#endif
     const R Bt2 = By * By + Bz * Bz;
 #if !HOWMHD_EXACT
     if constexpr (sizeof(R) == 4) {
@@ -399,20 +441,31 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
     } else
 #endif
     {
-    // unscaled square roots (sq) only where the operand stays far above
+    // unscaled square roots (sq, sqp) only where the operand stays far above
     // 2^-767 in MHD flows: c_s^2, root^2, c_f^2, c_f^2 - c_slow^2 (>= 1e-30
     // here), B_t^2 (>= 1e-30) and rho.  c_a^2 and c_slow^2 scale with B_n^2,
     // and the alpha numerators vanish where B_t does: IEEE square roots.
     const R root = sq(rmax(R(0), (bbn2 + cs2) * (bbn2 + cs2) - R(4) * bnx2 * cs2));
+#if HOWMHD_EXACT
+    const R lf = sqp(DM == DIV_UNSCALED ? R(0.5) * (bbn2 + cs2 + root) : rmax(R(0), R(0.5) * (bbn2 + cs2 + root)));
+#else
     const R lf = sq(rmax(R(0), R(0.5) * (bbn2 + cs2 + root)));
+#endif
     const R ls = rsqrt_(rmax(R(0), R(0.5) * (bbn2 + cs2 - root)));
     e.lf = lf; e.ls = ls;
     R af, as;
     if ((lf * lf - ls * ls) >= R(1.0e-30)) {
 #if HOWMHD_EXACT
-        const R sd = sq(lf * lf - ls * ls);
-        af = rsqrt_(rmax(R(0), cs2 - ls * ls)) / sd;
-        as = rsqrt_(rmax(R(0), lf * lf - cs2)) / sd;
+        const R sd = sqp(lf * lf - ls * ls);
+        const R an = rsqrt_(rmax(R(0), cs2 - ls * ls)), sn = rsqrt_(rmax(R(0), lf * lf - cs2));
+        if constexpr (DM == DIV_UNSCALED) {
+            const R isd = recip_rn(sd);
+            af = div_pos<R>(an, sd, isd);
+            as = div_pos<R>(sn, sd, isd);
+        } else {
+            af = an / sd;
+            as = sn / sd;
+        }
 #else
         const R rd = rcp_fast(rsqrt_(lf * lf - ls * ls));
         af = rsqrt_(rmax(R(0), cs2 - ls * ls)) * rd;
@@ -427,7 +480,7 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
     R bty, btz;
     if (Bt2 >= R(1.0e-30)) {
 #if HOWMHD_EXACT
-        const R sbt = sq(Bt2);
+        const R sbt = sqp(Bt2);
         bty = By / sbt;
         btz = Bz / sbt;
 #else
@@ -439,13 +492,18 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
         bty = R(1) / rsqrt_(R(2));
         btz = R(1) / rsqrt_(R(2));
     }
+#if HOWMHD_EXACT
+    const R sqrtrho = sqp(rho);
+#else
     const R sqrtrho = sq(rho);
+#endif
     e.vx = vx; e.vy = vy; e.vz = vz; e.By = By; e.Bz = Bz; e.vv2 = vv2;
     e.cs = cs; e.cs2 = cs2;
     e.bty = bty; e.btz = btz; e.sgnBx = sign1(Bx);
     e.sqrtrho = sqrtrho;
 #if HOWMHD_EXACT
-    e.invsqrtrho = R(1) / sqrtrho;
+    if constexpr (DM == DIV_UNSCALED) e.invsqrtrho = recip_rn(sqrtrho);
+    else e.invsqrtrho = R(1) / sqrtrho;
 #else
     e.invsqrtrho = rcp_fast(sqrtrho);
 #endif
@@ -454,7 +512,9 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
     e.nrm_half = R(0.5) * ics2;
     e.nrm_ent = (gam - R(1)) * ics2;
 #else
-    e.nrm_half = R(1) / cs2;   // RN(1/cs2): the L-row normalisation divides by cs2 through div_by
+    // RN(1/cs2): the L-row normalisation divides by cs2 through it
+    if constexpr (DM == DIV_UNSCALED) e.nrm_half = recip_rn(cs2);
+    else e.nrm_half = R(1) / cs2;
     e.nrm_ent = R(0);
     if (sqbad) *sqbad = *sqbad || sb;
 #endif
@@ -541,6 +601,9 @@ __device__ __forceinline__ void l_row(R gam, const Eig<R>& e, R* L, const GasCon
 #if HOWMHD_EXACT
         if constexpr (M == 1 || M == 5) L[c] = R(0.5) * L[c];
         else if constexpr (M == 3) L[c] = div_q<DM>(-gam0 * L[c], cs2, e.nrm_half);
+        // (0.5 L) / cs2 = L / (2 cs2) with RN(1/(2 cs2)) = RN(1/cs2) / 2: the
+        // same quotient without the product
+        else if constexpr (DM == DIV_UNSCALED) L[c] = div_pos<R>(L[c], R(2) * cs2, R(0.5) * e.nrm_half);
         else L[c] = div_q<DM>(R(0.5) * L[c], cs2, e.nrm_half);
 #else
         if constexpr (M == 1 || M == 5) L[c] = R(0.5) * L[c];
@@ -629,9 +692,13 @@ __device__ __forceinline__ void r_col(R gam, const Eig<R>& e, R* Rc, const GasCo
 // phi_N(a,b,c,d) = w0 (a-2b+c)/3 + (w2-1/2)(b-2c+d)/6 with
 // IS0 = 13(a-b)^2 + 3(a-3b)^2, IS1 = 13(b-c)^2 + 3(b+c)^2,
 // IS2 = 13(c-d)^2 + 3(3c-d)^2, alpha = (1,6,3)/(eps+IS)^2, eps = 1e-10.
+// In the unscaled mode the arguments and the result are twice the reference's
+// (weno_wave): the indicators are four times theirs, eps too, and everything
+// below them scales by powers of two, so the weights have the same bits and
+// the result is exactly twice the reference's.
 template <typename R, int DM = DIV_IEEE>
 __device__ __forceinline__ R weno_side(R a, R b, R c, R d, unsigned long long& bad, R* w0_out = nullptr, R* w2_out = nullptr) {
-    const R eps = R(1.0e-10);
+    const R eps = DM == DIV_UNSCALED ? R(4) * R(1.0e-10) : R(1.0e-10);
     const R IS0 = R(13) * (a - b) * (a - b) + R(3) * (a - R(3) * b) * (a - R(3) * b);
     const R IS1 = R(13) * (b - c) * (b - c) + R(3) * (b + c) * (b + c);
     const R IS2 = R(13) * (c - d) * (c - d) + R(3) * (R(3) * c - d) * (R(3) * c - d);
@@ -701,6 +768,13 @@ __device__ __forceinline__ R weno_wave(const R* Fsk, const R* qsk, R amx, unsign
         dq[k] = qsk[k + 1] - qsk[k];
     }
     const R first = div_c<R>(-Fsk[1] + R(7) * Fsk[2] + R(7) * Fsk[3] - Fsk[4], R(12), R(1.0 / 12.0));
+    if constexpr (DM == DIV_UNSCALED) {
+        // the halves of the LLF splitting are taken from the sums: eight
+        // products less, and first - second and + third stay single roundings
+        const R s2 = weno_side<R, DM>(dF[0] + amx * dq[0], dF[1] + amx * dq[1], dF[2] + amx * dq[2], dF[3] + amx * dq[3], bad);
+        const R t2 = weno_side<R, DM>(dF[4] - amx * dq[4], dF[3] - amx * dq[3], dF[2] - amx * dq[2], dF[1] - amx * dq[1], bad);
+        return fma(R(0.5), t2, fma(R(-0.5), s2, first));
+    }
     const R second = weno_side<R, DM>(R(0.5) * (dF[0] + amx * dq[0]), R(0.5) * (dF[1] + amx * dq[1]),
                                       R(0.5) * (dF[2] + amx * dq[2]), R(0.5) * (dF[3] + amx * dq[3]), bad);
     const R third = weno_side<R, DM>(R(0.5) * (dF[4] - amx * dq[4]), R(0.5) * (dF[3] - amx * dq[3]),
@@ -720,13 +794,15 @@ __device__ __forceinline__ R weno_wave_dev(const R* Fsk, const R* qsk, R amx, R&
         dq[k] = qsk[k + 1] - qsk[k];
     }
     const R first = div_c<R>(-Fsk[1] + R(7) * Fsk[2] + R(7) * Fsk[3] - Fsk[4], R(12), R(1.0 / 12.0));
+    constexpr R h = DM == DIV_UNSCALED ? R(1) : R(0.5);  // see weno_wave
     R w0, w2;
-    const R second = weno_side<R, DM>(R(0.5) * (dF[0] + amx * dq[0]), R(0.5) * (dF[1] + amx * dq[1]),
-                                      R(0.5) * (dF[2] + amx * dq[2]), R(0.5) * (dF[3] + amx * dq[3]), bad, &w0, &w2);
+    const R second = weno_side<R, DM>(h * (dF[0] + amx * dq[0]), h * (dF[1] + amx * dq[1]),
+                                      h * (dF[2] + amx * dq[2]), h * (dF[3] + amx * dq[3]), bad, &w0, &w2);
     dev = rmax(dev, rmax(rabs(w0 - R(0.1)), rmax(rabs(w2 - R(0.3)), rabs(R(1) - w0 - w2 - R(0.6)))));
-    const R third = weno_side<R, DM>(R(0.5) * (dF[4] - amx * dq[4]), R(0.5) * (dF[3] - amx * dq[3]),
-                                     R(0.5) * (dF[2] - amx * dq[2]), R(0.5) * (dF[1] - amx * dq[1]), bad, &w0, &w2);
+    const R third = weno_side<R, DM>(h * (dF[4] - amx * dq[4]), h * (dF[3] - amx * dq[3]),
+                                     h * (dF[2] - amx * dq[2]), h * (dF[1] - amx * dq[1]), bad, &w0, &w2);
     dev = rmax(dev, rmax(rabs(w0 - R(0.1)), rmax(rabs(w2 - R(0.3)), rabs(R(1) - w0 - w2 - R(0.6)))));
+    if constexpr (DM == DIV_UNSCALED) return fma(R(0.5), third, fma(R(-0.5), second, first));
     return first - second + third;
 }
 

@@ -1,0 +1,68 @@
+"""Rewrites of the reference-rounding sweep that change no bit, on the CPU.
+
+  * division by 3, 6, 12, 18 and 24 as RN(x h + RN(x l)), h = RN(1/c),
+    l = RN(1/c - h), in exact rational arithmetic against the correctly rounded
+    quotient: random operands, multiples of the divisor, all-ones
+    significands, operands next to the quotients' rounding boundaries, zeros;
+  * the WENO5 side on doubled arguments with four times eps: exactly twice the
+    side on the arguments themselves, weights bit for bit (NumPy doubles),
+    from 1e-140 to 1e45; a wrong eps fails.
+"""
+from fractions import Fraction
+
+import numpy as np
+import pytest
+
+
+def _rn(f):
+    return f.numerator / f.denominator  # int / int is correctly rounded
+
+
+def _two_step(x, c):
+    h = 1.0 / c
+    lo = _rn((1 - Fraction(c) * Fraction(h)) / c)
+    return lo, _rn(Fraction(x) * Fraction(h) + Fraction(x * lo))
+
+
+@pytest.mark.parametrize("c", [3, 6, 12, 18, 24])
+def test_division_by_constant(c):
+    rng = np.random.default_rng(c)
+    xs = list(rng.standard_normal(4000) * 10.0 ** rng.integers(-280, 280, 4000))
+    for _ in range(2000):
+        m = int(rng.integers(1 << 52, 1 << 53))
+        e = int(rng.integers(-200, 200))
+        xs += [float(m) * 2.0 ** e, float(m // c * c) * 2.0 ** e, float((1 << 53) - 1 - int(rng.integers(0, 9))) * 2.0 ** e]
+        # next to c times a midpoint of two doubles
+        xs += [_rn(Fraction(2 * m + 1, 2) * c + k) for k in (-1, 0, 1)]
+    for x in xs:
+        assert _two_step(x, c)[1] == _rn(Fraction(x) / c), x.hex()
+    lo, _ = _two_step(1.0, c)
+    assert lo > 0.0
+    h = 1.0 / c
+    for x in (0.0, -0.0):  # the sum of products keeps the sign of a zero
+        assert np.signbit(x * h + x * lo) == np.signbit(x / c)
+
+
+def _side(a, b, c, d, eps):
+    is0 = 13.0 * (a - b) * (a - b) + 3.0 * (a - 3.0 * b) * (a - 3.0 * b)
+    is1 = 13.0 * (b - c) * (b - c) + 3.0 * (b + c) * (b + c)
+    is2 = 13.0 * (c - d) * (c - d) + 3.0 * (3.0 * c - d) * (3.0 * c - d)
+    t = [(eps + s) * (eps + s) for s in (is0, is1, is2)]
+    al = [1.0 / t[0], 6.0 / t[1], 3.0 / t[2]]
+    s = al[0] + al[1] + al[2]
+    w0, w2 = al[0] / s, al[2] / s
+    return w0, w2, w0 * (a - 2.0 * b + c) / 3.0 + (w2 - 0.5) * (b - 2.0 * c + d) / 6.0
+
+
+def test_doubled_weno_side():
+    rng = np.random.default_rng(1)
+    n = 200000
+    v = rng.standard_normal((4, n)) * 10.0 ** rng.uniform(-140, 45, n)
+    v[:, ::3] = v[0, ::3] * (1.0 + 1e-6 * rng.standard_normal((4, v[:, ::3].shape[1])))  # smooth
+    v[rng.integers(0, 4, n // 7), np.arange(n // 7)] = 0.0
+    v[:, -1] = 0.0
+    w0, w2, phi = _side(*v, 1.0e-10)
+    x0, x2, twice = _side(*(2.0 * v), 4.0 * 1.0e-10)
+    for a, b in ((w0, x0), (w2, x2), (2.0 * phi, twice)):
+        assert np.array_equal(a.view(np.int64), b.view(np.int64))
+    assert not np.array_equal(_side(*(2.0 * v), 1.0e-10)[2], twice)
