@@ -38,7 +38,15 @@ struct howmhd_gpu_ctx {
     void* ct[6] = {};          // fsy fsz gsx gsz hsx hsy
     void* O2[3] = {};
     void* O[3] = {};
-    unsigned long long* dmax = nullptr;
+    // one allocation for the device arrays below of a few values per block or
+    // tile, and smaller ones (howmhd_gpu_create); vmax_host and istats_host lie behind the transfer slots
+    void* arena = nullptr;
+    // per-step reductions: partials of their blocks, counters of the blocks
+    // done (zero between launches), and the CFL maxima in pinned host memory
+    double* cflfold = nullptr;
+    unsigned long long* statfold = nullptr;
+    unsigned* done = nullptr;
+    double* vmax_host = nullptr;
     // CFL maxima per block of the last stage-5 combination (3 per block of
     // k_combine); cfl_fresh: they belong to the current q(0)
     double* cflpart = nullptr;

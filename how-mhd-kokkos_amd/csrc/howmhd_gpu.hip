@@ -27,6 +27,8 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
+#include <vector>
 
 #if !HOWMHD_EXACT
 #error "howmhd_gpu.hip is built with HOWMHD_EXACT=1"
@@ -226,6 +228,14 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         }
         return true;
     };
+    // the arrays of a few values per block or tile, and smaller ones, share
+    // one allocation, 256-byte aligned
+    std::vector<std::pair<void**, size_t>> parts;
+    size_t arena = 0;
+    auto small = [&](void** ptr, size_t bytes) {
+        parts.push_back({ptr, arena});
+        arena += (bytes + 255) / 256 * 256;
+    };
     bool ok = true;
     for (int b = 0; b < 5 && ok; ++b) {
         ok = ok && alloc((void**)&c->qbuf[b], 8 * c->ncell * sizeof(double));
@@ -245,21 +255,28 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         if (!emf_fused) ok = ok && alloc(&c->O2[t], c->ncell * c->rsize);
         ok = ok && alloc(&c->O[t], c->ncell * c->rsize);
     }
-    ok = ok && alloc((void**)&c->dmax, 4 * sizeof(unsigned long long));
-    ok = ok && alloc((void**)&c->cflpart, 3 * (size_t)blocks_for(c->ncell, 256) * sizeof(double));
-    ok = ok && alloc((void**)&c->floorpart, 2 * (size_t)blocks_for(c->ncell, 256) * sizeof(unsigned));
-    ok = ok && alloc((void**)&c->diagpart, (size_t)DIAG_BLOCKS * DIAG_NV * sizeof(double));
-    ok = ok && alloc((void**)&c->diagout, DIAG_NV * sizeof(double));
+    small((void**)&c->cflfold, 3 * CFL_FOLD_BLOCKS * sizeof(double));
+    small((void**)&c->statfold, 4 * STAT_FOLD_BLOCKS * sizeof(unsigned long long));
+    small((void**)&c->done, 2 * sizeof(unsigned));
+    small((void**)&c->cflpart, 3 * (size_t)blocks_for(c->ncell, 256) * sizeof(double));
+    small((void**)&c->floorpart, 2 * (size_t)blocks_for(c->ncell, 256) * sizeof(unsigned));
+    small((void**)&c->diagpart, (size_t)DIAG_BLOCKS * DIAG_NV * sizeof(double));
+    small((void**)&c->diagout, DIAG_NV * sizeof(double));
     c->xfer_slot = xfer_slot(c->ncell, n[2]);
     c->xfer_n = xfer_slots(c->ncell, c->xfer_slot);
-    ok = ok && hipHostMalloc((void**)&c->xfer, c->xfer_n * c->xfer_slot * sizeof(double), hipHostMallocDefault) ==
-                   hipSuccess;
+    // pinned: the transfer slots, then what the per-step reductions tell
+    const size_t pinned = c->xfer_n * c->xfer_slot;
+    ok = ok && hipHostMalloc((void**)&c->xfer, (pinned + 8) * sizeof(double), hipHostMallocDefault) == hipSuccess;
+    if (ok) {
+        c->vmax_host = c->xfer + pinned;
+        c->istats_host = (unsigned long long*)(c->vmax_host + 4);
+    }
     for (int s = 0; s < c->xfer_n && ok; ++s) {
         hipEvent_t ev = nullptr;
         ok = hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
         if (ok) c->xfer_ev.push_back(ev);
     }
-    ok = ok && alloc((void**)&c->mlp, sizeof(MlpDev));
+    small((void**)&c->mlp, sizeof(MlpDev));
     // one slot per tile of the sweeps (x, y, z), four counter words each
     for (int d = 0; d < 3; ++d) {
         const dim3 gr = sweep_grid(c->g, d);
@@ -267,14 +284,15 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         if (n[d] > 1) c->nwave += 4LL * gr.x * gr.y * gr.z;
     }
     c->nwave = std::max(c->nwave, 4LL);
-    ok = ok && alloc((void**)&c->iwave, 5 * (size_t)c->nwave * sizeof(unsigned));
-    ok = ok && alloc((void**)&c->fixflag, (size_t)(c->nwave / 4) * sizeof(unsigned));
-    ok = ok && alloc((void**)&c->fixlist, (size_t)(c->nwave / 4) * sizeof(unsigned));
-    ok = ok && alloc((void**)&c->fixctl, 2 * sizeof(unsigned));
-    ok = ok && alloc((void**)&c->istats, 4 * sizeof(unsigned long long));
-    ok = ok && alloc((void**)&c->ilast, 2 * sizeof(unsigned long long));
-    ok = ok && hipHostMalloc((void**)&c->istats_host, 4 * sizeof(unsigned long long), hipHostMallocDefault) ==
-                   hipSuccess;
+    small((void**)&c->iwave, 5 * (size_t)c->nwave * sizeof(unsigned));
+    small((void**)&c->fixflag, (size_t)(c->nwave / 4) * sizeof(unsigned));
+    small((void**)&c->fixlist, (size_t)(c->nwave / 4) * sizeof(unsigned));
+    small((void**)&c->fixctl, 2 * sizeof(unsigned));
+    small((void**)&c->istats, 4 * sizeof(unsigned long long));
+    small((void**)&c->ilast, 2 * sizeof(unsigned long long));
+    ok = ok && alloc(&c->arena, arena);
+    for (auto& part : parts)
+        if (ok) *part.first = (char*)c->arena + part.second;
     ok = ok && hipEventCreateWithFlags(&c->istats_ev, hipEventDisableTiming) == hipSuccess;
     if (!ok) return cleanup_fail(HOWMHD_ENOMEM, "howmhd_gpu_create: device allocation failed");
     if (hipStreamSynchronize(c->stream) != hipSuccess)
@@ -297,21 +315,9 @@ int howmhd_gpu_destroy(howmhd_gpu_ctx* c) {
     }
     for (int t = 0; t < 6; ++t)
         if (c->ct[t]) (void)hipFree(c->ct[t]);
-    if (c->dmax) (void)hipFree(c->dmax);
-    if (c->cflpart) (void)hipFree(c->cflpart);
-    if (c->floorpart) (void)hipFree(c->floorpart);
-    if (c->diagpart) (void)hipFree(c->diagpart);
-    if (c->diagout) (void)hipFree(c->diagout);
+    if (c->arena) (void)hipFree(c->arena);
     if (c->xfer) (void)hipHostFree(c->xfer);
     for (hipEvent_t ev : c->xfer_ev) (void)hipEventDestroy(ev);
-    if (c->ilast) (void)hipFree(c->ilast);
-    if (c->mlp) (void)hipFree(c->mlp);
-    if (c->istats) (void)hipFree(c->istats);
-    if (c->iwave) (void)hipFree(c->iwave);
-    if (c->fixflag) (void)hipFree(c->fixflag);
-    if (c->fixlist) (void)hipFree(c->fixlist);
-    if (c->fixctl) (void)hipFree(c->fixctl);
-    if (c->istats_host) (void)hipHostFree(c->istats_host);
     if (c->istats_ev) (void)hipEventDestroy(c->istats_ev);
     drain_timing(c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -349,27 +355,24 @@ int howmhd_gpu_upload_faces(howmhd_gpu_ctx* c, const double* b) {
 
 int howmhd_gpu_tstep(howmhd_gpu_ctx* c, double* dt) {
     if (!c || !dt) return HOWMHD_EINVAL;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->dmax, 3);
-    HCHECK(c, hipGetLastError());
     {
         TimedLaunch tl(c, HOWMHD_K_CFL);
-        if (c->cfl_fresh) {
-            // maxima of the last step's stage-5 combination, which wrote q(0)
-            const long long nblk = blocks_for(c->ncell, 256);
-            const unsigned nb = std::min<unsigned>(blocks_for((size_t)nblk, 256), 256u);
-            hipLaunchKernelGGL(k_cfl_fold, dim3(nb), dim3(256), 0, c->stream, (const double*)c->cflpart, nblk, c->dmax);
-        } else {
-            const unsigned nb = std::min<unsigned>(blocks_for(c->ncell, 256), 2048u);
-            hipLaunchKernelGGL(k_cfl, dim3(nb), dim3(256), 0, c->stream, (const double*)c->qbuf[c->qid[0]], c->g,
-                               c->ph, c->dmax);
+        long long n = blocks_for(c->ncell, 256);
+        // without the maxima of the last step's stage-5 combination, which
+        // wrote q(0): those of q(0) itself
+        if (!c->cfl_fresh) {
+            n = std::min<long long>(n, 2048);
+            hipLaunchKernelGGL(k_cfl, dim3((unsigned)n), dim3(256), 0, c->stream, (const double*)c->qbuf[c->qid[0]],
+                               c->g, c->ph, c->cflpart);
+            HCHECK(c, hipGetLastError());
         }
+        const unsigned nb = std::min<unsigned>(blocks_for((size_t)n, 512), CFL_FOLD_BLOCKS);
+        hipLaunchKernelGGL(k_cfl_fold, dim3(nb), dim3(256), 0, c->stream, (const double*)c->cflpart, n, c->cflfold,
+                           c->done, c->vmax_host);
     }
     HCHECK(c, hipGetLastError());
-    unsigned long long h[3];
-    HCHECK(c, hipMemcpyAsync(h, c->dmax, sizeof(h), hipMemcpyDeviceToHost, c->stream));
     HCHECK(c, hipStreamSynchronize(c->stream));
-    double vmax[3];
-    for (int d = 0; d < 3; ++d) std::memcpy(&vmax[d], &h[d], sizeof(double));
+    const double vmax[3] = {c->vmax_host[0], c->vmax_host[1], c->vmax_host[2]};
     *dt = dt_from_vmax(c->p, vmax);
     return HOWMHD_OK;
 }
@@ -452,25 +455,19 @@ int howmhd_gpu_ssprk(howmhd_gpu_ctx* c, double dt) {
         if (rc) return rc;
     }
     if (c->route_now) {
-        // the step's per-wavefront counters into the totals and into the
-        // step's own (flagged, total) (slots cleared)
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->ilast, 2);
-        HCHECK(c, hipGetLastError());
+        // the step's per-wavefront counts into the totals and into the step's
+        // own (flagged, total); in mode 1 the totals go to the host
+        const bool tell = c->ind_mode == 1 && !c->istats_pending;
         const long long ntile = 5 * c->nwave / 4;
-        const unsigned nb = std::min(1024u, blocks_for((size_t)ntile, 256));
+        const unsigned nb = std::min(STAT_FOLD_BLOCKS, blocks_for((size_t)ntile, 256));
         hipLaunchKernelGGL(k_fold_wave_stats, dim3(nb), dim3(256), 0, c->stream, (const uint4*)c->iwave, ntile,
-                           c->istats, c->ilast);
+                           c->statfold, c->done + 1, c->istats, c->ilast, tell ? c->istats_host : nullptr);
         HCHECK(c, hipGetLastError());
         c->any_routed = true;
-    }
-    if (c->ind_mode == 1 && c->route_now && !c->istats_pending) {
-        // this step's totals to the host, then clear them for the next
-        HCHECK(c, hipMemcpyAsync(c->istats_host, c->istats, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                 c->stream));
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, c->istats, 4);
-        HCHECK(c, hipGetLastError());
-        HCHECK(c, hipEventRecord(c->istats_ev, c->stream));
-        c->istats_pending = true;
+        if (tell) {
+            HCHECK(c, hipEventRecord(c->istats_ev, c->stream));
+            c->istats_pending = true;
+        }
     }
     c->route_now = false;
     // q(0) <- q(5), faces likewise: exchange the buffers of stages 0 and 5

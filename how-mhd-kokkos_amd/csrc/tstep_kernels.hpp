@@ -8,11 +8,29 @@
 
 namespace howmhd {
 
+// ------------------------------------------------------- reductions per step
+// A reduction over many partials in one launch: every block leaves its own
+// result in part[blockIdx.x], and the last one to finish (`last_block`, true
+// in all its threads) combines them and writes the outcome, so that nothing
+// is cleared beforehand and no further launch or copy follows.  The counter
+// returns to zero.
+__device__ __forceinline__ bool last_block(unsigned* counter) {
+    __shared__ bool last;
+    __threadfence();  // this block's partial before its ticket
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        last = atomicAdd(counter, 1u) == gridDim.x - 1;
+        if (last) *counter = 0u;
+    }
+    __syncthreads();
+    if (last) __threadfence();  // every ticket before the partials are read
+    return last;
+}
+
 // ---------------------------------------------------------------- CFL (tstep)
 // Per-direction maximum of |v_d| + c_fast,d over active cells of q(0)
-// (src/tstep.cpp:28-83).  Non-negative doubles order like their bit patterns,
-// so the block maxima are combined with a 64-bit atomicMax.
-__global__ __launch_bounds__(256) void k_cfl(const double* q, Geom g, Phys ph, unsigned long long* out) {
+// (src/tstep.cpp:28-83), one triple per block.
+__global__ __launch_bounds__(256) void k_cfl(const double* q, Geom g, Phys ph, double* part) {
     double m0 = 0.0, m1 = 0.0, m2 = 0.0;
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < g.ncell; i += (long long)gridDim.x * 256) {
         double c[8];
@@ -20,27 +38,33 @@ __global__ __launch_bounds__(256) void k_cfl(const double* q, Geom g, Phys ph, u
         for (int m = 0; m < 8; ++m) c[m] = q[m * g.ncell + i];
         cfl_cell(c, ph, m0, m1, m2);
     }
-    __shared__ double bm[3];
-    block_max3(m0, m1, m2, bm);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) atomicMax(&out[d], (unsigned long long)__double_as_longlong(bm[d]));
+    block_max3(m0, m1, m2, part + 3 * (long long)blockIdx.x);
 }
 
-// The same maxima from the per-block maxima that the stage-5 combination
-// of the last step wrote (n blocks x 3).
-__global__ __launch_bounds__(256) void k_cfl_fold(const double* part, long long n, unsigned long long* out) {
-    double m0 = 0.0, m1 = 0.0, m2 = 0.0;
-    for (long long b = (long long)blockIdx.x * 256 + threadIdx.x; b < n; b += (long long)gridDim.x * 256) {
-        m0 = fmax(m0, part[3 * b]);
-        m1 = fmax(m1, part[3 * b + 1]);
-        m2 = fmax(m2, part[3 * b + 2]);
+// The maxima over n triples (of k_cfl, or of the last step's stage-5
+// combination) into out[0..2], pinned host memory that the host reads once the
+// stream is idle.  fold: a triple per block.  A clear, a fold by atomics and a
+// copy of the result to pageable memory were three launches: a step of
+// orszag_tang 128^2 211 -> 183 us, of cpaw3d 32^3 257 -> 229, of the 800-cell
+// shock tube 153 -> 125.
+constexpr unsigned CFL_FOLD_BLOCKS = 64;
+__global__ __launch_bounds__(256) void k_cfl_fold(const double* part, long long n, double* fold, unsigned* counter,
+                                                  double* out) {
+    auto reduce = [](const double* p, long long cnt, long long first, long long step, double* res) {
+        double m0 = 0.0, m1 = 0.0, m2 = 0.0;
+        for (long long b = first; b < cnt; b += step) {
+            m0 = fmax(m0, p[3 * b]);
+            m1 = fmax(m1, p[3 * b + 1]);
+            m2 = fmax(m2, p[3 * b + 2]);
+        }
+        block_max3(m0, m1, m2, res);
+    };
+    if (gridDim.x == 1) {
+        reduce(part, n, threadIdx.x, 256, out);
+        return;
     }
-    __shared__ double bm[3];
-    block_max3(m0, m1, m2, bm);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) atomicMax(&out[d], (unsigned long long)__double_as_longlong(bm[d]));
+    reduce(part, n, (long long)blockIdx.x * 256 + threadIdx.x, (long long)gridDim.x * 256, fold + 3 * blockIdx.x);
+    if (last_block(counter)) reduce(fold, gridDim.x, threadIdx.x, 256, out);
 }
 
 // The same maxima of a q(0) that the caller holds on the device in the
@@ -79,45 +103,53 @@ __global__ __launch_bounds__(256) void k_cfl_ref_fold(double* part, int nb) {
     block_max3(m0, m1, m2, part + 3 * CFL_REF_BLOCKS);
 }
 
-__global__ void k_zero_u64(unsigned long long* p, int n) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0ull;
-}
-
-// Adds the wavefront words of a step's routed sweeps (flagged | valid << 8;
-// n tiles of four, over the five stages) to the four totals (flagged, total,
-// wavefronts flagged, wavefronts total) and to (flagged, total) of the step in
-// last[0..1] (cleared before the launch).  Grid-stride loop; one atomic per
-// total and block.
-__global__ __launch_bounds__(256) void k_fold_wave_stats(const uint4* w, long long n, unsigned long long* tot,
-                                                         unsigned long long* last) {
-    unsigned long long s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+// Sums the wavefront words of a step's routed sweeps (flagged | valid << 8;
+// n tiles of four, over the five stages): adds (flagged, total, wavefronts
+// flagged, wavefronts total) to the totals tot and leaves (flagged, total) of
+// the step in last[0..1].  With `host`, the totals go there (pinned memory)
+// and start from zero again (rotor 512^2, FP32 + indicator: 299 -> 273 us a
+// step with the CFL fold).  fold: four sums per block.
+constexpr unsigned STAT_FOLD_BLOCKS = 256;
+__global__ __launch_bounds__(256) void k_fold_wave_stats(const uint4* w, long long n, unsigned long long* fold,
+                                                         unsigned* counter, unsigned long long* tot,
+                                                         unsigned long long* last, unsigned long long* host) {
+    unsigned long long s[4] = {0, 0, 0, 0};
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
         const uint4 v = w[i];
         const unsigned k[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const unsigned flagged = k[j] & 0xffu;
-            s0 += flagged;
-            s1 += k[j] >> 8;
-            s2 += flagged ? 1u : 0u;
-            s3 += k[j] ? 1u : 0u;
+            s[0] += flagged;
+            s[1] += k[j] >> 8;
+            s[2] += flagged ? 1u : 0u;
+            s[3] += k[j] ? 1u : 0u;
         }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        s0 += __shfl_down(s0, o, 64);
-        s1 += __shfl_down(s1, o, 64);
-        s2 += __shfl_down(s2, o, 64);
-        s3 += __shfl_down(s3, o, 64);
-    }
     __shared__ unsigned long long red[4][4];
-    const int wv = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { red[0][wv] = s0; red[1][wv] = s1; red[2][wv] = s2; red[3][wv] = s3; }
-    __syncthreads();
+    auto block_sum = [&]() -> unsigned long long {  // of s[k] in thread k < 4
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s[j] += __shfl_down(s[j], o, 64);
+        __syncthreads();  // red is free
+        if ((threadIdx.x & 63) == 0)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[j][threadIdx.x >> 6] = s[j];
+        __syncthreads();
+        return threadIdx.x < 4 ? red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3] : 0;
+    };
+    unsigned long long v = block_sum();
+    if (threadIdx.x < 4) fold[4 * blockIdx.x + threadIdx.x] = v;
+    if (!last_block(counter)) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = threadIdx.x < gridDim.x ? fold[4 * threadIdx.x + j] : 0;
+    v = block_sum();
     if (threadIdx.x < 4) {
         const int k = threadIdx.x;
-        const unsigned long long v = red[k][0] + red[k][1] + red[k][2] + red[k][3];
-        atomicAdd(&tot[k], v);
-        if (k < 2) atomicAdd(&last[k], v);
+        if (k < 2) last[k] = v;
+        v += tot[k];
+        if (host) host[k] = v;
+        tot[k] = host ? 0 : v;
     }
 }
 

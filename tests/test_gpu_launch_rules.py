@@ -66,3 +66,32 @@ def test_timed_launches_change_no_bit(require_gpu):
                 assert [g.timing()[k][1] for k in ("sweep_x", "sweep_y", "sweep_z")] == [10, 10, 10]
             out.append(g.q0())
     assert np.array_equal(out[0].view(np.int64), out[1].view(np.int64))
+
+
+# CFL maxima folded by one block (at most 512 partials) and by several, from
+# q(0) after the upload and from the step's own maxima
+@pytest.mark.parametrize("n", [(131072, 1, 1), (131073, 1, 1), (700, 800, 1)])
+def test_cfl_fold(n, require_gpu):
+    _step_matches("mpi_smooth3d", n, "periodic", steps=2)
+
+
+def test_counts_fold_over_blocks(require_gpu):
+    """Routed counts over more tiles than one block folds, in both counting
+    modes: every interface is counted once per sweep and stage."""
+    run = H.parse(H.make_input(problem="mhd_blast3d", nx=72, ny=64, nz=70, nt=1, tend=1.0))
+    q0 = H.init_problem(run)
+    P, thr = H.load_indicator(H.PKG_DIR / "weights" / "indicator_mlp.txt")
+    seen = []
+    for mode in (1, 2):
+        with H.GpuSolver(H.gpu_params(run)) as g:
+            g.set_indicator(P, thr, enable=mode)
+            g.upload_q0(q0)
+            g.init_faces()
+            for _ in range(3):
+                g.ssprk(g.tstep())
+            st = g.indicator_stats()
+            assert st["total"] == 3 * 5 * 3 * 72 * 64 * 70 and 0 < st["flagged"] < st["total"]
+            assert 0.0 < g.diag().flagged_fraction < 1.0
+            seen.append((st["flagged"], st["waves_flagged"], st["waves_total"], g.diag().flagged_fraction))
+            assert g.indicator_stats()["total"] == 0
+    assert seen[0] == seen[1]
