@@ -47,8 +47,12 @@ struct howmhd_gpu_ctx {
     unsigned long long* statfold = nullptr;
     unsigned* done = nullptr;
     double* vmax_host = nullptr;
-    // CFL maxima per block of the last stage-5 combination (3 per block of
-    // k_combine); cfl_fresh: they belong to the current q(0)
+    // grids of one x-y plane run k_plane after the sweeps
+    bool plane = false;
+    // blocks of the stage combination (k_combine or k_plane)
+    long long ncombine = 0;
+    // CFL maxima per block of the last stage-5 combination (3 per block);
+    // cfl_fresh: they belong to the current q(0)
     double* cflpart = nullptr;
     bool cfl_fresh = false;
     // cells whose density / pressure floor the stage-5 prot applied, per

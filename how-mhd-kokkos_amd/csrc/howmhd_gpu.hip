@@ -258,8 +258,13 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
     small((void**)&c->cflfold, 3 * CFL_FOLD_BLOCKS * sizeof(double));
     small((void**)&c->statfold, 4 * STAT_FOLD_BLOCKS * sizeof(unsigned long long));
     small((void**)&c->done, 2 * sizeof(unsigned));
-    small((void**)&c->cflpart, 3 * (size_t)blocks_for(c->ncell, 256) * sizeof(double));
-    small((void**)&c->floorpart, 2 * (size_t)blocks_for(c->ncell, 256) * sizeof(unsigned));
+    c->plane = n[0] > 1 && n[1] > 1 && n[2] == 1;
+    const dim3 pg = plane_grid(c->g);
+    c->ncombine = c->plane ? (long long)pg.x * pg.y : blocks_for(c->ncell, 256);
+    // (k_cfl leaves its partials in cflpart, too)
+    const size_t nred = std::max<size_t>(c->ncombine, blocks_for(c->ncell, 256));
+    small((void**)&c->cflpart, 3 * nred * sizeof(double));
+    small((void**)&c->floorpart, 2 * nred * sizeof(unsigned));
     small((void**)&c->diagpart, (size_t)DIAG_BLOCKS * DIAG_NV * sizeof(double));
     small((void**)&c->diagout, DIAG_NV * sizeof(double));
     c->xfer_slot = xfer_slot(c->ncell, n[2]);
@@ -357,11 +362,11 @@ int howmhd_gpu_tstep(howmhd_gpu_ctx* c, double* dt) {
     if (!c || !dt) return HOWMHD_EINVAL;
     {
         TimedLaunch tl(c, HOWMHD_K_CFL);
-        long long n = blocks_for(c->ncell, 256);
+        long long n = c->ncombine;
         // without the maxima of the last step's stage-5 combination, which
         // wrote q(0): those of q(0) itself
         if (!c->cfl_fresh) {
-            n = std::min<long long>(n, 2048);
+            n = std::min<long long>(blocks_for(c->ncell, 256), 2048);
             hipLaunchKernelGGL(k_cfl, dim3((unsigned)n), dim3(256), 0, c->stream, (const double*)c->qbuf[c->qid[0]],
                                c->g, c->ph, c->cflpart);
             HCHECK(c, hipGetLastError());
@@ -500,7 +505,7 @@ int howmhd_gpu_diag(howmhd_gpu_ctx* c, howmhd_diag* d) {
     a.dy = c->p.dy;
     a.dz = c->p.dz;
     a.floors = c->floors_fresh ? c->floorpart : nullptr;
-    a.nfloor = blocks_for(c->ncell, 256);
+    a.nfloor = c->ncombine;
     a.part = c->diagpart;
     const int nb = (int)std::min<size_t>(DIAG_BLOCKS, blocks_for(c->ncell, 256));
     hipLaunchKernelGGL(k_diag, dim3(nb), dim3(256), 0, c->stream, a);

@@ -1457,9 +1457,12 @@ __device__ __forceinline__ double i6(double a, double b, double c, double d, dou
 // (prot.cpp:10-51).  v receives the new q of the cell; rho_floor / p_floor
 // whether prot raised rho / p (a value below the floor or not a number:
 // fmax returns the floor for both).
-template <typename R>
+// With `centre` (k_plane) the cell-centred B comes from centre(v), else from the
+// faces in memory.
+struct FromMemory {};
+template <typename R, typename Centre = FromMemory>
 __device__ __forceinline__ void combine_cell(const CombineArgs<R>& A, long long i, int x, int y, int z, double* v,
-                                             bool& rho_floor, bool& p_floor) {
+                                             bool& rho_floor, bool& p_floor, const Centre& centre = Centre{}) {
     const Geom& g = A.g;
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
     const StageCoef& s = A.s;
@@ -1517,7 +1520,11 @@ __device__ __forceinline__ void combine_cell(const CombineArgs<R>& A, long long 
             v[m] = v[m] + d;
         }
     }
-    if (A.f.active) {
+    if constexpr (!std::is_same<Centre, FromMemory>::value) {
+        // (always true there; the branch keeps the FMA forms from fusing across
+        // it, so that they round as they do with the faces in memory)
+        if (A.f.active) centre(v);
+    } else if (A.f.active) {
         const double* bx = A.bo;
         const double* by = A.bo + g.ncell;
         const double* bz = A.bo + 2 * g.ncell;
@@ -1578,6 +1585,146 @@ __global__ __launch_bounds__(256) void k_combine(CombineArgs<R> A) {
     if (A.cfl) {
         block_max3(m0, m1, m2, A.cfl + 3 * (long long)blockIdx.x);
         block_count2(rho_floor, p_floor, A.floors + 2 * (long long)blockIdx.x);
+    }
+}
+
+// Everything of a stage after the sweeps, in one launch, for grids of one
+// plane (nz = 1, nx and ny above 1): corner EMF build and smoothing (k_emf2,
+// k_emf), face update (k_faces) and stage combination (k_combine), term for
+// term, on a PLANE_TX x PLANE_TY tile.  The intermediate arrays live in LDS
+// with the halos their stencils need, which neighbouring tiles compute again:
+//   face Bx     columns x0-3 .. x0+TX+1          (face -> centre along x)
+//   face By     rows    y0-3 .. y0+TY+1          (along y)
+//   Ox          columns and rows -3 .. +1 beyond the tile (D4 of the faces)
+//   O2x         one more on every side           (smoothing)
+//   gsx, fsy    -1 .. +2 more along x, along y   (EMF interpolation)
+// Positions are unmapped coordinates.  On a periodic axis a position beyond
+// the grid is a translation of its image and holds the image's value.  On an
+// open axis only positions inside the grid are computed, and a reader takes
+// the position clamped to the grid, as bmap does.
+//
+// Bound: a grid of this kind is small, and four launches of 3-8 us (each a
+// round trip through memory) were most of its step; on large planes the bytes:
+// O2x, Ox and the faces are not passed through memory.  Against the four
+// launches, a step: orszag_tang 64^2 169 -> 145 us, 128^2 183 -> 148, 256^2
+// 223 -> 188; rotor 512^2 FP64 504 -> 463, 2048^2 FP64 5.97 -> 5.77 ms, FP32 +
+// indicator 2.41 -> 2.30 ms.
+constexpr int PLANE_TX = 32, PLANE_TY = 8;
+
+__host__ __device__ inline dim3 plane_grid(const Geom& g) {
+    return dim3(blocks_for(g.n[0], PLANE_TX), blocks_for(g.n[1], PLANE_TY));
+}
+
+template <typename R>
+struct PlaneArgs {
+    FaceArgs<R> f;   // faces of the stages, coefficients (Ox, Oy, Oz unused)
+    CombineArgs<R> c;
+    const R *gsx, *fsy;
+};
+
+// Image of position a on an axis of n cells, any distance outside.
+__device__ __forceinline__ int image_of(int a, int n, int per) {
+    if (!per) return min(max(a, 0), n - 1);
+    a %= n;
+    return a < 0 ? a + n : a;
+}
+
+template <typename R, int EX>
+__global__ __launch_bounds__(256) void k_plane(PlaneArgs<R> A) {
+    static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
+    constexpr int TX = PLANE_TX, TY = PLANE_TY;
+    // column c (row r) of each array holds position x0 - its lower halo + c
+    constexpr int OX = TX + 5, OY = TY + 5;      // Ox: halo 3 | 2
+    constexpr int PX = OX + 2, PY = OY + 2;      // O2x: halo 4 | 3
+    constexpr int GX = PX + 3, FY = PY + 3;      // gsx: columns 5 | 5, fsy: rows 5 | 5
+    __shared__ R sg[PY][GX], sf[FY][PX], s2[PY][PX], so[OY][OX];
+    __shared__ double sbx[TY][OX], sby[OY][TX];
+    const Geom& g = A.c.g;
+    const StageCoef& s = A.c.s;
+    const int nx = g.n[0], ny = g.n[1], px = g.per[0], py = g.per[1];
+    const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY, tid = threadIdx.x;
+    auto imx = [&](int a) { return image_of(a, nx, px); };
+    auto imy = [&](int a) { return image_of(a, ny, py); };
+    // a position that holds a value: any on a periodic axis, else inside
+    auto has = [&](int x, int y) { return (px || (x >= 0 && x < nx)) && (py || (y >= 0 && y < ny)); };
+    // position whose value a reader of position a takes (open: clamped)
+    auto rx = [&](int a) { return px ? a : min(max(a, 0), nx - 1); };
+    auto ry = [&](int a) { return py ? a : min(max(a, 0), ny - 1); };
+
+    for (int e = tid; e < PY * GX; e += 256) {
+        const int r = e / GX, c = e % GX;
+        sg[r][c] = A.gsx[(size_t)imy(y0 - 4 + r) * nx + imx(x0 - 5 + c)];
+    }
+    for (int e = tid; e < FY * PX; e += 256) {
+        const int r = e / PX, c = e % PX;
+        sf[r][c] = A.fsy[(size_t)imy(y0 - 5 + r) * nx + imx(x0 - 4 + c)];
+    }
+    __syncthreads();
+    for (int e = tid; e < PY * PX; e += 256) {
+        const int r = e / PX, c = e % PX;
+        s2[r][c] = i4<R>(sg[r][c], sg[r][c + 1], sg[r][c + 2], sg[r][c + 3]) -
+                   i4<R>(sf[r][c], sf[r + 1][c], sf[r + 2][c], sf[r + 3][c]);
+    }
+    __syncthreads();
+    for (int e = tid; e < OY * OX; e += 256) {
+        const int r = e / OX, c = e % OX, x = x0 - 3 + c, y = y0 - 3 + r;
+        if (!has(x, y)) continue;
+        const int cl = rx(x - 1) - x0 + 4, cr = rx(x + 1) - x0 + 4, rl = ry(y - 1) - y0 + 4, rr = ry(y + 1) - y0 + 4;
+        const R o = s2[r + 1][c + 1];
+        so[r][c] = o + lap24<R>(s2[r + 1][cl], o, s2[r + 1][cr]) + lap24<R>(s2[rl][c + 1], o, s2[rr][c + 1]);
+    }
+    __syncthreads();
+    auto binit = [&](int m, size_t i) -> double {
+        const size_t o = (size_t)m * g.ncell + i;
+        return s.stage5 ? A.f.b0[o] + s.c4 * A.f.b2[o] + s.c5 * A.f.b3[o] : A.f.b0[o];
+    };
+    const double none = 0.0;  // the EMF differences along the axis of one cell
+    // Ox at the positions of a column or row stencil around (x, y)
+    auto ox = [&](int x, int y) -> double { return (double)so[ry(y) - y0 + 3][rx(x) - x0 + 3]; };
+    for (int e = tid; e < TY * OX; e += 256) {
+        const int r = e / OX, c = e % OX, x = x0 - 3 + c, y = y0 + r;
+        if (!has(x, y)) continue;
+        const size_t i = (size_t)imy(y) * nx + imx(x);
+        const double b = binit(0, i);
+        const double dOx = d4(ox(x, y - 3), ox(x, y - 2), ox(x, y - 1), ox(x, y), ox(x, y + 1), ox(x, y + 2));
+        const double v = s.k1 * b + s.k3 * A.f.bp[i] - s.dtdy * dOx + s.dtdz * none;
+        sbx[r][c] = v;
+        if (x >= x0 && x < x0 + TX && x < nx && y < ny) st_nt(&A.f.bo[i], v);
+    }
+    for (int e = tid; e < OY * TX; e += 256) {
+        const int r = e / TX, c = e % TX, x = x0 + c, y = y0 - 3 + r;
+        if (!has(x, y)) continue;
+        const size_t i = (size_t)imy(y) * nx + imx(x);
+        const double b = binit(1, i);
+        const double dOx = d4(ox(x - 3, y), ox(x - 2, y), ox(x - 1, y), ox(x, y), ox(x + 1, y), ox(x + 2, y));
+        const double v = s.k1 * b + s.k3 * A.f.bp[g.ncell + i] - s.dtdz * none + s.dtdx * dOx;
+        sby[r][c] = v;
+        if (y >= y0 && y < y0 + TY && x < nx && y < ny) st_nt(&A.f.bo[g.ncell + i], v);
+    }
+    __syncthreads();
+    const int x = x0 + tid % TX, y = y0 + tid / TX;
+    double m0 = 0.0, m1 = 0.0, m2 = 0.0;      // CFL maxima (stage 5)
+    bool rho_floor = false, p_floor = false;  // prot raised rho / p (stage 5)
+    if (x < nx && y < ny) {
+        const size_t i = (size_t)y * nx + x;
+        double v[8];
+        auto bx = [&](int a) { return sbx[y - y0][rx(a) - x0 + 3]; };
+        auto by = [&](int a) { return sby[ry(a) - y0 + 3][x - x0]; };
+        const double bz = binit(2, i);  // no CT update in the plane
+        st_nt(&A.f.bo[2 * g.ncell + i], bz);
+        combine_cell<R>(A.c, (long long)i, x, y, 0, v, rho_floor, p_floor, [&](double* w) {
+            w[4] = i6(bx(x - 3), bx(x - 2), bx(x - 1), bx(x), bx(x + 1), bx(x + 2));
+            w[5] = i6(by(y - 3), by(y - 2), by(y - 1), by(y), by(y + 1), by(y + 2));
+            w[6] = bz;
+        });
+#pragma unroll
+        for (int m = 0; m < 8; ++m) st_nt(&A.c.qo[(size_t)m * g.ncell + i], v[m]);
+        if (A.c.cfl) cfl_cell(v, A.c.ph, m0, m1, m2);
+    }
+    if (A.c.cfl) {
+        const size_t blk = blockIdx.x + (size_t)gridDim.x * blockIdx.y;
+        block_max3(m0, m1, m2, A.c.cfl + 3 * blk);
+        block_count2(rho_floor, p_floor, A.c.floors + 2 * blk);
     }
 }
 

@@ -178,6 +178,22 @@ CombineArgs<R> combine_args(howmhd_gpu_ctx* c, int iw, double dt) {
     return ca;
 }
 
+// The face update of stage iw.
+template <typename R>
+FaceArgs<R> face_args(howmhd_gpu_ctx* c, int iw, double dt) {
+    FaceArgs<R> fa{};
+    fa.Ox = (const R*)c->O[0]; fa.Oy = (const R*)c->O[1]; fa.Oz = (const R*)c->O[2];
+    fa.b0 = c->fbuf[c->qid[0]];
+    fa.b2 = c->fbuf[c->qid[2]];
+    fa.b3 = c->fbuf[c->qid[3]];
+    fa.bp = c->fbuf[c->qid[iw - 1]];
+    fa.bo = c->fbuf[c->qid[iw]];
+    fa.g = c->g;
+    fa.f = c->ctf;
+    fa.s = stage_coef(c, iw, dt);
+    return fa;
+}
+
 // The sweeps of a stage: one launch, or one per axis while the kernels are
 // being timed.
 template <typename R>
@@ -211,15 +227,17 @@ int launch_sweeps(howmhd_gpu_ctx* c, int iw, const double* qsrc) {
 
 template <typename R>
 int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
-    const StageCoef s = stage_coef(c, iw, dt);
     const double* qp = c->qbuf[c->qid[iw - 1]];
-    const double* b0 = c->fbuf[c->qid[0]];
-    const double* bp = c->fbuf[c->qid[iw - 1]];
-    double* bo = c->fbuf[c->qid[iw]];
-
     int rc = launch_sweeps<R>(c, iw, qp);
     if (rc) return rc;
 
+    if (c->plane) {
+        PlaneArgs<R> a{face_args<R>(c, iw, dt), combine_args<R>(c, iw, dt), (const R*)c->ct[2], (const R*)c->ct[0]};
+        TimedLaunch tl(c, HOWMHD_K_COMBINE);
+        hipLaunchKernelGGL((k_plane<R, EX>), plane_grid(c->g), dim3(256), 0, c->stream, a);
+        HCHECK(c, hipGetLastError());
+        return HOWMHD_OK;
+    }
     const unsigned nb = blocks_for(c->ncell, 256);
     if (c->ctf.use_x && c->ctf.use_y && c->ctf.use_z) {
         EmfMarchArgs<R> e;
@@ -260,16 +278,7 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
         }
         HCHECK(c, hipGetLastError());
     }
-    FaceArgs<R> fa;
-    fa.Ox = (const R*)c->O[0]; fa.Oy = (const R*)c->O[1]; fa.Oz = (const R*)c->O[2];
-    fa.b0 = b0;
-    fa.b2 = c->fbuf[c->qid[2]];
-    fa.b3 = c->fbuf[c->qid[3]];
-    fa.bp = bp;
-    fa.bo = bo;
-    fa.g = c->g;
-    fa.f = c->ctf;
-    fa.s = s;
+    FaceArgs<R> fa = face_args<R>(c, iw, dt);
     {
         TimedLaunch tl(c, HOWMHD_K_FACES);
         if (c->ctf.use_x && c->ctf.use_y && c->ctf.use_z) {

@@ -95,3 +95,12 @@ def test_counts_fold_over_blocks(require_gpu):
             seen.append((st["flagged"], st["waves_flagged"], st["waves_total"], g.diag().flagged_fraction))
             assert g.indicator_stats()["total"] == 0
     assert seen[0] == seen[1]
+
+
+# one-plane grids: everything after the sweeps in one launch of 32 x 8 tiles.
+# Axes shorter than the halos (3 to 5 cells), one cell more and less than a
+# tile, a last tile of one column or row, both boundaries
+@pytest.mark.parametrize("n", [(3, 3, 1), (5, 4, 1), (31, 7, 1), (32, 8, 1), (33, 9, 1), (64, 17, 1), (130, 77, 1)])
+@pytest.mark.parametrize("bc", ["periodic", "open"])
+def test_one_plane(n, bc, require_gpu):
+    _step_matches("mpi_smooth3d", n, bc, steps=2)
