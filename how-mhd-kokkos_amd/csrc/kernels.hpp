@@ -91,10 +91,19 @@ struct Phys {
 // Two tile shapes.  ALONG_X (x sweep): 64 interfaces along x per row, 4 rows
 // (y) per block.  ACROSS_X (y and z sweeps): HOWMHD_YZ_LANES x-columns,
 // 256/HOWMHD_YZ_LANES interfaces along the sweep axis per block.
-enum TileShape { ALONG_X = 0, ACROSS_X = 1 };
+// The split sweep (k_sweep_split) gives a block the 64 interfaces of one
+// wavefront: ALONG_X_64 a row of 64, ACROSS_X_64 16 x-columns of 4.
+enum TileShape { ALONG_X = 0, ACROSS_X = 1, ALONG_X_64 = 2, ACROSS_X_64 = 3 };
+__host__ __device__ constexpr bool along_x(int ts) { return ts == ALONG_X || ts == ALONG_X_64; }
 template <int TS> struct SweepTile;
 template <> struct SweepTile<ALONG_X> {
     static constexpr int LANES = 64, ROWS = 4, CELLS = (64 + 5) * 4;
+};
+template <> struct SweepTile<ALONG_X_64> {
+    static constexpr int LANES = 64, ROWS = 1, CELLS = 64 + 5;
+};
+template <> struct SweepTile<ACROSS_X_64> {
+    static constexpr int LANES = 16, ROWS = 4, CELLS = 16 * (4 + 5);
 };
 #ifndef HOWMHD_YZ_LANES
 #define HOWMHD_YZ_LANES 32
@@ -120,11 +129,12 @@ template <> struct SweepTile<ACROSS_X> {
 __host__ __device__ inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // Tiles of the sweep along axis d: (x tiles, tiles along the second axis,
-// planes).
+// planes), in the shapes SX along x and SA across it.
+template <int SX = ALONG_X, int SA = ACROSS_X>
 __host__ __device__ inline dim3 sweep_grid(const Geom& g, int d) {
     const int nif = g.per[d] ? g.n[d] : g.n[d] + 1;
-    using X = SweepTile<ALONG_X>;
-    using T = SweepTile<ACROSS_X>;
+    using X = SweepTile<SX>;
+    using T = SweepTile<SA>;
     if (d == 0) return dim3(blocks_for(nif, X::LANES), blocks_for(g.n[1], X::ROWS), g.n[2]);
     return dim3(blocks_for(g.n[0], T::LANES), blocks_for(nif, T::ROWS), d == 1 ? g.n[2] : g.n[1]);
 }
@@ -269,21 +279,29 @@ __device__ __forceinline__ void opaque(Eig<R>& o) {
     opq(o.sqrtrho); opq(o.invsqrtrho); opq(o.nrm_half); opq(o.nrm_ent);
 }
 
+// LDS slot of stencil cell k = 0..5 of the interface of phase-2 thread (row,
+// lane).
+template <int TS>
+__device__ __forceinline__ int stencil_slot(int row, int lane, int k) {
+    using T = SweepTile<TS>;
+    if constexpr (along_x(TS)) return row * (T::LANES + 5) + lane + k;
+    else return (row + k) * T::LANES + lane;
+}
+
 // Characteristic LLF-WENO5 flux of the interface of phase-2 thread (row,
 // lane) from the sweep tile in LDS (src/ssprk.cpp:825-946): interface
 // eigensystem, the 7 wave maxima, then the waves in pairs, added to dFo in
 // wave order.  The WENO weights divide in mode DM (DivMode); `bad` collects
 // the lanes whose operands left the range of the unscaled division.
-template <typename R, int TS, int MODE, int DM>
+// ONLY >= 0: that pass alone; the products of its waves with their columns of
+// R go to prod[(wave * 7 + component) * 64] instead of into dFo.
+template <typename R, int TS, int MODE, int DM, int ONLY = -1>
 __device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>::CELLS],
                                                const R (*lo)[SweepTile<TS>::CELLS], int row, int lane, R gam,
-                                               const GasConst& gc, R (&dFo)[7], R& mdev, unsigned long long& bad) {
-    using T = SweepTile<TS>;
+                                               const GasConst& gc, R (&dFo)[7], R& mdev, unsigned long long& bad,
+                                               R* prod = nullptr) {
     (void)mdev;
-    auto slot = [&](int k) -> int {
-        if constexpr (TS == ALONG_X) return row * (T::LANES + 5) + lane + k;
-        else return (row + k) * T::LANES + lane;
-    };
+    auto slot = [&](int k) -> int { return stencil_slot<TS>(row, lane, k); };
     // interface state from cells k = 2, 3: (rho, vn, vt1, vt2, Bn, Bt1, Bt2, p, H)
     R u0[9], u1[9];
     {
@@ -342,6 +360,7 @@ __device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>:
     };
     sfor<0, 4>([&](auto pc) {
         constexpr int P = decltype(pc)::value;
+        if constexpr (ONLY >= 0 && P != ONLY) return;
         constexpr int ma = P;                // 0, 1, 2, 3
         constexpr int mb = 6 - P;            // 6, 5, 4 (3: none)
         constexpr bool two = (P < 3);
@@ -412,6 +431,21 @@ __device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>:
         }
         opaque_after(e, Fsa);
         if constexpr (two) opaque_after(e, Fsb);
+        if constexpr (ONLY >= 0) {
+            // (products that add_col and add_prod skip are +-0: 0 here)
+            R Rc[7];
+            r_col<ma>(gam, e, Rc, gc);
+#pragma unroll
+            for (int r = 0; r < 7; ++r)
+                prod[(ma * 7 + r) * 64] = (ma == 1 && r < 2) || (ma == 3 && (r == 4 || r == 5)) ? R(0) : Rc[r] * Fsa;
+            if constexpr (two) {
+                R Rb[7];
+                r_col<mb>(gam, e, Rb, gc);
+#pragma unroll
+                for (int r = 0; r < 7; ++r) prod[(mb * 7 + r) * 64] = mb == 5 && r < 2 ? R(0) : Rb[r] * Fsb;
+            }
+            return;
+        }
         R Rc[7];
         r_col<ma>(gam, e, Rc, gc);
         add_col(std::integral_constant<int, ma>{}, Rc, Fsa);
@@ -458,7 +492,7 @@ __device__ __forceinline__ unsigned tile_cell_index(const Geom& g, const SweepAx
     using T = SweepTile<TS>;
     int along;
     unsigned base;
-    if constexpr (TS == ALONG_X) {
+    if constexpr (along_x(TS)) {
         const int row = s / (T::LANES + 5), c = s % (T::LANES + 5);
         along = t0 - 3 + c;
         int cy = a0 + row;
@@ -473,7 +507,7 @@ __device__ __forceinline__ unsigned tile_cell_index(const Geom& g, const SweepAx
     }
     if (along > X.n + 2) along = X.n + 2;
     const int a = bmap(along, X.n, X.per);
-    if constexpr (TS == ALONG_X) return base + a;
+    if constexpr (along_x(TS)) return base + a;
     else return base + (unsigned)a * X.sA;
 }
 
@@ -532,7 +566,7 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
     const int lane = tid % T::LANES, row = tid / T::LANES;
     int t, x, o;  // interface; ALONG_X: (y, z) = (x, o), ACROSS_X: column and other coordinate
     bool valid;
-    if constexpr (TS == ALONG_X) {
+    if constexpr (along_x(TS)) {
         t = t0 + lane; x = a0 + row; o = b0;
         valid = (t <= nd && x < g.n[1]);
     } else {
@@ -540,13 +574,13 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
         valid = (t <= nd && x < g.n[0]);
     }
     auto slot = [&](int k) -> int {
-        if constexpr (TS == ALONG_X) return row * (T::LANES + 5) + lane + k;
+        if constexpr (along_x(TS)) return row * (T::LANES + 5) + lane + k;
         else return (row + k) * T::LANES + lane;
     };
     // index of interface u = t - tbeg among the samples
     auto sample = [&]() -> unsigned {
         const unsigned u = t - (X.per ? 1 : 0);
-        if constexpr (TS == ALONG_X) return ((unsigned)o * g.n[1] + x) * X.oS + u;
+        if constexpr (along_x(TS)) return ((unsigned)o * g.n[1] + x) * X.oS + u;
         else return u * X.sS + (unsigned)o * X.oS + x;
     };
     // indicator features: the 6-cell stencils of rho, p and |B|
@@ -616,7 +650,7 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
 
     // dF and (below) the CT terms of the cell left of the interface
     unsigned fi, ci;
-    if constexpr (TS == ALONG_X) {
+    if constexpr (along_x(TS)) {
         const unsigned r = (unsigned)o * g.n[1] + x;
         fi = r * (nd + 1) + t;
         ci = r * nd + (t - 1);
@@ -684,8 +718,8 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
     const int tid = threadIdx.x;
     const int gy = (int)X.gy;
     // tile origin: first interface, first column (ALONG_X: first row y), plane
-    auto first_if = [&](int by) { return tbeg + (TS == ALONG_X ? bx * T::LANES : by * T::ROWS); };
-    const int a0 = TS == ALONG_X ? by0 * T::ROWS : bx * T::LANES;
+    auto first_if = [&](int by) { return tbeg + (along_x(TS) ? bx * T::LANES : by * T::ROWS); };
+    const int a0 = along_x(TS) ? by0 * T::ROWS : bx * T::LANES;
     auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * (by + (long long)gy * bz); };
     // a cell without positive shared reciprocals: the tile goes (once) on the
     // list of the IEEE-division launch that follows
@@ -849,6 +883,91 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             else across(A.ax[0]);
         }
     }
+}
+
+// The plain reference-rounding sweeps of a grid that leaves most of the chip
+// idle: a block has the 64 interfaces of one wavefront, and each of its four
+// wavefronts takes one projection pass ((0,6), (1,5), (2,4), (3)) of all of
+// them.  The products of the waves' fluxes with their columns of R meet in LDS
+// and are added in wave order, so every value is the one k_sweep computes.  A
+// tile with an operand out of the unscaled range is done again by the same
+// block with IEEE divisions: no recompute launch.  The eigensystem's scalars
+// are computed four times over, so this pays only while the chip has room
+// (split_sweep in stage.hpp).
+template <int EX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEEP_WAVES))) void k_sweep_split(
+    SweepArgs<double> A) {
+    static_assert(EX == HOWMHD_EXACT && EX == 1, "the reference-rounding form");
+    using R = double;
+    constexpr int CELLS = SweepTile<ACROSS_X_64>::CELLS;
+    static_assert(CELLS <= 256 && SweepTile<ALONG_X_64>::CELLS <= CELLS, "one cell per thread");
+    __shared__ alignas(16) unsigned char raw[tile_lds_bytes<R, SW_PLAIN, ACROSS_X_64>()];
+    __shared__ R prod[7 * 7 * 64];
+    auto tile = [&](auto tsc, const SweepAxis<R>& X) {
+        constexpr int TS = decltype(tsc)::value;
+        using T = SweepTile<TS>;
+        const unsigned L = blockIdx.x - X.first, rr = div(L, X.by_gx), uz = div(rr, X.by_gy);
+        const int bx = (int)(L - rr * X.gx), by = (int)(rr - uz * X.gy), bz = (int)uz;
+        const TileLds<R, TS> lds = tile_lds<R, TS>(raw);
+        const int tid = threadIdx.x, l = tid & 63, pass = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int t0 = (X.per ? 1 : 0) + (along_x(TS) ? bx * T::LANES : by * T::ROWS);
+        const int a0 = along_x(TS) ? by * T::ROWS : bx * T::LANES;
+        const int lane = l % T::LANES, row = l / T::LANES;
+        const int t = along_x(TS) ? t0 + lane : t0 + row, x = along_x(TS) ? a0 + row : a0 + lane;
+        const bool valid = t <= X.n && x < A.g.n[along_x(TS) ? 1 : 0];
+        double q[8];
+        if (tid < T::CELLS) {
+            const unsigned idx = tile_cell_index<R, TS>(A.g, X, tid, t0, a0, bz);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) q[m] = A.q[X.qoff[m] + idx];
+        }
+        auto compute = [&](auto dmc) -> bool {
+            constexpr int DM = decltype(dmc)::value;
+            bool cell_bad = false;
+            if (tid < T::CELLS) store_cell<R, TS, SW_PLAIN, DM>(A, lds, tid, q, cell_bad);
+            __syncthreads();
+            unsigned long long bad = 0ull;
+            if (valid) {
+                R none[7], dev;
+                auto one = [&](auto pc) {
+                    weno_interface<R, TS, SW_PLAIN, DM, decltype(pc)::value>(
+                        const_cast<const UF<R>(*)[T::CELLS]>(lds.luf), const_cast<const R(*)[T::CELLS]>(lds.lo), row,
+                        lane, A.ph.gam, A.gc, none, dev, bad, prod + l);
+                };
+                if (pass == 0) one(std::integral_constant<int, 0>{});
+                else if (pass == 1) one(std::integral_constant<int, 1>{});
+                else if (pass == 2) one(std::integral_constant<int, 2>{});
+                else one(std::integral_constant<int, 3>{});
+            }
+            return __syncthreads_or(cell_bad || bad != 0ull);  // the products are in LDS
+        };
+        if (compute(std::integral_constant<int, DIV_UNSCALED>{})) (void)compute(std::integral_constant<int, DIV_IEEE>{});
+        if (!valid) return;
+        unsigned fi, ci;
+        if constexpr (along_x(TS)) {
+            const unsigned r = (unsigned)bz * A.g.n[1] + x;
+            fi = r * (X.n + 1) + t;
+            ci = r * X.n + (t - 1);
+        } else {
+            fi = (unsigned)bz * X.oF + t * X.tF + x;
+            ci = (unsigned)bz * X.sB + (unsigned)(t - 1) * X.sA + x;
+        }
+        // components pass and pass + 4 of this wavefront's interfaces
+        for (int c = pass; c < 7; c += 4) {
+            R dF = R(0);
+#pragma unroll
+            for (int m = 0; m < 7; ++m) dF += prod[(m * 7 + c) * 64 + l];
+            if (!(A.ct_active && (c == 4 || c == 5))) X.dF[c * X.cF + fi] = dF;
+            if ((c == 4 || c == 5) && t >= 1) {  // CT term, as in sweep_interfaces
+                const int s2 = stencil_slot<TS>(row, lane, 2), s3 = stencil_slot<TS>(row, lane, 3);
+                const int vt = c == 4 ? O_VT1 : O_VT2;
+                const R b2 = lds.lo[O_BN][s2] * lds.lo[vt][s2], b3 = lds.lo[O_BN][s3] * lds.lo[vt][s3];
+                (c == 4 ? X.ct_a : X.ct_b)[ci] = dF + div_c<R>(R(9) * b2 + R(9) * b3, R(18), R(1.0 / 18.0));
+            }
+        }
+    };
+    if (blockIdx.x >= A.ax[2].first) tile(std::integral_constant<int, ALONG_X_64>{}, A.ax[2]);
+    else tile(std::integral_constant<int, ACROSS_X_64>{}, A.ax[blockIdx.x >= A.ax[1].first ? 1 : 0]);
 }
 
 template <typename R>

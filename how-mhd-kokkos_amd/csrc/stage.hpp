@@ -70,10 +70,30 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
     return (int)std::min<unsigned long long>(cz, (unsigned long long)most);
 }
 
+// Whether the plain reference-rounding sweeps of a stage run as k_sweep_split:
+// while its blocks are at most two rounds of the 512 the chip holds.  A round
+// of it takes 7-8 us where a tile of k_sweep takes 13 us and its recompute
+// launch 4, however few there are.  Per step: shock tube 800 cells 123 -> 82
+// us, 60,000 cells (938 blocks) 193 -> 143; orszag_tang 32^2 143 -> 105, 128^2
+// (512 blocks) 149 -> 118, 160^2 (880) 156 -> 160; 3-D 16^3 198 -> 157, 20^3
+// (800) 198 -> 188; beyond, 24^3 (1,152) 227 -> 215 but 28^3 (1,568) 232 -> 254
+// and 32^3 230 -> 273.
+constexpr unsigned kSplitBlocks = 1024;
+inline bool split_sweep(const howmhd_gpu_ctx* c) {
+    if (c->march_force > 0) return false;
+    unsigned long long n = 0;
+    for (int d = 0; d < 3; ++d) {
+        const dim3 t = sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d);
+        if (c->g.n[d] > 1) n += (unsigned long long)t.x * t.y * t.z;
+    }
+    return n <= kSplitBlocks;
+}
+
 // Arguments of stage iw's sweeps of the axes in `mask` (bit d: axis d) from qsrc;
 // *blocks receives the blocks of the launch.
 template <typename R, int MODE>
-SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned mask, unsigned* blocks) {
+SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned mask, unsigned* blocks,
+                        bool split = false) {
     SweepArgs<R> a{};
     a.q = qsrc;
     a.g = c->g;
@@ -107,12 +127,12 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
         x.oF = (unsigned)(d == 2 ? nx : nx * (ny + 1));
         x.sS = x.sA;
         x.oS = (unsigned)(d == 0 ? nif : d == 1 ? nx * nif : nx);
-        const dim3 gr = sweep_grid(c->g, d);
+        const dim3 gr = split ? sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d) : sweep_grid(c->g, d);
         x.gx = gr.x; x.gy = gr.y; x.gz = gr.z;
         x.first = nb;
         x.march = 1;
         x.tile0 = c->tile0[d];
-        if (d != 0 && sweep_marches<R, MODE>())
+        if (d != 0 && sweep_marches<R, MODE>() && !split)
             x.march = c->march_force > 0 ? (int)std::min<unsigned>(c->march_force, gr.y) : march_steps(gr);
         x.by_gx = launch_div(gr.x);
         x.by_gy = launch_div((gr.y + x.march - 1) / x.march);
@@ -207,6 +227,13 @@ int launch_sweeps(howmhd_gpu_ctx* c, int iw, const double* qsrc) {
             SweepArgs<R> a = sweep_args<R, SW_ROUTED>(c, iw, qsrc, mask, &nb);
             launch_sweep<R, SW_ROUTED>(c, a, nb);
         } else {
+            if constexpr (EX) {
+                if (split_sweep(c)) {
+                    const SweepArgs<R> a = sweep_args<R, SW_PLAIN>(c, iw, qsrc, mask, &nb, true);
+                    if (nb) hipLaunchKernelGGL((k_sweep_split<EX>), dim3(nb), dim3(256), 0, c->stream, a);
+                    return;
+                }
+            }
             SweepArgs<R> a = sweep_args<R, SW_PLAIN>(c, iw, qsrc, mask, &nb);
             launch_sweep<R, SW_PLAIN>(c, a, nb);
         }

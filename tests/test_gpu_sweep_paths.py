@@ -1,0 +1,44 @@
+"""The reference-rounding sweeps of the smallest grids run split over the
+wavefronts of a block, the others as tiles that may march and that queue tiles
+for an IEEE-division launch (needs a GPU).  Every parity case is small enough
+for the split sweep; here the same cases run on the other one
+(HOWMHD_SWEEP_MARCH), bit for bit against the CPU restatement: the case list,
+operands beyond the unscaled divisions, subnormal squares, a cell without
+positive density, and one cell along x.  And a grid on each side of the rule.
+"""
+import pytest
+
+import test_gpu_parity as P
+from test_gpu_launch_rules import _step_matches
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=["1", "2"])
+def tiles(request, monkeypatch):
+    monkeypatch.setenv("HOWMHD_SWEEP_MARCH", request.param)
+    print(f"[sweep paths] {request.param} tiles a block", flush=True)
+
+
+@pytest.mark.parametrize("case", list(P.CASES))
+def test_tiles_on_parity_cases(case, tiles, require_gpu):
+    P.test_fp64_bitwise(case, require_gpu)
+
+
+@pytest.mark.parametrize("problem,kw", [("mhd_blast3d", dict(nx=16, ny=16, nz=16)),
+                                        ("orszag_tang", dict(nx=32, ny=32, nz=1, cour=0.8))])
+def test_tiles_recompute(problem, kw, tiles, require_gpu):
+    P.test_fp64_bitwise_large_weno_operands(problem, kw, require_gpu)
+    P.test_fp64_bitwise_small_sqrt_operands(problem, kw, require_gpu)
+    P.test_fp64_bitwise_nonpositive_density_cell(-0.25, require_gpu)
+    P.test_fp64_bitwise_nonpositive_density_cell(1e-300, require_gpu)
+    P.test_fp64_bitwise_degenerate_x("mpi_smooth3d", dict(nx=1, ny=12, nz=10), require_gpu)
+
+
+# 1,024 blocks of the split sweep (the last grid it takes), 1,048 and 1,428;
+# interfaces that fill the 64 of a block and one more, last columns of 1 to 15
+@pytest.mark.parametrize("n,bc", [((256, 128, 1), "periodic"), ((256, 130, 1), "periodic"), ((65, 17, 17), "open"),
+                                  ((64, 20, 18), "open"), ((63, 5, 3), "open"), ((64, 16, 1), "periodic"),
+                                  ((65, 17, 1), "open")])
+def test_split_rule(n, bc, require_gpu):
+    _step_matches("mpi_smooth3d", n, bc, steps=2)
