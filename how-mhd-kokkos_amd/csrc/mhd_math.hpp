@@ -350,7 +350,9 @@ struct GasConst {
 template <typename R>
 struct Eig {
     R vx, vy, vz, By, Bz, vv2, cs, cs2, lf, ls, af, as, bty, btz, sgnBx, sqrtrho, invsqrtrho;
-    R nrm_half, nrm_ent;  // FMA form: 0.5/cs2 and (gam-1)/cs2; reference rounding: nrm_half = RN(1/cs2)
+    // FMA form: half of the normalisations 0.5/cs2 and (gam-1)/cs2 (weno_wave);
+    // reference rounding: nrm_half = RN(1/cs2)
+    R nrm_half, nrm_ent;
 };
 
 // FP32 form: fast/slow speeds and the alpha_f, alpha_s normalisations of
@@ -509,8 +511,8 @@ __device__ __forceinline__ void eig_scalars(R gam, const R* u0, const R* u1, Eig
 #endif
 #if !HOWMHD_EXACT
     const R ics2 = rcp_fast(cs2);
-    e.nrm_half = R(0.5) * ics2;
-    e.nrm_ent = (gam - R(1)) * ics2;
+    e.nrm_half = R(0.25) * ics2;
+    e.nrm_ent = R(0.5) * ((gam - R(1)) * ics2);
 #else
     // RN(1/cs2): the L-row normalisation divides by cs2 through it
     if constexpr (DM == DIV_UNSCALED) e.nrm_half = recip_rn(cs2);
@@ -606,7 +608,9 @@ __device__ __forceinline__ void l_row(R gam, const Eig<R>& e, R* L, const GasCon
         else if constexpr (DM == DIV_UNSCALED) L[c] = div_pos<R>(L[c], R(2) * cs2, R(0.5) * e.nrm_half);
         else L[c] = div_q<DM>(R(0.5) * L[c], cs2, e.nrm_half);
 #else
-        if constexpr (M == 1 || M == 5) L[c] = R(0.5) * L[c];
+        // half the reference's rows (Eig): the projected values come out
+        // halved, exactly, and the LLF splitting needs no product by 0.5
+        if constexpr (M == 1 || M == 5) L[c] = R(0.25) * L[c];
         else if constexpr (M == 3) L[c] = L[c] * e.nrm_ent;
         else L[c] = L[c] * e.nrm_half;
 #endif
@@ -767,6 +771,15 @@ __device__ __forceinline__ R weno_wave(const R* Fsk, const R* qsk, R amx, unsign
         dF[k] = Fsk[k + 1] - Fsk[k];
         dq[k] = qsk[k + 1] - qsk[k];
     }
+#if !HOWMHD_EXACT
+    // Fsk and qsk are half the projected values (l_row): their sums are the LLF
+    // halves, and `first` is doubled through its constant.  All by powers of
+    // two, so every value below has the bits of the unhalved form.
+    const R first = (-Fsk[1] + R(7) * Fsk[2] + R(7) * Fsk[3] - Fsk[4]) * (R(2) * R(1.0 / 12.0));
+    const R second = weno_side<R, DM>(dF[0] + amx * dq[0], dF[1] + amx * dq[1], dF[2] + amx * dq[2], dF[3] + amx * dq[3], bad);
+    const R third = weno_side<R, DM>(dF[4] - amx * dq[4], dF[3] - amx * dq[3], dF[2] - amx * dq[2], dF[1] - amx * dq[1], bad);
+    return first - second + third;
+#else
     const R first = div_c<R>(-Fsk[1] + R(7) * Fsk[2] + R(7) * Fsk[3] - Fsk[4], R(12), R(1.0 / 12.0));
     if constexpr (DM == DIV_UNSCALED) {
         // the halves of the LLF splitting are taken from the sums: eight
@@ -780,6 +793,7 @@ __device__ __forceinline__ R weno_wave(const R* Fsk, const R* qsk, R amx, unsign
     const R third = weno_side<R, DM>(R(0.5) * (dF[4] - amx * dq[4]), R(0.5) * (dF[3] - amx * dq[3]),
                                      R(0.5) * (dF[2] - amx * dq[2]), R(0.5) * (dF[1] - amx * dq[1]), bad);
     return first - second + third;
+#endif
 }
 
 // weno_wave that also raises `dev` to the largest |w_r - d_r| of both sides,
