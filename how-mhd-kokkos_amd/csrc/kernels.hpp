@@ -1286,6 +1286,7 @@ __device__ __forceinline__ double d4(double om3, double om2, double om1, double 
 
 // fluxct_update_bfield, src/fluxct.cpp:850-877, with the stage initialisation
 // of copy_bfield_stage / prepare_bfield_stage5 (111-135) folded in.
+// For the grids of two axes that k_plane does not take (xz and yz).
 // Block = FACE_TX x FACE_TY cells of one z plane.  The in-plane stencils
 // (Ox along x and y, Oy along y, Oz along x) are read from LDS copies of the
 // tile with its 3-cell halo (each value read once per block instead of six
@@ -1308,20 +1309,18 @@ __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
     // into the range bmap covers (those entries are never read)
     auto hx = [&](int c) { const int a = x0 - 3 + c; return bmap(a > nx + 2 ? nx + 2 : a, nx, px); };
     auto hy = [&](int r) { const int a = y0 - 3 + r; return bmap(a > ny + 2 ? ny + 2 : a, ny, py); };
-    if (f.active) {
-        if (f.use_Ox)
-            for (int k = tid; k < HY * HX; k += 256) sOx[k / HX][k % HX] = A.Ox[lin(g, hx(k % HX), hy(k / HX), z)];
-        if (f.use_Oy)
-            for (int k = tid; k < HY * FACE_TX; k += 256) {
-                const int c = k % FACE_TX, xx = x0 + c < nx ? x0 + c : nx - 1;
-                sOy[k / FACE_TX][c] = A.Oy[lin(g, xx, hy(k / FACE_TX), z)];
-            }
-        if (f.use_Oz)
-            for (int k = tid; k < FACE_TY * HX; k += 256) {
-                const int r = k / HX, yy = y0 + r < ny ? y0 + r : ny - 1;
-                sOz[r][k % HX] = A.Oz[lin(g, hx(k % HX), yy, z)];
-            }
-    }
+    if (f.use_Ox)
+        for (int k = tid; k < HY * HX; k += 256) sOx[k / HX][k % HX] = A.Ox[lin(g, hx(k % HX), hy(k / HX), z)];
+    if (f.use_Oy)
+        for (int k = tid; k < HY * FACE_TX; k += 256) {
+            const int c = k % FACE_TX, xx = x0 + c < nx ? x0 + c : nx - 1;
+            sOy[k / FACE_TX][c] = A.Oy[lin(g, xx, hy(k / FACE_TX), z)];
+        }
+    if (f.use_Oz)
+        for (int k = tid; k < FACE_TY * HX; k += 256) {
+            const int r = k / HX, yy = y0 + r < ny ? y0 + r : ny - 1;
+            sOz[r][k % HX] = A.Oz[lin(g, hx(k % HX), yy, z)];
+        }
     __syncthreads();
     const int tx = tid % FACE_TX, ty = tid / FACE_TX;
     const int x = x0 + tx, y = y0 + ty;
@@ -1348,27 +1347,25 @@ __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
                   (double)r[tx + 5]);
     };
     double bx = binit[0], by = binit[1], bz = binit[2];
-    if (f.active) {
-        if (f.use_Ox || f.use_Oz) {
-            double dOx = 0.0, dOz = 0.0;
-            if (f.use_Ox) dOx = col6(sOx, tx + 3);
-            if (f.use_Oz) dOz = dz_of(A.Oz);
-            bx = s.k1 * binit[0] + s.k3 * A.bp[i] - s.dtdy * dOx + s.dtdz * dOz;
-        }
-        if (f.use_Oy || f.use_Ox) {
-            double dOy = 0.0, dOx = 0.0;
-            if (f.use_Oy) dOy = dz_of(A.Oy);
-            if (f.use_Ox) dOx = row6(sOx[ty + 3]);
-            by = s.k1 * binit[1] + s.k3 * A.bp[g.ncell + i] - s.dtdz * dOy + s.dtdx * dOx;
-        }
-        if (f.use_Oz || f.use_Oy) {
-            double dOz = 0.0, dOy = 0.0;
-            if (f.use_Oz) dOz = row6(sOz[ty]);
-            if (f.use_Oy)
-                dOy = d4((double)sOy[ty][tx], (double)sOy[ty + 1][tx], (double)sOy[ty + 2][tx], (double)sOy[ty + 3][tx],
-                         (double)sOy[ty + 4][tx], (double)sOy[ty + 5][tx]);
-            bz = s.k1 * binit[2] + s.k3 * A.bp[2 * g.ncell + i] - s.dtdx * dOz + s.dtdy * dOy;
-        }
+    if (f.use_Ox || f.use_Oz) {
+        double dOx = 0.0, dOz = 0.0;
+        if (f.use_Ox) dOx = col6(sOx, tx + 3);
+        if (f.use_Oz) dOz = dz_of(A.Oz);
+        bx = s.k1 * binit[0] + s.k3 * A.bp[i] - s.dtdy * dOx + s.dtdz * dOz;
+    }
+    if (f.use_Oy || f.use_Ox) {
+        double dOy = 0.0, dOx = 0.0;
+        if (f.use_Oy) dOy = dz_of(A.Oy);
+        if (f.use_Ox) dOx = row6(sOx[ty + 3]);
+        by = s.k1 * binit[1] + s.k3 * A.bp[g.ncell + i] - s.dtdz * dOy + s.dtdx * dOx;
+    }
+    if (f.use_Oz || f.use_Oy) {
+        double dOz = 0.0, dOy = 0.0;
+        if (f.use_Oz) dOz = row6(sOz[ty]);
+        if (f.use_Oy)
+            dOy = d4((double)sOy[ty][tx], (double)sOy[ty + 1][tx], (double)sOy[ty + 2][tx], (double)sOy[ty + 3][tx],
+                     (double)sOy[ty + 4][tx], (double)sOy[ty + 5][tx]);
+        bz = s.k1 * binit[2] + s.k3 * A.bp[2 * g.ncell + i] - s.dtdx * dOz + s.dtdy * dOy;
     }
     st_nt(&A.bo[i], bx);
     st_nt(&A.bo[g.ncell + i], by);
@@ -1706,10 +1703,23 @@ __device__ __forceinline__ void combine_cell(const CombineArgs<R>& A, long long 
     v[0] = rho;
 }
 
+// Stage combination of the faces of cell i (src/fluxct.cpp:111-135).
+template <typename R>
+__device__ __forceinline__ void face_init(const FaceArgs<R>& A, long long i, double* b) {
+    const StageCoef& s = A.s;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const long long o = (long long)c * A.g.ncell + i;
+        b[c] = s.stage5 ? A.b0[o] + s.c4 * A.b2[o] + s.c5 * A.b3[o] : A.b0[o];
+    }
+}
+
 // The stage combination over every cell (one thread per cell); at stage 5
-// also the per-block CFL maxima and floor counts.
-template <typename R, int EX>
-__global__ __launch_bounds__(256) void k_combine(CombineArgs<R> A) {
+// also the per-block CFL maxima and floor counts.  LINE: a grid with one axis
+// of more than one cell has no EMF, its faces are only carried through the
+// stages, and that is done here instead of in a launch of k_faces.
+template <typename R, int EX, bool LINE>
+__global__ __launch_bounds__(256) void k_combine(CombineArgs<R> A, FaceArgs<R> F) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     const Geom& g = A.g;
@@ -1722,6 +1732,12 @@ __global__ __launch_bounds__(256) void k_combine(CombineArgs<R> A) {
         combine_cell<R>(A, i, x, y, z, v, rho_floor, p_floor);
 #pragma unroll
         for (int m = 0; m < 8; ++m) st_nt(&A.qo[(long long)m * g.ncell + i], v[m]);
+        if constexpr (LINE) {
+            double b[3];
+            face_init(F, i, b);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) st_nt(&F.bo[(long long)c * g.ncell + i], b[c]);
+        }
         if (A.cfl) cfl_cell(v, A.ph, m0, m1, m2);
     }
     if (A.cfl) {

@@ -306,7 +306,7 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
         HCHECK(c, hipGetLastError());
     }
     FaceArgs<R> fa = face_args<R>(c, iw, dt);
-    {
+    if (c->ctf.active) {
         TimedLaunch tl(c, HOWMHD_K_FACES);
         if (c->ctf.use_x && c->ctf.use_y && c->ctf.use_z) {
             dim3 fgrid(blocks_for(c->g.n[0], FACE_TX), blocks_for(c->g.n[1], FACE_TY));
@@ -323,7 +323,10 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
     {
         const CombineArgs<R> ca = combine_args<R>(c, iw, dt);
         TimedLaunch tl(c, HOWMHD_K_COMBINE);
-        hipLaunchKernelGGL((k_combine<R, EX>), dim3(nb), dim3(256), 0, c->stream, ca);
+        if (c->ctf.active)
+            hipLaunchKernelGGL((k_combine<R, EX, false>), dim3(nb), dim3(256), 0, c->stream, ca, fa);
+        else
+            hipLaunchKernelGGL((k_combine<R, EX, true>), dim3(nb), dim3(256), 0, c->stream, ca, fa);
     }
     HCHECK(c, hipGetLastError());
     return HOWMHD_OK;
