@@ -8,15 +8,15 @@
 // without ghosts.  Host threads move chunks between the caller's (pageable)
 // memory and their slots, filling the ghost layers with their images on the
 // way down, while the transpose kernel reads or writes the other slots of the
-// pinned memory over PCIe; each thread owns two slots, so that its copy
-// overlaps its kernel.
+// pinned memory over PCIe; on large grids each thread owns two slots, so that
+// its copy overlaps its kernel.
 //
 // Bound: PCIe (56 GB/s each way) for large grids, the first touch of the
 // caller's pages on the way down, the start of the threads and one chunk's
 // latency for small ones.  q(0) up and down, against one variable at a time
 // through the runtime's pageable copies, ghosts included: 256^3 (1.15 GB)
-// 39 -> 23 and 111 -> 35 ms, 512x512 4.3 -> 1.2 and 12.1 -> 3.6 ms, 32^3
-// 0.24 -> 0.17 and 0.41 -> 0.25 ms.
+// 39 -> 23 and 111 -> 35 ms, 512x512 4.2 -> 0.96 and 11.9 -> 3.3 ms, 48x40x50
+// 0.42 -> 0.37 and 0.74 -> 0.38 ms, 32^3 0.24 -> 0.16 and 0.37 -> 0.19 ms.
 #pragma once
 
 #include "context.hpp"
@@ -37,19 +37,22 @@
 namespace howmhd {
 namespace {
 
-constexpr int kXferThreads = 8, kXferSlots = 2 * kXferThreads;
+constexpr int kXferThreads = 8, kXferChunks = 2 * kXferThreads;
 constexpr size_t kXferSlotMax = 1u << 18, kXferSlotMin = 1u << 15;  // values: 2 MiB, 256 KiB
 
-// Values per slot and slots of a context of ncell cells: two chunks for every
-// slot when eight variables move, within the bounds; a row of nz values fits.
-// (One chunk a slot pins twice the memory of a mid-sized grid, which create
-// pays for: 512x512 5.6 against 3.7 ms; four leave 64^3 with 256 KiB chunks,
-// up in 0.89 instead of 0.69 ms.)
+// Values per slot of a context of ncell cells: eight variables in 16 chunks,
+// within the bounds; a row of nz values fits.  (32 chunks: 48x40x50 up in 0.52
+// instead of 0.36 ms, because the chunks' kernels follow one another.)
 inline size_t xfer_slot(size_t ncell, int nz) {
-    return std::max(std::min(std::max(8 * ncell / (2 * kXferSlots), kXferSlotMin), kXferSlotMax), (size_t)nz);
+    return std::max(std::min(std::max(8 * ncell / kXferChunks, kXferSlotMin), kXferSlotMax), (size_t)nz);
 }
+// Slots: two a thread where the chunks are at their bound and every thread
+// moves many (144^3 down in 5.7 instead of 6.9 ms); else one, which costs the
+// transfer nothing and halves the memory that create pins and the first
+// transfer touches (64^3: first upload 1.20 against 1.58 ms).
 inline int xfer_slots(size_t ncell, size_t slot) {
-    return (int)std::min<size_t>(kXferSlots, (8 * ncell + slot - 1) / slot);
+    const size_t most = slot < kXferSlotMax ? kXferThreads : 2 * kXferThreads;
+    return (int)std::min(most, (8 * ncell + slot - 1) / slot);
 }
 
 struct Chunk {
