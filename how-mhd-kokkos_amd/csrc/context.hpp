@@ -39,7 +39,7 @@ struct howmhd_gpu_ctx {
     void* O2[3] = {};
     void* O[3] = {};
     // one allocation for the device arrays below of a few values per block or
-    // tile, and smaller ones (howmhd_gpu_create); vmax_host and istats_host lie behind the transfer slots
+    // tile, and smaller ones (howmhd_gpu_create); vmax_host, istats_host and fixhost lie behind the transfer slots
     void* arena = nullptr;
     // per-step reductions: partials of their blocks, counters of the blocks
     // done (zero between launches), and the CFL maxima in pinned host memory
@@ -86,6 +86,7 @@ struct howmhd_gpu_ctx {
     unsigned* fixflag = nullptr;
     unsigned* fixlist = nullptr;
     unsigned* fixctl = nullptr;
+    unsigned* fixhost = nullptr;  // pinned: a collecting sweep queued a tile
     unsigned long long* istats = nullptr;
     // (flagged, total) of the most recent routed step, and whether one ran
     unsigned long long* ilast = nullptr;

@@ -271,10 +271,11 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
     c->xfer_n = xfer_slots(c->ncell, c->xfer_slot);
     // pinned: the transfer slots, then what the per-step reductions tell
     const size_t pinned = c->xfer_n * c->xfer_slot;
-    ok = ok && hipHostMalloc((void**)&c->xfer, (pinned + 8) * sizeof(double), hipHostMallocDefault) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&c->xfer, (pinned + 9) * sizeof(double), hipHostMallocDefault) == hipSuccess;
     if (ok) {
         c->vmax_host = c->xfer + pinned;
         c->istats_host = (unsigned long long*)(c->vmax_host + 4);
+        c->fixhost = (unsigned*)(c->vmax_host + 8);
     }
     for (int s = 0; s < c->xfer_n && ok; ++s) {
         hipEvent_t ev = nullptr;
@@ -570,7 +571,6 @@ int howmhd_gpu_collect_samples(howmhd_gpu_ctx* c, int dir, float* X, float* y, i
     // recomputes them from its own source
     const int rc = collect_fp64(c, dir, X, y, nullptr);
     if (rc) return rc;
-    HCHECK(c, hipStreamSynchronize(c->stream));
     *count = need;
     return HOWMHD_OK;
 }
@@ -589,7 +589,6 @@ int howmhd_gpu_indicator_logits(howmhd_gpu_ctx* c, int dir, float* logits, int64
         return fail(c, HOWMHD_EINVAL, "howmhd_gpu_indicator_logits: needs precision fp64");
     const int rc = collect_fp64(c, dir, nullptr, nullptr, logits);
     if (rc) return rc;
-    HCHECK(c, hipStreamSynchronize(c->stream));
     *count = need;
     return HOWMHD_OK;
 }

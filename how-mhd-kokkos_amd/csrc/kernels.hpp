@@ -215,10 +215,12 @@ struct SweepArgs {
     // reference-rounding form: tiles whose WENO weight operands left the
     // range of the unscaled division, for the IEEE-division launch that
     // follows: a flag per tile slot (a tile is queued once), the queue, and
-    // (queue length, blocks done) of that launch
+    // (queue length, blocks done) of that launch; SW_COLLECT: fixhost (pinned)
+    // is set where a tile is queued
     unsigned* fix;
     unsigned* fixlist;
     unsigned* fixctl;
+    unsigned* fixhost;
     // the axes of the launch in the order of their blocks: y, z, x (an axis
     // without blocks starts where the next one does)
     SweepAxis<R> ax[3];
@@ -548,6 +550,14 @@ __device__ __forceinline__ void store_cell(const SweepArgs<R>& A, const TileLds<
         L.lbmag[s] = sqrtf((float)(out[C_BN] * out[C_BN] + out[C_BT1] * out[C_BT1] + out[C_BT2] * out[C_BT2]));
 }
 
+// The tile goes (once) on the list of the IEEE-division launch that follows.
+template <typename R, int MODE>
+__device__ __forceinline__ void queue_tile(const SweepArgs<R>& A, long long slot) {
+    if (atomicExch(&A.fix[slot], 1u) != 0u) return;
+    A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)slot;
+    if constexpr (MODE == SW_COLLECT) *A.fixhost = 1u;
+}
+
 // Phase 2 of a tile whose cell values are in LDS: one interface per thread
 // (t0, a0, b0: the tile origin; slot: its tile slot).
 template <typename R, int TS, int MODE, int EX, int DM>
@@ -621,10 +631,9 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
     if (MODE != SW_ROUTED || flagged) {
         unsigned long long bad = 0ull;
         weno_interface<R, TS, MODE, DM>(luf, lo, row, lane, R(A.ph.gam), A.gc, dF, maxdev, bad);
-        // a WENO weight operand beyond the unscaled-division range: the tile
-        // goes (once) on the list of the IEEE-division launch that follows
+        // a WENO weight operand beyond the unscaled-division range
         if constexpr (EX && DM == DIV_UNSCALED) {
-            if (bad && atomicExch(&A.fix[tslot], 1u) == 0u) A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)tslot;
+            if (bad) queue_tile<R, MODE>(A, tslot);
         }
     } else {
         // linear upwind-5 with one LLF speed: the largest |v_n| + c_f over the
@@ -721,12 +730,10 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
     auto first_if = [&](int by) { return tbeg + (along_x(TS) ? bx * T::LANES : by * T::ROWS); };
     const int a0 = along_x(TS) ? by0 * T::ROWS : bx * T::LANES;
     auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * (by + (long long)gy * bz); };
-    // a cell without positive shared reciprocals: the tile goes (once) on the
-    // list of the IEEE-division launch that follows
+    // a cell without positive shared reciprocals
     auto queue = [&](bool bad, long long slot) {
         if constexpr (EX && DM == DIV_UNSCALED) {
-            if (__ballot(bad) && atomicExch(&A.fix[slot], 1u) == 0u)
-                A.fixlist[atomicAdd(&A.fixctl[0], 1u)] = (unsigned)slot;
+            if (__ballot(bad)) queue_tile<R, MODE>(A, slot);
         }
     };
     // Loads of the next step's cell issued before the interfaces of this

@@ -105,6 +105,7 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
     a.fix = c->fixflag;
     a.fixlist = c->fixlist;
     a.fixctl = c->fixctl;
+    a.fixhost = c->fixhost;
     const long long nx = c->g.n[0], ny = c->g.n[1], nz = c->g.n[2];
     const int order[3] = {1, 2, 0};
     unsigned nb = 0;
@@ -142,9 +143,17 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
     return a;
 }
 
+// The IEEE-division launch for the tiles that the sweeps before it queued (it
+// exits at once when there are none; no counting there).
+template <typename R, int MODE>
+void launch_recompute(howmhd_gpu_ctx* c, SweepArgs<R>& a) {
+    a.stats = nullptr;
+    hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(kRecomputeBlocks), dim3(256), 0, c->stream, a);
+}
+
 // The sweeps of the axes in `mask`, one launch.  Reference rounding: the
-// sweeps with unscaled WENO divisions, then the IEEE-division launch for the
-// tiles they queued (it exits at once when there are none; no counting there).
+// sweeps with unscaled WENO divisions, then the launch for the tiles they
+// queued (SW_COLLECT: left to the caller, who waits for the sweep anyway).
 // One launch instead of one per axis: the last round of one axis's blocks,
 // the tail of its marches and its empty recompute launch cost 2% of the
 // sweeps at 256^3, and on a grid that leaves the chip idle the axes run side
@@ -154,8 +163,7 @@ void launch_sweep(howmhd_gpu_ctx* c, SweepArgs<R>& a, unsigned blocks) {
     if (blocks == 0) return;
     if constexpr (EX) {
         hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED>), dim3(blocks), dim3(256), 0, c->stream, a);
-        a.stats = nullptr;
-        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(kRecomputeBlocks), dim3(256), 0, c->stream, a);
+        if constexpr (MODE != SW_COLLECT) launch_recompute<R, MODE>(c, a);
     } else {
         hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(blocks), dim3(256), 0, c->stream, a);
     }

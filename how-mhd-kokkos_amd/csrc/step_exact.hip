@@ -13,6 +13,9 @@ namespace howmhd {
 
 int stage_fp64(howmhd_gpu_ctx* c, int iw, double dt) { return launch_stage<double>(c, iw, dt); }
 
+// Synchronises.  The sweep tells the host where it queued a tile, and the
+// IEEE-division launch runs only then: empty, it and the gap before it took 6 us
+// of a collection at 64^3 (55 -> 49 us) and 2 us at 30x20x25 (26.6 -> 24.9).
 int collect_fp64(howmhd_gpu_ctx* c, int dir, float* X, float* y, float* logits) {
     unsigned nb = 0;
     SweepArgs<double> a = sweep_args<double, SW_COLLECT>(c, 1, c->qbuf[c->qid[0]], 1u << dir, &nb);
@@ -20,8 +23,15 @@ int collect_fp64(howmhd_gpu_ctx* c, int dir, float* X, float* y, float* logits) 
     a.label = y;
     a.logit = logits;
     a.stats = nullptr;
+    *c->fixhost = 0u;
     launch_sweep<double, SW_COLLECT>(c, a, nb);
     HCHECK(c, hipGetLastError());
+    HCHECK(c, hipStreamSynchronize(c->stream));
+    if (*(volatile unsigned*)c->fixhost) {
+        launch_recompute<double, SW_COLLECT>(c, a);
+        HCHECK(c, hipGetLastError());
+        HCHECK(c, hipStreamSynchronize(c->stream));
+    }
     return HOWMHD_OK;
 }
 

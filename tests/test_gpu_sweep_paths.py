@@ -8,6 +8,9 @@ positive density, and one cell along x.  And a grid on each side of the rule.
 """
 import pytest
 
+import howmhd as H
+import mlp_oracle as M
+import oracle_ctypes as O
 import test_gpu_parity as P
 from test_gpu_launch_rules import _step_matches
 
@@ -42,3 +45,32 @@ def test_tiles_recompute(problem, kw, tiles, require_gpu):
                                   ((65, 17, 1), "open")])
 def test_split_rule(n, bc, require_gpu):
     _step_matches("mpi_smooth3d", n, bc, steps=2)
+
+
+@pytest.mark.parametrize("n,bc", [((16, 16, 16), "periodic"), ((33, 17, 15), "open")])
+def test_labels_beyond_the_unscaled_range(n, bc, require_gpu):
+    """Samples of a flow scaled as in the large-operand parity test, whose tiles
+    go through the IEEE-division launch, and of the flow itself afterwards on
+    the same solver, whose tiles do not: labels of both match the restatement."""
+    torch = pytest.importorskip("torch")
+    run = H.parse(H.make_input(problem="mhd_blast3d", nx=n[0], ny=n[1], nz=n[2], nt=1,
+                               tend=1.0, x1bc=bc, x2bc=bc, x3bc=bc))
+    p, q0 = H.gpu_params(run), H.init_problem(run)
+    big = q0.copy()
+    big[[0, 1, 2, 3, 7]] *= 1e50
+    big[[4, 5, 6]] *= 1e25
+    print(f"[sweep paths] labels {n} {bc}", flush=True)
+    with H.GpuSolver(p) as g:
+        for q, scaled in ((big, True), (q0, False), (big, True)):
+            g.upload_q0(q)
+            g.init_faces()
+            O.large_t_count(reset=True)
+            for d in range(3):
+                X = torch.empty((g.n_samples(d), H.MLP_NFEAT), dtype=torch.float32, device="cuda")
+                y = torch.empty(g.n_samples(d), dtype=torch.float32, device="cuda")
+                g.collect_samples(d, X, y)
+                lab, dev = M.interface_labels(H.active(g.q0()), d, p.bc[d] == H.BC["periodic"], p.gam, O.line_maxdev,
+                                              p.rhomin, p.pgmin)
+                clear = abs(dev - 0.05) > 1e-9
+                assert (y.cpu().numpy() == lab)[clear].all()
+            assert (O.large_t_count() > 0) == scaled
