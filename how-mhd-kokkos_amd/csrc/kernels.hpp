@@ -559,9 +559,11 @@ __device__ __forceinline__ void queue_tile(const SweepArgs<R>& A, long long slot
 }
 
 // Phase 2 of a tile whose cell values are in LDS: one interface per thread
-// (t0, a0, b0: the tile origin; slot: its tile slot).
-template <typename R, int TS, int MODE, int EX, int DM>
-__device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const SweepAxis<R>& X, const TileLds<R, TS>& L,
+// (t0, a0, b0: the tile origin; tslot: its tile slot).  In the unscaled mode
+// true for a thread with a WENO weight operand beyond the range; QUEUE: it also
+// queues the tile.
+template <typename R, int TS, int MODE, int EX, int DM, bool QUEUE>
+__device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const SweepAxis<R>& X, const TileLds<R, TS>& L,
                                                  int t0, int a0, int b0, long long tslot) {
     using T = SweepTile<TS>;
     const Geom& g = A.g;
@@ -624,16 +626,17 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
             if ((tid & 63) == 0) A.stats[4 * tslot + (tid >> 6)] = (unsigned)__popcll(fb) | (unsigned)__popcll(vb) << 8;
         }
     }
-    if (!valid) return;
+    if (!valid) return false;
 
+    bool out_of_range = false;
     R dF[7] = {R(0), R(0), R(0), R(0), R(0), R(0), R(0)};
     R maxdev = R(0);
     if (MODE != SW_ROUTED || flagged) {
         unsigned long long bad = 0ull;
         weno_interface<R, TS, MODE, DM>(luf, lo, row, lane, R(A.ph.gam), A.gc, dF, maxdev, bad);
-        // a WENO weight operand beyond the unscaled-division range
         if constexpr (EX && DM == DIV_UNSCALED) {
-            if (bad) queue_tile<R, MODE>(A, tslot);
+            out_of_range = bad != 0ull;
+            if (QUEUE && out_of_range) queue_tile<R, MODE>(A, tslot);
         }
     } else {
         // linear upwind-5 with one LLF speed: the largest |v_n| + c_f over the
@@ -690,7 +693,7 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
         st_nt(&X.ct_b[ci], dF[5] + ftmp2);
     }
     if constexpr (MODE == SW_COLLECT) {
-        if (!A.feat) return;
+        if (!A.feat) return out_of_range;
         float f[MLP_IN];
         features(f);
         const size_t si = sample();
@@ -698,13 +701,15 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
         for (int j = 0; j < MLP_IN; ++j) A.feat[si * MLP_IN + j] = f[j];
         A.label[si] = (maxdev > R(0.05)) ? 1.f : 0.f;
     }
+    return out_of_range;
 }
 
 // Up to `nsteps` consecutive tiles (bx, by0 ..) of plane bz along the sweep
 // axis (ALONG_X: one).  DM (DivMode) of the WENO weights: the FMA forms and
 // the reference-rounding recompute launch divide with IEEE divisions; the
-// reference-rounding sweep proper with div_recip/div_with, queueing its tile
-// for the recompute launch where an operand leaves their range.
+// reference-rounding sweep proper with div_recip/div_with; where an operand
+// leaves their range it queues its tile for the recompute launch, or (REDO) does
+// the tile again at once with IEEE divisions.
 //
 // Phase 1 puts the cell values of the tile (stencil halo included) into LDS,
 // phase 2 computes one interface per thread.  Consecutive y/z tiles share 5
@@ -712,11 +717,12 @@ __device__ __forceinline__ void sweep_interfaces(const SweepArgs<R>& A, const Sw
 // previous tile to rows 0..4 of the LDS tile and converts only its 8 new
 // rows, one cell per thread.  Every value is the one a single tile computes;
 // queueing and statistics use the tile's own slot.
-template <typename R, int TS, int MODE, int EX, int DM>
+template <typename R, int TS, int MODE, int EX, int DM, bool REDO = false>
 __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAxis<R>& X, unsigned char* raw, int bx,
                                             int by0, int bz, int nsteps) {
     using T = SweepTile<TS>;
-    constexpr bool MARCH = TS == ACROSS_X && sweep_marches<R, MODE>() && !(EX && DM == DIV_IEEE);
+    constexpr bool MARCH = TS == ACROSS_X && sweep_marches<R, MODE>() && !(EX && DM == DIV_IEEE) && !REDO;
+    static_assert(!REDO || (EX && DM == DIV_UNSCALED), "the unscaled mode redoes tiles");
     constexpr int HALO = 5 * T::LANES;        // slots of rows 0..4
     constexpr int NEW = T::CELLS - HALO;      // slots of rows 5..12
     constexpr int KEEP = T::ROWS * T::LANES;  // first slot of rows 8..12
@@ -732,7 +738,7 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
     auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * (by + (long long)gy * bz); };
     // a cell without positive shared reciprocals
     auto queue = [&](bool bad, long long slot) {
-        if constexpr (EX && DM == DIV_UNSCALED) {
+        if constexpr (EX && DM == DIV_UNSCALED && !REDO) {
             if (__ballot(bad)) queue_tile<R, MODE>(A, slot);
         }
     };
@@ -757,7 +763,11 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
             if (by + 1 < by1) load_new(t0 + T::ROWS);
         }
         __syncthreads();  // the tile's cells are in LDS
-        sweep_interfaces<R, TS, MODE, EX, DM>(A, X, L, t0, a0, bz, tile_slot(by));
+        const bool again = sweep_interfaces<R, TS, MODE, EX, DM, !REDO>(A, X, L, t0, a0, bz, tile_slot(by));
+        if constexpr (REDO) {
+            // (also the barrier between this pass's LDS reads and the next's writes)
+            if (__syncthreads_or(again || cell_bad)) sweep_tiles<R, TS, MODE, EX, DIV_IEEE>(A, X, raw, bx, by0, bz, 1);
+        }
     };
     {
         // A thread's cells are tid, tid + 256, ...; all their loads are
@@ -843,7 +853,8 @@ __device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X,
 // recompute launch (a few blocks) takes the tiles queued by the sweep proper
 // (A.fixlist, A.fixctl[0] of them), clears their flags, and the last block
 // to finish empties the queue; with an empty queue every block exits at once.
-template <typename R, int MODE, int EX, int DM>
+// REDO: single tiles that are redone in place; nothing is queued.
+template <typename R, int MODE, int EX, int DM, bool REDO = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves<R, MODE>()))) void k_sweep(
     SweepArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
@@ -874,7 +885,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
         if (b >= A.ax[2].first) {
             int bx, by, bz;
             xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by, bz);
-            sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, A.ax[2], raw, bx, by, bz, 1);
+            sweep_tiles<R, ALONG_X, MODE, EX, DM, REDO>(A, A.ax[2], raw, bx, by, bz, 1);
         } else {
             // The y and z sweeps are one code (strides) where it marches:
             // 31 KB an axis in FP64.  The single-tile forms have it once per
@@ -883,9 +894,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             auto across = [&](const SweepAxis<R>& X) {
                 const unsigned L = b - X.first, r = div(L, X.by_gx), bz = div(r, X.by_gy);
                 const int bx = (int)(L - r * X.gx), by = (int)(r - bz * X.by_gy.d);
-                sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by * X.march, (int)bz, X.march);
+                sweep_tiles<R, ACROSS_X, MODE, EX, DM, REDO>(A, X, raw, bx, by * X.march, (int)bz, X.march);
             };
-            if constexpr (sweep_marches<R, MODE>()) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
+            if constexpr (sweep_marches<R, MODE>() && !REDO) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
             else if (b >= A.ax[1].first) across(A.ax[1]);
             else across(A.ax[0]);
         }

@@ -70,23 +70,27 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
     return (int)std::min<unsigned long long>(cz, (unsigned long long)most);
 }
 
-// Whether the plain reference-rounding sweeps of a stage run as k_sweep_split:
-// while its blocks are at most two rounds of the 512 the chip holds.  A round
-// of it takes 7-8 us where a tile of k_sweep takes 13 us and its recompute
-// launch 4, however few there are.  Per step: shock tube 800 cells 123 -> 82
-// us, 60,000 cells (938 blocks) 193 -> 143; orszag_tang 32^2 143 -> 105, 128^2
-// (512 blocks) 149 -> 118, 160^2 (880) 156 -> 160; 3-D 16^3 198 -> 157, 20^3
-// (800) 198 -> 188; beyond, 24^3 (1,152) 227 -> 215 but 28^3 (1,568) 232 -> 254
-// and 32^3 230 -> 273.
-constexpr unsigned kSplitBlocks = 1024;
+// Whether the plain reference-rounding sweeps of a stage run as k_sweep_split.
+// With b blocks on a CU a stage of it takes about 4.6 b - 1 us, and one of
+// k_sweep, whose blocks have four times the interfaces, 6.4 b + 6.6 us; on a
+// line of cells a k_sweep block has no more than the other, and on thin grids
+// not many more.  Per step, k_sweep / split, us: orszag_tang 100^2 143 / 126,
+// 128^2 136 / 122, 144^2 138 / 147, 180^2 170 / 183; 3-D 16^3 186 / 166, 18^3
+// 190 / 185, 20^3 187 / 192, 24^3 212 / 214, 32^3 214 / 273; 60 x 200 218 / 180,
+// 8,192 x 3 237 / 205; lines of 800 cells 106 / 84, 100,000 279 / 189, 1,000,000
+// 1,867 / 1,259.
+constexpr unsigned kCUs = 256;
 inline bool split_sweep(const howmhd_gpu_ctx* c) {
     if (c->march_force > 0) return false;
-    unsigned long long n = 0;
+    unsigned long long ns = 0, nk = 0;
+    auto per_cu = [](unsigned long long n) { return (n + kCUs - 1) / kCUs; };
     for (int d = 0; d < 3; ++d) {
-        const dim3 t = sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d);
-        if (c->g.n[d] > 1) n += (unsigned long long)t.x * t.y * t.z;
+        if (c->g.n[d] == 1) continue;
+        const dim3 t = sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d), k = sweep_grid(c->g, d);
+        ns += (unsigned long long)t.x * t.y * t.z;
+        nk += (unsigned long long)k.x * k.y * k.z;
     }
-    return n <= kSplitBlocks;
+    return 46 * per_cu(ns) < 64 * per_cu(nk) + 71;
 }
 
 // Arguments of stage iw's sweeps of the axes in `mask` (bit d: axis d) from qsrc;
@@ -153,7 +157,12 @@ void launch_recompute(howmhd_gpu_ctx* c, SweepArgs<R>& a) {
 
 // The sweeps of the axes in `mask`, one launch.  Reference rounding: the
 // sweeps with unscaled WENO divisions, then the launch for the tiles they
-// queued (SW_COLLECT: left to the caller, who waits for the sweep anyway).
+// queued (SW_COLLECT: left to the caller, who waits for the sweep anyway).  Plain
+// sweeps of single tiles redo such a tile in place: no launch, which took 4 us
+// when empty (a step at 32^3 229 -> 213 us, 64^3 719 -> 700, 96^3 2,249 ->
+// 2,207), and no queue for a few blocks where many tiles are out of range (a
+// 512^2 run that ends in NaN 3.42 -> 0.74 ms).  The march and the routed sweep
+// have no registers for it (816 bytes of scratch a thread).
 // One launch instead of one per axis: the last round of one axis's blocks,
 // the tail of its marches and its empty recompute launch cost 2% of the
 // sweeps at 256^3, and on a grid that leaves the chip idle the axes run side
@@ -161,6 +170,12 @@ void launch_recompute(howmhd_gpu_ctx* c, SweepArgs<R>& a) {
 template <typename R, int MODE>
 void launch_sweep(howmhd_gpu_ctx* c, SweepArgs<R>& a, unsigned blocks) {
     if (blocks == 0) return;
+    if constexpr (EX && MODE == SW_PLAIN) {
+        if (a.ax[0].march == 1 && a.ax[1].march == 1) {
+            hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED, true>), dim3(blocks), dim3(256), 0, c->stream, a);
+            return;
+        }
+    }
     if constexpr (EX) {
         hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED>), dim3(blocks), dim3(256), 0, c->stream, a);
         if constexpr (MODE != SW_COLLECT) launch_recompute<R, MODE>(c, a);

@@ -1,7 +1,7 @@
 """The reference-rounding sweeps of the smallest grids run split over the
-wavefronts of a block, the others as tiles that may march and that queue tiles
-for an IEEE-division launch (needs a GPU).  Every parity case is small enough
-for the split sweep; here the same cases run on the other one
+wavefronts of a block, the others as single tiles (1) or as marches that queue
+tiles for an IEEE-division launch (2) (needs a GPU).  Every parity case is small
+enough for the split sweep; here the same cases run on the others
 (HOWMHD_SWEEP_MARCH), bit for bit against the CPU restatement: the case list,
 operands beyond the unscaled divisions, subnormal squares, a cell without
 positive density, and one cell along x.  And a grid on each side of the rule.
@@ -38,11 +38,13 @@ def test_tiles_recompute(problem, kw, tiles, require_gpu):
     P.test_fp64_bitwise_degenerate_x("mpi_smooth3d", dict(nx=1, ny=12, nz=10), require_gpu)
 
 
-# 1,024 blocks of the split sweep (the last grid it takes), 1,048 and 1,428;
-# interfaces that fill the 64 of a block and one more, last columns of 1 to 15
+# grids on both sides of the rule (512 blocks of the split sweep and one row
+# more), a line longer than 512 blocks, thin grids; interfaces that fill the 64
+# of a block and one more, last columns of 1 to 15
 @pytest.mark.parametrize("n,bc", [((256, 128, 1), "periodic"), ((256, 130, 1), "periodic"), ((65, 17, 17), "open"),
                                   ((64, 20, 18), "open"), ((63, 5, 3), "open"), ((64, 16, 1), "periodic"),
-                                  ((65, 17, 1), "open")])
+                                  ((65, 17, 1), "open"), ((128, 128, 1), "open"), ((128, 132, 1), "periodic"),
+                                  ((40001, 1, 1), "open"), ((4100, 3, 1), "periodic"), ((3, 1, 2050), "periodic")])
 def test_split_rule(n, bc, require_gpu):
     _step_matches("mpi_smooth3d", n, bc, steps=2)
 
