@@ -859,8 +859,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     SweepArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
     static_assert(EX || DM == DIV_IEEE, "the FMA forms divide with IEEE divisions");
-    __shared__ alignas(16) unsigned char raw[tile_lds_bytes<R, MODE, ACROSS_X>()];
-    static_assert(tile_lds_bytes<R, MODE, ALONG_X>() <= tile_lds_bytes<R, MODE, ACROSS_X>(), "LDS of both shapes");
+    extern __shared__ unsigned char raw[];  // a tile's values (sweep_lds)
     if constexpr (EX && DM == DIV_IEEE) {
         const unsigned n = A.fixctl[0];
         for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
