@@ -1,7 +1,8 @@
 // Learned smoothness indicator: an 18 -> 32 -> 32 -> 1 MLP (ReLU, ReLU,
-// sigmoid) evaluated with bf16 MFMA (v_mfma_f32_16x16x16_bf16, FP32
-// accumulation) by whole wavefronts: the 64 lanes of a wavefront are 64
-// interfaces (or training samples), split into four 16-row tiles.
+// sigmoid) evaluated with bf16 MFMA (FP32 accumulation) by whole wavefronts: in
+// the sweeps the 64 lanes are 64 interfaces, two tiles of 32
+// (v_mfma_f32_32x32x16_bf16, mlp_forward_wave); the kernels of indicator.hip
+// take tiles of 16 samples (v_mfma_f32_16x16x16_bf16).
 //
 // Inputs: the 6-cell stencils (the WENO5 stencil of the interface) of rho, p
 // and |B|, each mapped to [0,1] by its own min and max over the 6 cells.
