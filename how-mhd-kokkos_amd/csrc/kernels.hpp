@@ -8,18 +8,20 @@
 // is never stencilled by the time step).
 //
 // Per SSPRK stage iw the kernels are:
-//   k_sweep<X|Y|Z>  fused primit + eigensystem + characteristic LLF-WENO5:
-//                   interface fluxes dF (7 per interface) and CT flux terms
-//                   (src/ssprk.cpp:458-997, 1000-1272)
+//   k_sweep         fused primit + eigensystem + characteristic LLF-WENO5 of
+//                   every axis: interface fluxes dF (7 per interface) and CT
+//                   flux terms (src/ssprk.cpp:458-997, 1000-1272); the smallest
+//                   plain FP64 grids and lines take k_sweep_split
 //   k_emf_march     corner EMF build and smoothing (src/fluxct.cpp:809-840)
 //                   in one z-marching pass on 3-D grids; k_emf2, k_emf as two
-//                   passes on 1-D and 2-D grids
+//                   passes on x-z and y-z grids
 //   k_faces         face-B RK combination + 4th-order staggered curl
 //                   (src/fluxct.cpp:848-877, 111-135); k_faces_march, the
 //                   same marching through z on 3-D grids
 //   k_combine       stage combination k1*q_init + k3*q_prev + dX + dY + dZ,
 //                   face->centre B (src/fluxct.cpp:882-897) and the floors of
 //                   prot (src/prot.cpp:10-51)
+//   k_plane         on x-y grids, everything after the sweeps
 // Each kernel carries EX = HOWMHD_EXACT of the translation unit that
 // instantiates it (the plain FP64 unit: reference rounding; the FMA unit:
 // fp64fast and fp32), so the two units never share a kernel symbol.  The
@@ -477,7 +479,7 @@ __device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>:
 template <typename R, int MODE>
 constexpr int sweep_waves() { return (sizeof(R) == 4 && MODE != SW_COLLECT) ? HOWMHD_ROUTED_WAVES : HOWMHD_SWEEP_WAVES; }
 
-// y/z sweeps that march through consecutive tiles (sweep_march): the FP64
+// y/z sweeps that march through consecutive tiles (sweep_tiles): the FP64
 // ones but the collecting sweep.  The FP32 sweep at 4 waves per SIMD and the
 // collecting sweep have no registers for the march's state and would spill.
 template <typename R, int MODE>
@@ -902,15 +904,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     }
 }
 
-// The plain reference-rounding sweeps of a grid that leaves most of the chip
-// idle: a block has the 64 interfaces of one wavefront, and each of its four
+// The plain reference-rounding sweeps of a line or of a grid that leaves most of
+// the chip idle: a block has the 64 interfaces of one wavefront, and each of its four
 // wavefronts takes one projection pass ((0,6), (1,5), (2,4), (3)) of all of
 // them.  The products of the waves' fluxes with their columns of R meet in LDS
 // and are added in wave order, so every value is the one k_sweep computes.  A
 // tile with an operand out of the unscaled range is done again by the same
 // block with IEEE divisions: no recompute launch.  The eigensystem's scalars
-// are computed four times over, so this pays only while the chip has room
-// (split_sweep in stage.hpp).
+// are computed four times over, so this pays only while the chip has room, and on
+// lines, where a block of k_sweep has no more interfaces (split_sweep in stage.hpp).
 template <int EX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEEP_WAVES))) void k_sweep_split(
     SweepArgs<double> A) {

@@ -37,7 +37,7 @@ inline RK rk_coeff(int iw) {
 // Blocks of the IEEE-division recompute launch of the reference-rounding form.
 constexpr unsigned kRecomputeBlocks = 64;
 
-// Tiles a y/z-sweep block marches through (sweep_march): as many as keep at
+// Tiles a y/z-sweep block marches through (sweep_tiles): as many as keep at
 // least kMarchMinBlocks blocks in the launch, at most HOWMHD_MARCH_STEPS.
 #ifndef HOWMHD_MARCH_STEPS
 #define HOWMHD_MARCH_STEPS 8
