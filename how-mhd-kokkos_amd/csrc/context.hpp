@@ -77,6 +77,7 @@ struct howmhd_gpu_ctx {
     howmhd::MlpDev* mlp = nullptr;
     int ind_mode = 0;
     bool route_now = false;              // the running step routes
+    int xlanes = 64;  // interfaces per row of an x tile (x_lanes)
     unsigned* iwave = nullptr;
     long long nwave = 0;
     long long tile0[3] = {0, 0, 0};

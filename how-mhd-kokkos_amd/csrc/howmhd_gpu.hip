@@ -283,11 +283,12 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         if (ok) c->xfer_ev.push_back(ev);
     }
     small((void**)&c->mlp, sizeof(MlpDev));
+    c->xlanes = x_lanes(c->g);
     // one slot per tile of the sweeps (x, y, z), four counter words each
     for (int d = 0; d < 3; ++d) {
-        const dim3 gr = sweep_grid(c->g, d);
+        const dim3 gr = sweep_grid(c->g, d, 64, false);  // no packed grid has more
         c->tile0[d] = c->nwave / 4;
-        if (n[d] > 1) c->nwave += 4LL * gr.x * gr.y * gr.z;
+        if (n[d] > 1) c->nwave += 4LL * gr.x * gr.y;
     }
     c->nwave = std::max(c->nwave, 4LL);
     small((void**)&c->iwave, 5 * (size_t)c->nwave * sizeof(unsigned));

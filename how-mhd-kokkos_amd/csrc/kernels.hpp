@@ -11,7 +11,7 @@
 //   k_sweep         fused primit + eigensystem + characteristic LLF-WENO5 of
 //                   every axis: interface fluxes dF (7 per interface) and CT
 //                   flux terms (src/ssprk.cpp:458-997, 1000-1272); the smallest
-//                   plain FP64 grids and lines take k_sweep_split
+//                   plain FP64 grids take k_sweep_split
 //   k_emf_march     corner EMF build and smoothing (src/fluxct.cpp:809-840)
 //                   in one z-marching pass on 3-D grids; k_emf2, k_emf as two
 //                   passes on x-z and y-z grids
@@ -90,19 +90,30 @@ struct Phys {
 };
 
 // ------------------------------------------------------------- sweep tiling
-// Two tile shapes.  ALONG_X (x sweep): 64 interfaces along x per row, 4 rows
-// (y) per block.  ACROSS_X (y and z sweeps): HOWMHD_YZ_LANES x-columns,
-// 256/HOWMHD_YZ_LANES interfaces along the sweep axis per block.
+// Two tile shapes.  ALONG_X (x sweep): W interfaces along x of each of 256 / W
+// consecutive rows (lines of cells along x).  ACROSS_X (y and z sweeps):
+// HOWMHD_YZ_LANES consecutive columns (lines along the sweep axis, numbered x
+// fastest), 256/HOWMHD_YZ_LANES interfaces of each.  Packed, the rows and
+// columns are numbered through both transverse axes, so only the last tile has
+// idle ones, and W follows nx (x_lanes).  The routed sweeps are not packed: W is
+// 64, and the rows (columns) of each plane are filled up to whole tiles, because
+// their wavefronts are counted and decide about routing.
+//   Plain sweeps packed instead of filled up, a step, us: FP64 48^3 448 -> 411,
+// 72^3 1,310 -> 999, 80^3 1,534 -> 1,286, 97x75x61 1,391 -> 1,200, 112^3 3,416 -> 3,157,
+// 144^3 7,156 -> 6,425; FP32 265 -> 252, 629 -> 514, 732 -> 642, 679 -> 609, 1,599 ->
+// 1,505, 3,285 -> 3,036; 4x600x300 13,578 -> 3,591 and 5,068 -> 1,638; a line of 1,000,000
+// 1,254 -> 872 and 664 -> 501; where 64 and 32 divide the grid the index
+// arithmetic costs up to 0.5%.
 // The split sweep (k_sweep_split) gives a block the 64 interfaces of one
 // wavefront: ALONG_X_64 a row of 64, ACROSS_X_64 16 x-columns of 4.
 enum TileShape { ALONG_X = 0, ACROSS_X = 1, ALONG_X_64 = 2, ACROSS_X_64 = 3 };
 __host__ __device__ constexpr bool along_x(int ts) { return ts == ALONG_X || ts == ALONG_X_64; }
 template <int TS> struct SweepTile;
 template <> struct SweepTile<ALONG_X> {
-    static constexpr int LANES = 64, ROWS = 4, CELLS = (64 + 5) * 4;
+    static constexpr int THREADS = 256, MIN_W = 16, CELLS = 256 + 5 * (256 / MIN_W);  // rows of W + 5 cells
 };
 template <> struct SweepTile<ALONG_X_64> {
-    static constexpr int LANES = 64, ROWS = 1, CELLS = 64 + 5;
+    static constexpr int THREADS = 64, CELLS = 64 + 5;
 };
 template <> struct SweepTile<ACROSS_X_64> {
     static constexpr int LANES = 16, ROWS = 4, CELLS = 16 * (4 + 5);
@@ -130,15 +141,48 @@ template <> struct SweepTile<ACROSS_X> {
 
 __host__ __device__ inline unsigned blocks_for(size_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// Tiles of the sweep along axis d: (x tiles, tiles along the second axis,
-// planes), in the shapes SX along x and SA across it.
-template <int SX = ALONG_X, int SA = ACROSS_X>
-__host__ __device__ inline dim3 sweep_grid(const Geom& g, int d) {
-    const int nif = g.per[d] ? g.n[d] : g.n[d] + 1;
-    using X = SweepTile<SX>;
-    using T = SweepTile<SA>;
-    if (d == 0) return dim3(blocks_for(nif, X::LANES), blocks_for(g.n[1], X::ROWS), g.n[2]);
-    return dim3(blocks_for(g.n[0], T::LANES), blocks_for(nif, T::ROWS), d == 1 ? g.n[2] : g.n[1]);
+// Interfaces per row of a packed x tile (W): the fewest tiles, 64 a row where
+// that is within 3% of them.
+inline int x_lanes(const Geom& g) {
+    using X = SweepTile<ALONG_X>;
+    const unsigned nif = g.per[0] ? g.n[0] : g.n[0] + 1;
+    const size_t nrow = (size_t)(g.ncell / g.n[0]);
+    auto tiles = [&](unsigned w) { return (double)blocks_for(nif, w) * blocks_for(nrow, X::THREADS / w); };
+    unsigned best = 64;
+    for (unsigned w = X::THREADS; w >= X::MIN_W; --w)
+        if (tiles(w) < 0.97 * tiles(64) && tiles(w) < tiles(best)) best = w;
+    // the same tiles with the shortest even segments
+    return (int)std::max<unsigned>(blocks_for(nif, blocks_for(nif, best)), X::MIN_W);
+}
+
+// Rows (columns) of the sweep along axis d as the tiles number them: `in` of
+// each of the `out` planes, `period` from plane to plane, in tiles of `per_tile`.
+struct Lines {
+    size_t in, out, period;
+};
+inline Lines sweep_lines(const Geom& g, int d, bool packed, unsigned per_tile) {
+    const size_t ncol = (size_t)(g.ncell / g.n[d]);
+    if (packed && d != 1) return {ncol, 1, ncol};  // contiguous
+    const size_t in = d == 0 ? g.n[1] : g.n[0];
+    return {in, ncol / in, packed ? in : (size_t)blocks_for(in, per_tile) * per_tile};
+}
+
+// Tiles of the sweep along axis d (W: of the x tiles): (tiles along x, groups
+// of rows) or (groups of columns, tiles along the axis).  split_grid: those of
+// k_sweep_split.
+inline dim3 sweep_grid(const Geom& g, int d, int W, bool packed) {
+    using T = SweepTile<ACROSS_X>;
+    const size_t nif = g.per[d] ? g.n[d] : g.n[d] + 1;
+    const unsigned per_tile = d == 0 ? SweepTile<ALONG_X>::THREADS / W : T::LANES;
+    const Lines l = sweep_lines(g, d, packed, per_tile);
+    const unsigned groups = blocks_for(l.period * l.out, per_tile);
+    return d == 0 ? dim3(blocks_for(nif, W), groups) : dim3(groups, blocks_for(nif, T::ROWS));
+}
+inline dim3 split_grid(const Geom& g, int d) {
+    using T = SweepTile<ACROSS_X_64>;
+    const size_t nif = g.per[d] ? g.n[d] : g.n[d] + 1, ncol = (size_t)(g.ncell / g.n[d]);
+    if (d == 0) return dim3(blocks_for(nif, SweepTile<ALONG_X_64>::THREADS), (unsigned)ncol);
+    return dim3(blocks_for(ncol, T::LANES), blocks_for(nif, T::ROWS));
 }
 
 // Sweep variants: plain characteristic WENO5; the same plus indicator
@@ -166,23 +210,31 @@ __host__ __device__ __forceinline__ unsigned div(unsigned n, const LaunchDiv& v)
 
 // What one axis of a launch needs: its arrays, the strides that make the y
 // and z sweeps one code (cells, interfaces t = 0..n of dF and samples lie on
-// lines along the sweep axis; `other` is the axis that is neither x nor the
-// sweep axis), and its place in the launch.
+// lines along the sweep axis: line c of the tiles is line x = c - o period of
+// plane o, sweep_lines), and its place in the launch.
 template <typename R>
 struct SweepAxis {
     R* dF;              // 7 components, cF apart
     R* ct_a;            // CT term "bsy": fsy (x), gsz (y), hsx (z)
     R* ct_b;            // CT term "bsz": fsz (x), gsx (y), hsy (z)
     long long qoff[8];  // offset of the variable in sweep slot m (sweep_perm)
-    int n, per, nother; // cells along the axis; periodic; cells of `other`
+    int n, per;         // cells along the axis; periodic
+    int in, nc;         // lines of a plane, and of all (planes x period)
     // cell and interface indices fit 32 bits: a context of 2^32 / 2 cells
     // would need more than four times the 288 GB of the device
-    unsigned sA, sB;    // cell strides along the axis and along `other`
-    unsigned tF, oF;    // dF strides: interface, other (components: cF)
+    unsigned sA, sB;    // cell index of a column: x + o sB + along sA
+    unsigned tF, oF;    // dF index: x + o oF + t tF (components: cF apart)
     long long cF;
-    unsigned sS, oS;    // sample strides: interface, other
-    unsigned gx, gy, gz;   // tiles (sweep_grid)
-    LaunchDiv by_gx, by_gy; // by gx, and by the blocks along gy
+    unsigned sS, oS;    // sample index: x + o oS + u sS
+    unsigned rows_o;    // x: rows from plane to plane (row x + o rows_o)
+    LaunchDiv by_o;     // c -> o: by the period
+    int W, rows;        // x: interfaces per row and rows of a tile
+    LaunchDiv by_w, by_w5;  // by W and W + 5
+    unsigned gx, gy;    // tiles (sweep_grid)
+    LaunchDiv by_gx;
+    // y and z: a plane's tiles, then the blocks along the axis, then the next
+    // plane's, so that tiles that share halos along the axis run close in time
+    LaunchDiv by_chunk, by_blocks;
     unsigned first;     // first block of the launch on this axis
     int march;          // consecutive tiles along the axis per block
     long long tile0;    // first tile slot of the axis (queue, statistics)
@@ -283,17 +335,40 @@ __device__ __forceinline__ void opaque(Eig<R>& o) {
     opq(o.sqrtrho); opq(o.invsqrtrho); opq(o.nrm_half); opq(o.nrm_ent);
 }
 
-// LDS slot of stencil cell k = 0..5 of the interface of phase-2 thread (row,
-// lane).
+// LDS slot of stencil cell k = 0..5 of the interface whose cell 0 is in slot s0.
 template <int TS>
-__device__ __forceinline__ int stencil_slot(int row, int lane, int k) {
-    using T = SweepTile<TS>;
-    if constexpr (along_x(TS)) return row * (T::LANES + 5) + lane + k;
-    else return (row + k) * T::LANES + lane;
+__device__ __forceinline__ int stencil_slot(int s0, int k) {
+    if constexpr (along_x(TS)) return s0 + k;
+    else return s0 + k * SweepTile<TS>::LANES;
 }
 
-// Characteristic LLF-WENO5 flux of the interface of phase-2 thread (row,
-// lane) from the sweep tile in LDS (src/ssprk.cpp:825-946): interface
+// Phase-2 thread `tid` of a tile: its interface and row along x, or its
+// interface along the axis and column; the slot of its stencil's cell 0.
+struct TileLane {
+    int lane, row, s0;
+    bool used;
+};
+template <typename R, int TS>
+__device__ __forceinline__ TileLane tile_lane(const SweepAxis<R>& X, int tid) {
+    using T = SweepTile<TS>;
+    if constexpr (TS == ALONG_X_64) {
+        return {tid, 0, tid, true};
+    } else if constexpr (TS == ALONG_X) {
+        const int row = (int)div((unsigned)tid, X.by_w), lane = tid - row * X.W;
+        return {lane, row, row * (X.W + 5) + lane, row < X.rows};
+    } else {
+        return {tid % T::LANES, tid / T::LANES, tid, true};
+    }
+}
+// Cells of a tile.
+template <typename R, int TS>
+__device__ __forceinline__ int tile_cells(const SweepAxis<R>& X) {
+    if constexpr (TS == ALONG_X) return X.rows * (X.W + 5);
+    else return SweepTile<TS>::CELLS;
+}
+
+// Characteristic LLF-WENO5 flux of the interface whose stencil starts in
+// slot cell0 of the sweep tile in LDS (src/ssprk.cpp:825-946): interface
 // eigensystem, the 7 wave maxima, then the waves in pairs, added to dFo in
 // wave order.  The WENO weights divide in mode DM (DivMode); `bad` collects
 // the lanes whose operands left the range of the unscaled division.
@@ -301,11 +376,11 @@ __device__ __forceinline__ int stencil_slot(int row, int lane, int k) {
 // R go to prod[(wave * 7 + component) * 64] instead of into dFo.
 template <typename R, int TS, int MODE, int DM, int ONLY = -1>
 __device__ __forceinline__ void weno_interface(const UF<R> (*luf)[SweepTile<TS>::CELLS],
-                                               const R (*lo)[SweepTile<TS>::CELLS], int row, int lane, R gam,
+                                               const R (*lo)[SweepTile<TS>::CELLS], int cell0, R gam,
                                                const GasConst& gc, R (&dFo)[7], R& mdev, unsigned long long& bad,
                                                R* prod = nullptr) {
     (void)mdev;
-    auto slot = [&](int k) -> int { return stencil_slot<TS>(row, lane, k); };
+    auto slot = [&](int k) -> int { return stencil_slot<TS>(cell0, k); };
     // interface state from cells k = 2, 3: (rho, vn, vt1, vt2, Bn, Bt1, Bt2, p, H)
     R u0[9], u1[9];
     {
@@ -485,34 +560,63 @@ constexpr int sweep_waves() { return (sizeof(R) == 4 && MODE != SW_COLLECT) ? HO
 template <typename R, int MODE>
 constexpr bool sweep_marches() { return sizeof(R) == 8 && MODE != SW_COLLECT; }
 
+// Line c of the tiles: x of plane o; `real` unless it only fills a tile.
+struct TileLine {
+    unsigned x, o;
+    bool real;
+};
+template <typename R>
+__device__ __forceinline__ TileLine tile_line(const SweepAxis<R>& X, int c) {
+    const unsigned o = div((unsigned)c, X.by_o), x = c - o * X.by_o.d;
+    return {x, o, c < X.nc && x < (unsigned)X.in};
+}
+
 // Stored index of slot s of the LDS tile whose first interface is t0 (the
-// tile's cells run from t0 - 3 to t0 + ROWS + 1 along the sweep axis, x
-// sweep: t0 - 3 to t0 + LANES + 1), through the boundary map.  (x0, o0):
-// first column and other coordinate (ACROSS_X); (y0, z0) of the rows
-// (ALONG_X).
+// tile's cells run from t0 - 3 to 1 beyond its last interface along the sweep
+// axis) and whose first line is a0, through the boundary map.  A line that
+// only fills the tile reads the last one.
 template <typename R, int TS>
-__device__ __forceinline__ unsigned tile_cell_index(const Geom& g, const SweepAxis<R>& X, int s, int t0, int a0,
-                                                     int b0) {
+__device__ __forceinline__ unsigned tile_cell_index(const SweepAxis<R>& X, int s, int t0, int a0) {
     using T = SweepTile<TS>;
-    int along;
-    unsigned base;
-    if constexpr (along_x(TS)) {
-        const int row = s / (T::LANES + 5), c = s % (T::LANES + 5);
-        along = t0 - 3 + c;
-        int cy = a0 + row;
-        if (cy >= g.n[1]) cy = g.n[1] - 1;
-        base = ((unsigned)b0 * g.n[1] + cy) * (unsigned)g.n[0];
+    int along, c;
+    if constexpr (TS == ALONG_X_64) {
+        along = t0 - 3 + s;
+        c = a0;
+    } else if constexpr (TS == ALONG_X) {
+        const int row = (int)div((unsigned)s, X.by_w5);
+        along = t0 - 3 + (s - row * (X.W + 5));
+        c = a0 + row;
     } else {
-        const int row = s / T::LANES, lane = s % T::LANES;
-        along = t0 - 3 + row;
-        int cx = a0 + lane;
-        if (cx >= g.n[0]) cx = g.n[0] - 1;
-        base = cx + (unsigned)b0 * X.sB;
+        along = t0 - 3 + s / T::LANES;
+        c = a0 + s % T::LANES;
     }
+    const TileLine l = tile_line(X, min(c, X.nc - 1));
+    const unsigned x = min(l.x, (unsigned)X.in - 1);
     if (along > X.n + 2) along = X.n + 2;
-    const int a = bmap(along, X.n, X.per);
-    if constexpr (along_x(TS)) return base + a;
-    else return base + (unsigned)a * X.sA;
+    const unsigned a = bmap(along, X.n, X.per);
+    if constexpr (along_x(TS)) return (x + l.o * X.rows_o) * (unsigned)X.n + a;
+    else return x + l.o * X.sB + a * X.sA;
+}
+
+// Where the interface t of line l goes: dF, CT term (of the cell left of it)
+// and sample.
+template <typename R, int TS>
+__device__ __forceinline__ void interface_index(const SweepAxis<R>& X, int t, const TileLine& l, unsigned& fi,
+                                                unsigned& ci) {
+    if constexpr (along_x(TS)) {
+        const unsigned r = l.x + l.o * X.rows_o;
+        fi = r * (X.n + 1) + t;
+        ci = r * X.n + (t - 1);
+    } else {
+        fi = l.x + l.o * X.oF + t * X.tF;
+        ci = l.x + l.o * X.sB + (unsigned)(t - 1) * X.sA;
+    }
+}
+template <typename R, int TS>
+__device__ __forceinline__ unsigned sample_index(const SweepAxis<R>& X, int t, const TileLine& l) {
+    const unsigned u = t - (X.per ? 1 : 0);
+    if constexpr (along_x(TS)) return (l.x + l.o * X.rows_o) * X.sS + u;
+    else return l.x + l.o * X.oS + u * X.sS;
 }
 
 // The LDS of a tile: (U_j, F_j) pairs, the other cell fields, and |B| of each
@@ -561,15 +665,13 @@ __device__ __forceinline__ void queue_tile(const SweepArgs<R>& A, long long slot
 }
 
 // Phase 2 of a tile whose cell values are in LDS: one interface per thread
-// (t0, a0, b0: the tile origin; tslot: its tile slot).  In the unscaled mode
+// (t0, a0: the tile origin; tslot: its tile slot).  In the unscaled mode
 // true for a thread with a WENO weight operand beyond the range; QUEUE: it also
 // queues the tile.
 template <typename R, int TS, int MODE, int EX, int DM, bool QUEUE>
 __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const SweepAxis<R>& X, const TileLds<R, TS>& L,
-                                                 int t0, int a0, int b0, long long tslot) {
+                                                 int t0, int a0, long long tslot) {
     using T = SweepTile<TS>;
-    const Geom& g = A.g;
-    const int nd = X.n;
     // opaque, so that a march computes its addresses in every step instead of
     // holding them in registers across the interfaces
     int tid = threadIdx.x;
@@ -577,26 +679,13 @@ __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const Sw
     const auto luf = const_cast<const UF<R>(*)[T::CELLS]>(L.luf);
     const auto lo = const_cast<const R(*)[T::CELLS]>(L.lo);
     const float* lbmag = L.lbmag;
-    const int lane = tid % T::LANES, row = tid / T::LANES;
-    int t, x, o;  // interface; ALONG_X: (y, z) = (x, o), ACROSS_X: column and other coordinate
-    bool valid;
-    if constexpr (along_x(TS)) {
-        t = t0 + lane; x = a0 + row; o = b0;
-        valid = (t <= nd && x < g.n[1]);
-    } else {
-        t = t0 + row; x = a0 + lane; o = b0;
-        valid = (t <= nd && x < g.n[0]);
-    }
-    auto slot = [&](int k) -> int {
-        if constexpr (along_x(TS)) return row * (T::LANES + 5) + lane + k;
-        else return (row + k) * T::LANES + lane;
-    };
-    // index of interface u = t - tbeg among the samples
-    auto sample = [&]() -> unsigned {
-        const unsigned u = t - (X.per ? 1 : 0);
-        if constexpr (along_x(TS)) return ((unsigned)o * g.n[1] + x) * X.oS + u;
-        else return u * X.sS + (unsigned)o * X.oS + x;
-    };
+    const TileLane tl = tile_lane<R, TS>(X, tid);
+    const int t = t0 + (along_x(TS) ? tl.lane : tl.row);
+    const TileLine line = tile_line(X, a0 + (along_x(TS) ? tl.row : tl.lane));
+    const bool valid = tl.used && t <= X.n && line.real;
+    auto slot = [&](int k) -> int { return stencil_slot<TS>(tl.s0, k); };
+    // index of the interface among the samples
+    auto sample = [&]() -> unsigned { return sample_index<R, TS>(X, t, line); };
     // indicator features: the 6-cell stencils of rho, p and |B|
     auto features = [&](float* f) {
         float rr[6], pp[6], bb[6];
@@ -635,7 +724,7 @@ __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const Sw
     R maxdev = R(0);
     if (MODE != SW_ROUTED || flagged) {
         unsigned long long bad = 0ull;
-        weno_interface<R, TS, MODE, DM>(luf, lo, row, lane, R(A.ph.gam), A.gc, dF, maxdev, bad);
+        weno_interface<R, TS, MODE, DM>(luf, lo, tl.s0, R(A.ph.gam), A.gc, dF, maxdev, bad);
         if constexpr (EX && DM == DIV_UNSCALED) {
             out_of_range = bad != 0ull;
             if (QUEUE && out_of_range) queue_tile<R, MODE>(A, tslot);
@@ -664,14 +753,7 @@ __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const Sw
 
     // dF and (below) the CT terms of the cell left of the interface
     unsigned fi, ci;
-    if constexpr (along_x(TS)) {
-        const unsigned r = (unsigned)o * g.n[1] + x;
-        fi = r * (nd + 1) + t;
-        ci = r * nd + (t - 1);
-    } else {
-        fi = (unsigned)o * X.oF + t * X.tF + x;
-        ci = (unsigned)o * X.sB + (unsigned)(t - 1) * X.sA + x;
-    }
+    interface_index<R, TS>(X, t, line, fi, ci);
 #pragma unroll
     for (int c = 0; c < 7; ++c)
         if (!(A.ct_active && (c == 4 || c == 5))) st_nt(&X.dF[c * X.cF + fi], dF[c]);
@@ -706,8 +788,8 @@ __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const Sw
     return out_of_range;
 }
 
-// Up to `nsteps` consecutive tiles (bx, by0 ..) of plane bz along the sweep
-// axis (ALONG_X: one).  DM (DivMode) of the WENO weights: the FMA forms and
+// Up to `nsteps` consecutive tiles (bx, by0 ..) along the sweep axis (ALONG_X:
+// one).  DM (DivMode) of the WENO weights: the FMA forms and
 // the reference-rounding recompute launch divide with IEEE divisions; the
 // reference-rounding sweep proper with div_recip/div_with; where an operand
 // leaves their range it queues its tile for the recompute launch, or (REDO) does
@@ -721,23 +803,28 @@ __device__ __forceinline__ bool sweep_interfaces(const SweepArgs<R>& A, const Sw
 // queueing and statistics use the tile's own slot.
 template <typename R, int TS, int MODE, int EX, int DM, bool REDO = false>
 __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAxis<R>& X, unsigned char* raw, int bx,
-                                            int by0, int bz, int nsteps) {
+                                            int by0, int nsteps) {
     using T = SweepTile<TS>;
     constexpr bool MARCH = TS == ACROSS_X && sweep_marches<R, MODE>() && !(EX && DM == DIV_IEEE) && !REDO;
     static_assert(!REDO || (EX && DM == DIV_UNSCALED), "the unscaled mode redoes tiles");
-    constexpr int HALO = 5 * T::LANES;        // slots of rows 0..4
-    constexpr int NEW = T::CELLS - HALO;      // slots of rows 5..12
-    constexpr int KEEP = T::ROWS * T::LANES;  // first slot of rows 8..12
-    static_assert(!MARCH || (NEW == 256 && KEEP + HALO == T::CELLS), "one new cell per thread");
+    // the march's slots: rows 0..4, first slot of rows 8..12; one new cell per
+    // thread in rows 5..12
+    using M = SweepTile<ACROSS_X>;
+    constexpr int HALO = 5 * M::LANES, KEEP = M::ROWS * M::LANES;
+    static_assert(M::CELLS - HALO == 256 && KEEP + HALO == M::CELLS, "one new cell per thread");
     const TileLds<R, TS> L = tile_lds<R, TS>(raw);
-    const Geom& g = A.g;
     const int tbeg = X.per ? 1 : 0;  // periodic: interface 0 is the image of n
     const int tid = threadIdx.x;
     const int gy = (int)X.gy;
-    // tile origin: first interface, first column (ALONG_X: first row y), plane
-    auto first_if = [&](int by) { return tbeg + (along_x(TS) ? bx * T::LANES : by * T::ROWS); };
-    const int a0 = along_x(TS) ? by0 * T::ROWS : bx * T::LANES;
-    auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * (by + (long long)gy * bz); };
+    // tile origin: first interface, first column (ALONG_X: row)
+    auto first_if = [&](int by) {
+        if constexpr (along_x(TS)) return tbeg + bx * X.W;
+        else return tbeg + by * T::ROWS;
+    };
+    int a0;
+    if constexpr (along_x(TS)) a0 = by0 * X.rows;
+    else a0 = bx * T::LANES;
+    auto tile_slot = [&](int by) { return X.tile0 + bx + (long long)X.gx * by; };
     // a cell without positive shared reciprocals
     auto queue = [&](bool bad, long long slot) {
         if constexpr (EX && DM == DIV_UNSCALED && !REDO) {
@@ -753,7 +840,7 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
     bool bad_prev = false;   // this thread converted a cell out of range in the previous step
     const int by1 = MARCH ? min(by0 + nsteps, gy) : by0 + 1;
     auto load_new = [&](int t0) {  // the new cell of the tile starting at row t0
-        const unsigned idx = tile_cell_index<R, TS>(g, X, HALO + tid, t0, a0, bz);
+        const unsigned idx = tile_cell_index<R, TS>(X, HALO + tid, t0, a0);
 #pragma unroll
         for (int m = 0; m < 8; ++m) qn[m] = A.q[X.qoff[m] + idx];
     };
@@ -762,13 +849,13 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
         queue(cell_bad || bad_prev, tile_slot(by));
         bad_prev = cell_bad;
         if constexpr (EARLY) {
-            if (by + 1 < by1) load_new(t0 + T::ROWS);
+            if (by + 1 < by1) load_new(t0 + M::ROWS);
         }
         __syncthreads();  // the tile's cells are in LDS
-        const bool again = sweep_interfaces<R, TS, MODE, EX, DM, !REDO>(A, X, L, t0, a0, bz, tile_slot(by));
+        const bool again = sweep_interfaces<R, TS, MODE, EX, DM, !REDO>(A, X, L, t0, a0, tile_slot(by));
         if constexpr (REDO) {
             // (also the barrier between this pass's LDS reads and the next's writes)
-            if (__syncthreads_or(again || cell_bad)) sweep_tiles<R, TS, MODE, EX, DIV_IEEE>(A, X, raw, bx, by0, bz, 1);
+            if (__syncthreads_or(again || cell_bad)) sweep_tiles<R, TS, MODE, EX, DIV_IEEE>(A, X, raw, bx, by0, 1);
         }
     };
     {
@@ -777,11 +864,12 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
         constexpr int NIT = (T::CELLS + 255) / 256;
         double qs[NIT][8];
         bool cell_bad = false;
+        const int ncells = tile_cells<R, TS>(X);
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
             const int s = tid + 256 * it;
-            if (s < T::CELLS) {
-                const unsigned idx = tile_cell_index<R, TS>(g, X, s, first_if(by0), a0, bz);
+            if (s < ncells) {
+                const unsigned idx = tile_cell_index<R, TS>(X, s, first_if(by0), a0);
 #pragma unroll
                 for (int m = 0; m < 8; ++m) qs[it][m] = A.q[X.qoff[m] + idx];
             }
@@ -789,7 +877,7 @@ __device__ __forceinline__ void sweep_tiles(const SweepArgs<R>& A, const SweepAx
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
             const int s = tid + 256 * it;
-            if (s < T::CELLS) store_cell<R, TS, MODE, DM>(A, L, s, qs[it], cell_bad);
+            if (s < ncells) store_cell<R, TS, MODE, DM>(A, L, s, qs[it], cell_bad);
         }
         finish(by0, cell_bad);
     }
@@ -832,12 +920,12 @@ struct CtFlags {
 // the 3-cell stencil halo that it shares with its neighbours (1.5x the row's
 // bytes).  Here workgroups L and L + 8 (the same XCD, dispatched one after
 // the other) take neighbouring x-tiles of one row; rows beyond the last full
-// group of 8 keep the launch order.  A bijection on the gx x gy x gz tiles.
+// group of 8 keep the launch order.  A bijection on the gx x gy tiles.
 template <typename R>
-__device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X, int& bx, int& by, int& bz) {
-    const unsigned gx = X.gx, nrow = X.gy * X.gz;
+__device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X, int& bx, int& by) {
+    const unsigned gx = X.gx;
     unsigned row;
-    if (gx == 1 || L >= (nrow / 8) * 8 * gx) {
+    if (gx == 1 || L >= (X.gy / 8) * 8 * gx) {
         row = div(L, X.by_gx);
         bx = (int)(L - row * gx);
     } else {
@@ -845,8 +933,7 @@ __device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X,
         row = r * 8 + L % 8;
         bx = (int)(a - r * gx);
     }
-    bz = (int)div(row, X.by_gy);
-    by = (int)(row - bz * X.gy);
+    by = (int)row;
 }
 
 // The sweeps of one launch: the blocks of the y axis, of the z axis (marching
@@ -871,9 +958,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             const int k = slot < A.ax[0].tile0 ? 2 : slot < A.ax[1].tile0 ? 0 : 1;
             const SweepAxis<R>& X = A.ax[k];
             const unsigned b = slot - (unsigned)X.tile0;
-            const int bx = (int)(b % X.gx), by = (int)((b / X.gx) % X.gy), bz = (int)(b / (X.gx * X.gy));
-            if (k == 2) sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, X, raw, bx, by, bz, 1);
-            else sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by, bz, 1);
+            const int bx = (int)(b % X.gx), by = (int)(b / X.gx);
+            if (k == 2) sweep_tiles<R, ALONG_X, MODE, EX, DM>(A, X, raw, bx, by, 1);
+            else sweep_tiles<R, ACROSS_X, MODE, EX, DM>(A, X, raw, bx, by, 1);
             if (threadIdx.x == 0) A.fix[slot] = 0u;
         }
         __syncthreads();  // every thread of the block has read the count
@@ -884,18 +971,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     } else {
         const unsigned b = blockIdx.x;
         if (b >= A.ax[2].first) {
-            int bx, by, bz;
-            xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by, bz);
-            sweep_tiles<R, ALONG_X, MODE, EX, DM, REDO>(A, A.ax[2], raw, bx, by, bz, 1);
+            int bx, by;
+            xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by);
+            sweep_tiles<R, ALONG_X, MODE, EX, DM, REDO>(A, A.ax[2], raw, bx, by, 1);
         } else {
             // The y and z sweeps are one code (strides) where it marches:
             // 31 KB an axis in FP64.  The single-tile forms have it once per
             // axis: their constants then come straight from the kernel
             // arguments (routed FP32 y/z sweeps at 256^3 444/459 -> 429/445 us).
             auto across = [&](const SweepAxis<R>& X) {
-                const unsigned L = b - X.first, r = div(L, X.by_gx), bz = div(r, X.by_gy);
-                const int bx = (int)(L - r * X.gx), by = (int)(r - bz * X.by_gy.d);
-                sweep_tiles<R, ACROSS_X, MODE, EX, DM, REDO>(A, X, raw, bx, by * X.march, (int)bz, X.march);
+                const unsigned L = b - X.first, r = div(L, X.by_chunk), hi = div(r, X.by_blocks);
+                const unsigned bx = hi * X.by_chunk.d + (L - r * X.by_chunk.d), by = r - hi * X.by_blocks.d;
+                if (bx >= X.gx) return;  // the last chunk is short
+                sweep_tiles<R, ACROSS_X, MODE, EX, DM, REDO>(A, X, raw, (int)bx, (int)by * X.march, X.march);
             };
             if constexpr (sweep_marches<R, MODE>() && !REDO) across(A.ax[b >= A.ax[1].first ? 1 : 0]);
             else if (b >= A.ax[1].first) across(A.ax[1]);
@@ -904,15 +992,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     }
 }
 
-// The plain reference-rounding sweeps of a line or of a grid that leaves most of
-// the chip idle: a block has the 64 interfaces of one wavefront, and each of its four
+// The plain reference-rounding sweeps of a grid that leaves most of the chip
+// idle: a block has the 64 interfaces of one wavefront, and each of its four
 // wavefronts takes one projection pass ((0,6), (1,5), (2,4), (3)) of all of
 // them.  The products of the waves' fluxes with their columns of R meet in LDS
 // and are added in wave order, so every value is the one k_sweep computes.  A
 // tile with an operand out of the unscaled range is done again by the same
 // block with IEEE divisions: no recompute launch.  The eigensystem's scalars
-// are computed four times over, so this pays only while the chip has room, and on
-// lines, where a block of k_sweep has no more interfaces (split_sweep in stage.hpp).
+// are computed four times over, so this pays only while the chip has room
+// (split_sweep in stage.hpp).
 template <int EX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEEP_WAVES))) void k_sweep_split(
     SweepArgs<double> A) {
@@ -925,18 +1013,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
     auto tile = [&](auto tsc, const SweepAxis<R>& X) {
         constexpr int TS = decltype(tsc)::value;
         using T = SweepTile<TS>;
-        const unsigned L = blockIdx.x - X.first, rr = div(L, X.by_gx), uz = div(rr, X.by_gy);
-        const int bx = (int)(L - rr * X.gx), by = (int)(rr - uz * X.gy), bz = (int)uz;
+        const unsigned L = blockIdx.x - X.first, rr = div(L, X.by_gx);
+        const int bx = (int)(L - rr * X.gx), by = (int)rr;
         const TileLds<R, TS> lds = tile_lds<R, TS>(raw);
         const int tid = threadIdx.x, l = tid & 63, pass = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int t0 = (X.per ? 1 : 0) + (along_x(TS) ? bx * T::LANES : by * T::ROWS);
-        const int a0 = along_x(TS) ? by * T::ROWS : bx * T::LANES;
-        const int lane = l % T::LANES, row = l / T::LANES;
-        const int t = along_x(TS) ? t0 + lane : t0 + row, x = along_x(TS) ? a0 + row : a0 + lane;
-        const bool valid = t <= X.n && x < A.g.n[along_x(TS) ? 1 : 0];
+        int t0 = X.per ? 1 : 0, a0;
+        if constexpr (along_x(TS)) { t0 += bx * T::THREADS; a0 = by; }
+        else { t0 += by * T::ROWS; a0 = bx * T::LANES; }
+        const TileLane tl = tile_lane<R, TS>(X, l);
+        const int t = t0 + (along_x(TS) ? tl.lane : tl.row);
+        const TileLine line = tile_line(X, a0 + (along_x(TS) ? tl.row : tl.lane));
+        const bool valid = t <= X.n && line.real;
         double q[8];
         if (tid < T::CELLS) {
-            const unsigned idx = tile_cell_index<R, TS>(A.g, X, tid, t0, a0, bz);
+            const unsigned idx = tile_cell_index<R, TS>(X, tid, t0, a0);
 #pragma unroll
             for (int m = 0; m < 8; ++m) q[m] = A.q[X.qoff[m] + idx];
         }
@@ -950,8 +1040,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
                 R none[7], dev;
                 auto one = [&](auto pc) {
                     weno_interface<R, TS, SW_PLAIN, DM, decltype(pc)::value>(
-                        const_cast<const UF<R>(*)[T::CELLS]>(lds.luf), const_cast<const R(*)[T::CELLS]>(lds.lo), row,
-                        lane, A.ph.gam, A.gc, none, dev, bad, prod + l);
+                        const_cast<const UF<R>(*)[T::CELLS]>(lds.luf), const_cast<const R(*)[T::CELLS]>(lds.lo),
+                        tl.s0, A.ph.gam, A.gc, none, dev, bad, prod + l);
                 };
                 if (pass == 0) one(std::integral_constant<int, 0>{});
                 else if (pass == 1) one(std::integral_constant<int, 1>{});
@@ -963,14 +1053,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
         if (compute(std::integral_constant<int, DIV_UNSCALED>{})) (void)compute(std::integral_constant<int, DIV_IEEE>{});
         if (!valid) return;
         unsigned fi, ci;
-        if constexpr (along_x(TS)) {
-            const unsigned r = (unsigned)bz * A.g.n[1] + x;
-            fi = r * (X.n + 1) + t;
-            ci = r * X.n + (t - 1);
-        } else {
-            fi = (unsigned)bz * X.oF + t * X.tF + x;
-            ci = (unsigned)bz * X.sB + (unsigned)(t - 1) * X.sA + x;
-        }
+        interface_index<R, TS>(X, t, line, fi, ci);
         // components pass and pass + 4 of this wavefront's interfaces
         for (int c = pass; c < 7; c += 4) {
             R dF = R(0);
@@ -978,7 +1061,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
             for (int m = 0; m < 7; ++m) dF += prod[(m * 7 + c) * 64 + l];
             if (!(A.ct_active && (c == 4 || c == 5))) X.dF[c * X.cF + fi] = dF;
             if ((c == 4 || c == 5) && t >= 1) {  // CT term, as in sweep_interfaces
-                const int s2 = stencil_slot<TS>(row, lane, 2), s3 = stencil_slot<TS>(row, lane, 3);
+                const int s2 = stencil_slot<TS>(tl.s0, 2), s3 = stencil_slot<TS>(tl.s0, 3);
                 const int vt = c == 4 ? O_VT1 : O_VT2;
                 const R b2 = lds.lo[O_BN][s2] * lds.lo[vt][s2], b3 = lds.lo[O_BN][s3] * lds.lo[vt][s3];
                 (c == 4 ? X.ct_a : X.ct_b)[ci] = dF + div_c<R>(R(9) * b2 + R(9) * b3, R(18), R(1.0 / 18.0));

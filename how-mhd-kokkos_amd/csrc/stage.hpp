@@ -44,7 +44,7 @@ constexpr unsigned kRecomputeBlocks = 64;
 #endif
 constexpr unsigned kMarchMinBlocks = 2048;
 inline int march_steps(const dim3& tiles) {
-    const unsigned long long n = (unsigned long long)tiles.x * tiles.y * tiles.z;
+    const unsigned long long n = (unsigned long long)tiles.x * tiles.y;
     unsigned long long s = n / kMarchMinBlocks;
     if (s > HOWMHD_MARCH_STEPS) s = HOWMHD_MARCH_STEPS;
     if (s > tiles.y) s = tiles.y;
@@ -72,13 +72,10 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
 
 // Whether the plain reference-rounding sweeps of a stage run as k_sweep_split.
 // With b blocks on a CU a stage of it takes about 4.6 b - 1 us, and one of
-// k_sweep, whose blocks have four times the interfaces, 6.4 b + 6.6 us; on a
-// line of cells a k_sweep block has no more than the other, and on thin grids
-// not many more.  Per step, k_sweep / split, us: orszag_tang 100^2 143 / 126,
-// 128^2 136 / 122, 144^2 138 / 147, 180^2 170 / 183; 3-D 16^3 186 / 166, 18^3
-// 190 / 185, 20^3 187 / 192, 24^3 212 / 214, 32^3 214 / 273; 60 x 200 218 / 180,
-// 8,192 x 3 237 / 205; lines of 800 cells 106 / 84, 100,000 279 / 189, 1,000,000
-// 1,867 / 1,259.
+// k_sweep, whose blocks have four times the interfaces, 6.4 b + 6.6 us.  Per step,
+// k_sweep / split, us (k_sweep not packed): orszag_tang 100^2 143 / 126, 128^2
+// 136 / 122, 144^2 138 / 147, 180^2 170 / 183; 3-D 16^3 186 / 166, 18^3 190 / 185,
+// 20^3 187 / 192, 24^3 212 / 214, 32^3 214 / 273; a line of 800 cells 106 / 84.
 constexpr unsigned kCUs = 256;
 inline bool split_sweep(const howmhd_gpu_ctx* c) {
     if (c->march_force > 0) return false;
@@ -86,9 +83,9 @@ inline bool split_sweep(const howmhd_gpu_ctx* c) {
     auto per_cu = [](unsigned long long n) { return (n + kCUs - 1) / kCUs; };
     for (int d = 0; d < 3; ++d) {
         if (c->g.n[d] == 1) continue;
-        const dim3 t = sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d), k = sweep_grid(c->g, d);
-        ns += (unsigned long long)t.x * t.y * t.z;
-        nk += (unsigned long long)k.x * k.y * k.z;
+        const dim3 t = split_grid(c->g, d), k = sweep_grid(c->g, d, c->xlanes, true);
+        ns += (unsigned long long)t.x * t.y;
+        nk += (unsigned long long)k.x * k.y;
     }
     return 46 * per_cu(ns) < 64 * per_cu(nk) + 71;
 }
@@ -112,6 +109,7 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
     a.fixhost = c->fixhost;
     const long long nx = c->g.n[0], ny = c->g.n[1], nz = c->g.n[2];
     const int order[3] = {1, 2, 0};
+    constexpr bool packed = MODE != SW_ROUTED;
     unsigned nb = 0;
     for (int k = 0; k < 3; ++k) {
         const int d = order[k];
@@ -124,33 +122,46 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
         x.n = c->g.n[d];
         x.per = c->g.per[d];
         const long long nif = x.n + 1 - (x.per ? 1 : 0);  // computed interfaces per line
-        x.nother = (int)(d == 2 ? ny : nz);
+        const int W = !packed ? 64 : split ? SweepTile<ALONG_X_64>::THREADS : c->xlanes;
+        const Lines l = sweep_lines(c->g, d, packed, d == 0 ? SweepTile<ALONG_X>::THREADS / W : SweepTile<ACROSS_X>::LANES);
+        x.in = (int)l.in;
+        x.nc = (int)(l.period * l.out);
+        x.by_o = launch_div((unsigned)l.period);
+        x.rows_o = (unsigned)l.in;
         x.sA = (unsigned)(d == 0 ? 1 : d == 1 ? nx : nx * ny);
         x.sB = (unsigned)(d == 2 ? nx : nx * ny);
         x.cF = (long long)c->ncell / x.n * (x.n + 1);
         x.tF = x.sA;
         x.oF = (unsigned)(d == 2 ? nx : nx * (ny + 1));
-        x.sS = x.sA;
-        x.oS = (unsigned)(d == 0 ? nif : d == 1 ? nx * nif : nx);
-        const dim3 gr = split ? sweep_grid<ALONG_X_64, ACROSS_X_64>(c->g, d) : sweep_grid(c->g, d);
-        x.gx = gr.x; x.gy = gr.y; x.gz = gr.z;
+        x.sS = (unsigned)(d == 0 ? nif : x.sA);
+        x.oS = (unsigned)(d == 2 ? nx : nx * nif);
+        const dim3 gr = split ? split_grid(c->g, d) : sweep_grid(c->g, d, W, packed);
+        x.gx = gr.x; x.gy = gr.y;
+        if (d == 0) {
+            x.W = W;
+            x.rows = split ? 1 : SweepTile<ALONG_X>::THREADS / W;
+            x.by_w = launch_div(W);
+            x.by_w5 = launch_div(W + 5);
+        }
         x.first = nb;
         x.march = 1;
         x.tile0 = c->tile0[d];
         if (d != 0 && sweep_marches<R, MODE>() && !split)
             x.march = c->march_force > 0 ? (int)std::min<unsigned>(c->march_force, gr.y) : march_steps(gr);
         x.by_gx = launch_div(gr.x);
-        x.by_gy = launch_div((gr.y + x.march - 1) / x.march);
-        if (mask & (1u << d)) nb += gr.x * x.by_gy.d * gr.z;
+        const unsigned along = (gr.y + x.march - 1) / x.march;
+        const unsigned chunk = d == 0 ? gr.x : std::min(gr.x, blocks_for(nx, SweepTile<ACROSS_X>::LANES));
+        x.by_chunk = launch_div(chunk);
+        x.by_blocks = launch_div(along);
+        if (mask & (1u << d)) nb += split ? gr.x * gr.y : blocks_for(gr.x, chunk) * chunk * along;
     }
     *blocks = nb;
     return a;
 }
 
-// LDS of a launch of k_sweep: a tile's, of the larger shape that it holds.  The
-// x tile's alone lets a third FP64 block on a CU, which counts on lines of cells,
-// where three of a block's wavefronts leave at once (fp64fast, 1,000,000 cells,
-// a step: 1,480 -> 1,122 us; FP32 785 -> 669).
+// LDS of a launch of k_sweep: a tile's, of the larger shape that it holds.  With
+// the x tile's alone a CU has room for another block where those are not full:
+// on lines of cells in the routed sweep, whose tiles are not packed.
 template <typename R, int MODE>
 size_t sweep_lds(const SweepArgs<R>& a) {
     constexpr size_t x = tile_lds_bytes<R, MODE, ALONG_X>(), yz = tile_lds_bytes<R, MODE, ACROSS_X>();

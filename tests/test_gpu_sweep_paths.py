@@ -76,3 +76,13 @@ def test_labels_beyond_the_unscaled_range(n, bc, require_gpu):
                 clear = abs(dev - 0.05) > 1e-9
                 assert (y.cpu().numpy() == lab)[clear].all()
             assert (O.large_t_count() > 0) == scaled
+
+
+# rows and columns numbered through both transverse axes, x tiles of 16 to 256
+# interfaces a row: rows shorter than the least, one more and less than 16, 48, 64
+# and 256, tiles that span several planes, a last tile of one line
+@pytest.mark.parametrize("n,bc", [((5, 37, 11), "open"), ((17, 9, 16), "periodic"), ((47, 5, 13), "open"),
+                                  ((65, 3, 17), "periodic"), ((72, 11, 7), "open"), ((255, 3, 5), "open"),
+                                  ((257, 4, 3), "periodic"), ((33, 1, 65), "open"), ((300, 1, 1), "open")])
+def test_packed_lines(n, bc, tiles, require_gpu):
+    _step_matches("mpi_smooth3d", n, bc, steps=1)
