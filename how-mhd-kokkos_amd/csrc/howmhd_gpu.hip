@@ -115,9 +115,10 @@ double dt_from_vmax(const howmhd_params& p, const double* vmax) {
     return p.cour / invdt;
 }
 
-// Largest axis length the launch grids accept on the y and z axes: the
-// sweeps, the face update and the EMF build put an axis length (or a tile
-// count of it) into gridDim.y or gridDim.z.
+// Largest axis length the launch grids accept on the y and z axes: the face
+// update, the EMF build and k_plane put an axis length (or a tile count of it)
+// into gridDim.y or gridDim.z.  (The sweeps' blocks are numbered along x,
+// launch_parts.)
 constexpr int kMaxYZ = 65535;
 
 // Parameter checks of howmhd_gpu_create (no HIP call); "" when valid.

@@ -275,9 +275,11 @@ struct SweepArgs {
     unsigned* fixlist;
     unsigned* fixctl;
     unsigned* fixhost;
-    // the axes of the launch in the order of their blocks: y, z, x (an axis
-    // without blocks starts where the next one does)
+    // the axes of the sweeps in the order of their blocks: y, z, x (an axis
+    // without blocks starts where the next one does), and the first block of
+    // this launch (launch_parts)
     SweepAxis<R> ax[3];
+    unsigned block0;
 };
 
 // dF layout per direction: component-major, interface index t = 0..n along the
@@ -936,9 +938,9 @@ __device__ __forceinline__ void xcd_row_tiles(unsigned L, const SweepAxis<R>& X,
     by = (int)row;
 }
 
-// The sweeps of one launch: the blocks of the y axis, of the z axis (marching
-// blocks, the longest, first) and of the x axis (single tiles, which fill the
-// chip while the last marches end).  Reference rounding, DM = DIV_IEEE: the
+// The sweeps: the blocks of the y axis, of the z axis (marching blocks, the
+// longest, first) and of the x axis (single tiles, which fill the chip while
+// the last marches end).  Reference rounding, DM = DIV_IEEE: the
 // recompute launch (a few blocks) takes the tiles queued by the sweep proper
 // (A.fixlist, A.fixctl[0] of them), clears their flags, and the last block
 // to finish empties the queue; with an empty queue every block exits at once.
@@ -969,7 +971,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             A.fixctl[1] = 0u;
         }
     } else {
-        const unsigned b = blockIdx.x;
+        const unsigned b = A.block0 + blockIdx.x;
         if (b >= A.ax[2].first) {
             int bx, by;
             xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by);

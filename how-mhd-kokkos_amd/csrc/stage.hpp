@@ -70,6 +70,21 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
     return (int)std::min<unsigned long long>(cz, (unsigned long long)most);
 }
 
+// The sweeps' blocks in launches of at most kLaunchBlocks.  The runtime refuses
+// 2^32 threads along x, which 1-D launches of 256 reach at 2^24 blocks: routed
+// tiles are not packed, so a plane of 1 x 8192 x 8192 cells has as many.  (A
+// multiple of 8 keeps the launch's blocks on the XCDs that the tile order means.)
+constexpr unsigned kLaunchBlocks = 1u << 23;
+template <typename R, typename F>
+void launch_parts(SweepArgs<R>& a, unsigned blocks, const F& launch) {
+    for (unsigned done = 0; done < blocks;) {
+        const unsigned n = std::min(blocks - done, kLaunchBlocks);
+        a.block0 = done;
+        launch(n);
+        done += n;
+    }
+}
+
 // Whether the plain reference-rounding sweeps of a stage run as k_sweep_split.
 // With b blocks on a CU a stage of it takes about 4.6 b - 1 us, and one of
 // k_sweep, whose blocks have four times the interfaces, 6.4 b + 6.6 us.  Per step,
@@ -87,7 +102,7 @@ inline bool split_sweep(const howmhd_gpu_ctx* c) {
         ns += (unsigned long long)t.x * t.y;
         nk += (unsigned long long)k.x * k.y;
     }
-    return 46 * per_cu(ns) < 64 * per_cu(nk) + 71;
+    return ns <= kLaunchBlocks && 46 * per_cu(ns) < 64 * per_cu(nk) + 71;
 }
 
 // Arguments of stage iw's sweeps of the axes in `mask` (bit d: axis d) from qsrc;
@@ -178,7 +193,7 @@ void launch_recompute(howmhd_gpu_ctx* c, SweepArgs<R>& a) {
     hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(kRecomputeBlocks), dim3(256), lds, c->stream, a);
 }
 
-// The sweeps of the axes in `mask`, one launch.  Reference rounding: the
+// The sweeps of the axes in `mask`, one launch (launch_parts).  Reference rounding: the
 // sweeps with unscaled WENO divisions, then the launch for the tiles they
 // queued (SW_COLLECT: left to the caller, who waits for the sweep anyway).  Plain
 // sweeps of single tiles redo such a tile in place: no launch, which took 4 us
@@ -192,19 +207,21 @@ void launch_recompute(howmhd_gpu_ctx* c, SweepArgs<R>& a) {
 // by side.
 template <typename R, int MODE>
 void launch_sweep(howmhd_gpu_ctx* c, SweepArgs<R>& a, unsigned blocks) {
-    if (blocks == 0) return;
     const size_t lds = sweep_lds<R, MODE>(a);
     if constexpr (EX && MODE == SW_PLAIN) {
         if (a.ax[0].march == 1 && a.ax[1].march == 1) {
-            hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED, true>), dim3(blocks), dim3(256), lds, c->stream, a);
+            launch_parts(a, blocks, [&](unsigned nb) {
+                hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED, true>), dim3(nb), dim3(256), lds, c->stream, a);
+            });
             return;
         }
     }
-    if constexpr (EX) {
-        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED>), dim3(blocks), dim3(256), lds, c->stream, a);
-        if constexpr (MODE != SW_COLLECT) launch_recompute<R, MODE>(c, a);
-    } else {
-        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_IEEE>), dim3(blocks), dim3(256), lds, c->stream, a);
+    constexpr int DM = EX ? DIV_UNSCALED : DIV_IEEE;
+    launch_parts(a, blocks, [&](unsigned nb) {
+        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DM>), dim3(nb), dim3(256), lds, c->stream, a);
+    });
+    if constexpr (EX && MODE != SW_COLLECT) {
+        if (blocks) launch_recompute<R, MODE>(c, a);
     }
 }
 
