@@ -3,15 +3,20 @@
   * division by 3, 6, 12, 18 and 24 as RN(x h + RN(x l)), h = RN(1/c),
     l = RN(1/c - h), in exact rational arithmetic against the correctly rounded
     quotient: random operands, multiples of the divisor, all-ones
-    significands, operands next to the quotients' rounding boundaries, zeros;
+    significands, operands next to the quotients' rounding boundaries, zeros, the
+    smallest operands of the bound that the code states and those below it;
   * the WENO5 side on doubled arguments with four times eps: exactly twice the
     side on the arguments themselves, weights bit for bit (NumPy doubles),
     from 1e-140 to 1e45; a wrong eps fails.
 """
+import re
 from fractions import Fraction
+from pathlib import Path
 
 import numpy as np
 import pytest
+
+MATH = Path(__file__).resolve().parents[1] / "how-mhd-kokkos_amd" / "csrc" / "mhd_math.hpp"
 
 
 def _rn(f):
@@ -41,6 +46,36 @@ def test_division_by_constant(c):
     h = 1.0 / c
     for x in (0.0, -0.0):  # the sum of products keeps the sign of a zero
         assert np.signbit(x * h + x * lo) == np.signbit(x / c)
+
+
+# divisor -> its least operand of the stated bound that the margin gives (1/18 and
+# 1/6 ulp against a rounding error of 2^-1075)
+_LEAST = {3: 3.0 * 2.0 ** -1020, 6: 6.0 * 2.0 ** -1020, 12: 12.0 * 2.0 ** -1020, 18: 18.0 * 2.0 ** -1018,
+          24: 24.0 * 2.0 ** -1020}
+
+
+@pytest.mark.parametrize("c", [3, 6, 12, 18, 24])
+def test_division_by_constant_smallest_operands(c):
+    """Every binade from the bound that the code states up to 2^-1000, and the four
+    above the divisor's own: the correctly rounded quotient.  Below, for any
+    operand, one of the two doubles next to the quotient."""
+    text = MATH.read_text().split("x / c for a compile-time constant")[1]
+    bound = 2.0 ** -int(re.search(r"\|x\| >= 2\^-(\d+)", text).group(1))
+    assert bound >= _LEAST[c]
+    rng = np.random.default_rng(100 + c)
+
+    def binade(lo, n):
+        return np.concatenate([lo * (1.0 + rng.random(n)), [lo, np.nextafter(lo, np.inf)]])
+
+    lows = [2.0 ** -e for e in range(1000, -int(np.log2(bound)) + 1)] + [_LEAST[c] * 2.0 ** k for k in range(4)]
+    for lo in lows:
+        for x in binade(lo, 2000):
+            x = float(x)
+            assert _two_step(x, c)[1] == _rn(Fraction(x) / c), x.hex()
+    for e in range(1014, 1075):
+        for x in 2.0 ** -e * (1.0 + rng.random(50)):
+            got, exact = _two_step(float(x), c)[1], Fraction(float(x)) / c
+            assert Fraction(np.nextafter(got, -np.inf)) < exact < Fraction(np.nextafter(got, np.inf))
 
 
 def _side(a, b, c, d, eps):
