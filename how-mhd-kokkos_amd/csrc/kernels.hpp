@@ -950,7 +950,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
     SweepArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
     static_assert(EX || DM == DIV_IEEE, "the FMA forms divide with IEEE divisions");
-    extern __shared__ unsigned char raw[];  // a tile's values (sweep_lds)
+    // a tile's values (sweep_lds).  They lie behind the static LDS of the device
+    // functions called here (__syncthreads_or has 256 bytes), whatever its size.
+    extern __shared__ __align__(16) unsigned char raw[];
+    static_assert(__alignof__(raw) >= alignof(UF<R>), "(U, F) pairs are read as one LDS access");
     if constexpr (EX && DM == DIV_IEEE) {
         const unsigned n = A.fixctl[0];
         for (unsigned i = blockIdx.x; i < n; i += gridDim.x) {
@@ -1011,6 +1014,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
     constexpr int CELLS = SweepTile<ACROSS_X_64>::CELLS;
     static_assert(CELLS <= 256 && SweepTile<ALONG_X_64>::CELLS <= CELLS, "one cell per thread");
     __shared__ alignas(16) unsigned char raw[tile_lds_bytes<R, SW_PLAIN, ACROSS_X_64>()];
+    static_assert(__alignof__(raw) >= alignof(UF<R>), "(U, F) pairs are read as one LDS access");
     __shared__ R prod[7 * 7 * 64];
     auto tile = [&](auto tsc, const SweepAxis<R>& X) {
         constexpr int TS = decltype(tsc)::value;
