@@ -87,10 +87,14 @@ void launch_parts(SweepArgs<R>& a, unsigned blocks, const F& launch) {
 
 // Whether the plain reference-rounding sweeps of a stage run as k_sweep_split.
 // With b blocks on a CU a stage of it takes about 4.6 b - 1 us, and one of
-// k_sweep, whose blocks have four times the interfaces, 6.4 b + 6.6 us.  Per step,
-// k_sweep / split, us (k_sweep not packed): orszag_tang 100^2 143 / 126, 128^2
-// 136 / 122, 144^2 138 / 147, 180^2 170 / 183; 3-D 16^3 186 / 166, 18^3 190 / 185,
-// 20^3 187 / 192, 24^3 212 / 214, 32^3 214 / 273; a line of 800 cells 106 / 84.
+// k_sweep, whose blocks have up to four times the interfaces, 6.4 b + 6.6 us.  The
+// two are level at 3 blocks of it on a CU beside 1 of k_sweep.  Measured per step,
+// k_sweep / split, us: 2 beside 1, orszag_tang 100^2 144 / 124, 128^2 136 / 121;
+// 16^3 177 / 155, a line of 30,000 cells 112 / 94; 3 beside 1, 136^2 140 / 147,
+// 144^2 139 / 146, 20^3 184 / 179, 16 x 600 184 / 176, a line of 40,001 118 / 119;
+// more, 160^2 141 / 160, 24^3 189 / 200, 32^3 218 / 273, a line of 60,000 120 / 132.
+// (14^3, 15^3 and 18^3 take 240 us in k_sweep: the last group of columns has 1 or
+// 4 of its 32, and a wavefront with so few active lanes is slower.)
 constexpr unsigned kCUs = 256;
 inline bool split_sweep(const howmhd_gpu_ctx* c) {
     if (c->march_force > 0) return false;

@@ -86,3 +86,24 @@ def test_labels_beyond_the_unscaled_range(n, bc, require_gpu):
                                   ((257, 4, 3), "periodic"), ((33, 1, 65), "open"), ((300, 1, 1), "open")])
 def test_packed_lines(n, bc, tiles, require_gpu):
     _step_matches("mpi_smooth3d", n, bc, steps=1)
+
+
+# the largest grids of the split sweep beside the smallest of k_sweep (64 interfaces
+# a block, 256 CUs: 512 blocks and more; one row, column or line of cells apart
+# where the packed tiles allow it), for every set of axes; True: split.  The CPU
+# test of the launches checks the sides.
+SPLIT_EDGE = [((32768, 1, 1), "periodic", True), ((32769, 1, 1), "periodic", False),
+              ((32767, 1, 1), "open", True), ((32768, 1, 1), "open", False),
+              ((128, 128, 1), "periodic", True), ((128, 129, 1), "periodic", False),
+              ((127, 120, 1), "open", True), ((127, 128, 1), "open", False),
+              ((8192, 3, 1), "periodic", True), ((12000, 3, 1), "open", False),
+              ((128, 1, 128), "periodic", True), ((129, 1, 128), "periodic", False),
+              ((1, 127, 127), "open", True), ((1, 128, 132), "periodic", False),
+              ((17, 17, 17), "open", True), ((18, 18, 18), "periodic", False),
+              ((64, 16, 9), "periodic", True), ((65, 16, 9), "periodic", False)]
+
+
+@pytest.mark.parametrize("n,bc,split", SPLIT_EDGE)
+def test_split_edge(n, bc, split, require_gpu):
+    # (grids without an x axis end in NaN, whose sign bits are the processor's, in the second step)
+    _step_matches("mpi_smooth3d", n, bc, steps=2 if n[0] > 1 else 1)

@@ -6,12 +6,17 @@ The runtime takes fewer than 2^32 threads along an axis of a launch and at most
 tiles, so thin grids that fit the device have more tiles than one launch of
 256-thread blocks may: the grids below need 2^24 and more.  Every tile of every
 axis is computed once, however the blocks are divided into launches.
+
+Which plain FP64 grids take k_sweep_split: both sides of the rule, which the GPU
+test of the same grids runs.
 """
 import shutil
 import subprocess
 from pathlib import Path
 
 import pytest
+
+from test_gpu_sweep_paths import SPLIT_EDGE
 
 ROOT = Path(__file__).resolve().parents[1]
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -60,3 +65,11 @@ def test_launches_fit_and_cover(n, bc, form, stage_launches):
     for axis, (want, once, more) in tiles.items():
         assert (once, more) == (want, 0), axis
     assert {a for a, t in tiles.items() if t[0]} == {a for a, k in zip("xyz", n) if k > 1}
+
+
+@pytest.mark.parametrize("n,bc,split", SPLIT_EDGE + [((128, 128, 1), "open", False), ((800, 1, 1), "open", True),
+                                                     ((256, 256, 256), "periodic", False)])
+def test_split_sides(n, bc, split, stage_launches):
+    launches, _ = stage_launches(n, bc, "fp64")
+    assert any("k_sweep_split" in kernel for kernel, *_ in launches) == split
+    assert any("k_sweep<" in kernel for kernel, *_ in launches) != split
