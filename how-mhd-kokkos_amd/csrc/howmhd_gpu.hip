@@ -249,17 +249,20 @@ int howmhd_gpu_create(const howmhd_params* p, howmhd_gpu_ctx** out) {
         }
     }
     for (int t = 0; t < 6 && ok; ++t) ok = ok && alloc(&c->ct[t], c->ncell * c->rsize);
-    // the unsmoothed EMFs O2 live in memory only on 1-D/2-D grids; on 3-D
-    // grids k_emf_march keeps them on chip
+    // the EMFs that the grid's axes have, unless k_plane keeps them on chip; the
+    // unsmoothed ones O2 live in memory only on x-z and y-z grids (on 3-D grids
+    // k_emf_march keeps them on chip)
+    c->plane = n[0] > 1 && n[1] > 1 && n[2] == 1;
     const bool emf_fused = c->ctf.use_x && c->ctf.use_y && c->ctf.use_z;
-    for (int t = 0; t < 3 && ok; ++t) {
+    const int use_O[3] = {c->ctf.use_Ox, c->ctf.use_Oy, c->ctf.use_Oz};
+    for (int t = 0; t < 3 && ok && !c->plane; ++t) {
+        if (!use_O[t]) continue;
         if (!emf_fused) ok = ok && alloc(&c->O2[t], c->ncell * c->rsize);
         ok = ok && alloc(&c->O[t], c->ncell * c->rsize);
     }
     small((void**)&c->cflfold, 3 * CFL_FOLD_BLOCKS * sizeof(double));
     small((void**)&c->statfold, 4 * STAT_FOLD_BLOCKS * sizeof(unsigned long long));
     small((void**)&c->done, 2 * sizeof(unsigned));
-    c->plane = n[0] > 1 && n[1] > 1 && n[2] == 1;
     const dim3 pg = plane_grid(c->g);
     c->ncombine = c->plane ? (long long)pg.x * pg.y : blocks_for(c->ncell, 256);
     // (k_cfl leaves its partials in cflpart, too)

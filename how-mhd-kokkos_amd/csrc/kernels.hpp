@@ -1080,8 +1080,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
 
 template <typename R>
 struct EmfArgs {
-    const R *fsy, *fsz, *gsx, *gsz, *hsx, *hsy;
-    R *Ox2, *Oy2, *Oz2;
+    const R *fsz, *gsz, *hsx, *hsy;
+    R *Oy2, *Oz2;
     Geom g;
     CtFlags f;
 };
@@ -1093,7 +1093,8 @@ __device__ __forceinline__ R i4(R a, R b, R c, R d) {
     return div_c<R>(-a + R(9) * b + R(9) * c - d, R(16), R(1.0 / 16.0));
 }
 
-// fluxct_build_O2, src/fluxct.cpp:809-821, on active cells
+// fluxct_build_O2, src/fluxct.cpp:809-821, on active cells; k_emf2, k_emf and
+// k_faces run on x-z grids (Oz alone) and y-z grids (Oy alone)
 template <typename R, int EX>
 __global__ __launch_bounds__(256) void k_emf2(EmfArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
@@ -1103,12 +1104,6 @@ __global__ __launch_bounds__(256) void k_emf2(EmfArgs<R> A) {
     int x, y, z;
     cell_of(g, i, x, y, z);
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    if (A.f.use_Ox) {
-        const int xm = bmap(x - 1, nx, g.per[0]), xp = bmap(x + 1, nx, g.per[0]), xq = bmap(x + 2, nx, g.per[0]);
-        const int ym = bmap(y - 1, ny, g.per[1]), yp = bmap(y + 1, ny, g.per[1]), yq = bmap(y + 2, ny, g.per[1]);
-        A.Ox2[i] = i4<R>(A.gsx[lin(g, xm, y, z)], A.gsx[i], A.gsx[lin(g, xp, y, z)], A.gsx[lin(g, xq, y, z)]) -
-                   i4<R>(A.fsy[lin(g, x, ym, z)], A.fsy[i], A.fsy[lin(g, x, yp, z)], A.fsy[lin(g, x, yq, z)]);
-    }
     if (A.f.use_Oy) {
         const int ym = bmap(y - 1, ny, g.per[1]), yp = bmap(y + 1, ny, g.per[1]), yq = bmap(y + 2, ny, g.per[1]);
         const int zm = bmap(z - 1, nz, g.per[2]), zp = bmap(z + 1, nz, g.per[2]), zq = bmap(z + 2, nz, g.per[2]);
@@ -1131,8 +1126,8 @@ __device__ __forceinline__ R lap24(R m, R c, R p) {
 
 template <typename R>
 struct SmoothArgs {
-    const R *Ox2, *Oy2, *Oz2;
-    R *Ox, *Oy, *Oz;
+    const R *Oy2, *Oz2;
+    R *Oy, *Oz;
     Geom g;
     CtFlags f;
 };
@@ -1147,11 +1142,6 @@ __global__ __launch_bounds__(256) void k_emf(SmoothArgs<R> A) {
     int x, y, z;
     cell_of(g, i, x, y, z);
     const int nx = g.n[0], ny = g.n[1], nz = g.n[2];
-    if (A.f.use_Ox) {
-        const R o = A.Ox2[i];
-        A.Ox[i] = o + lap24<R>(A.Ox2[lin(g, bmap(x - 1, nx, g.per[0]), y, z)], o, A.Ox2[lin(g, bmap(x + 1, nx, g.per[0]), y, z)]) +
-                  lap24<R>(A.Ox2[lin(g, x, bmap(y - 1, ny, g.per[1]), z)], o, A.Ox2[lin(g, x, bmap(y + 1, ny, g.per[1]), z)]);
-    }
     if (A.f.use_Oy) {
         const R o = A.Oy2[i];
         A.Oy[i] = o + lap24<R>(A.Oy2[lin(g, x, bmap(y - 1, ny, g.per[1]), z)], o, A.Oy2[lin(g, x, bmap(y + 1, ny, g.per[1]), z)]) +
@@ -1394,17 +1384,15 @@ __device__ __forceinline__ double d4(double om3, double om2, double om1, double 
 
 // fluxct_update_bfield, src/fluxct.cpp:850-877, with the stage initialisation
 // of copy_bfield_stage / prepare_bfield_stage5 (111-135) folded in.
-// For the grids of two axes that k_plane does not take (xz and yz).
 // Block = FACE_TX x FACE_TY cells of one z plane.  The in-plane stencils
-// (Ox along x and y, Oy along y, Oz along x) are read from LDS copies of the
-// tile with its 3-cell halo (each value read once per block instead of six
-// times through L2); the z stencils of Oy and Oz are read from memory.
+// (Oy along y, Oz along x) are read from LDS copies of the tile with its 3-cell
+// halo (each value read once per block instead of six times through L2); the z
+// stencils of Oy and Oz are read from memory.
 constexpr int FACE_TX = 32, FACE_TY = 8;
 template <typename R, int EX>
 __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
     static_assert(EX == HOWMHD_EXACT, "kernel instantiated in a unit of the other rounding form");
     constexpr int HX = FACE_TX + 5, HY = FACE_TY + 5;
-    __shared__ R sOx[HY][HX];       // rows y0-3 .. y0+TY+1, columns x0-3 .. x0+TX+1
     __shared__ R sOy[HY][FACE_TX];  // rows y0-3 .. y0+TY+1
     __shared__ R sOz[FACE_TY][HX];  // columns x0-3 .. x0+TX+1
     const Geom& g = A.g;
@@ -1417,8 +1405,6 @@ __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
     // into the range bmap covers (those entries are never read)
     auto hx = [&](int c) { const int a = x0 - 3 + c; return bmap(a > nx + 2 ? nx + 2 : a, nx, px); };
     auto hy = [&](int r) { const int a = y0 - 3 + r; return bmap(a > ny + 2 ? ny + 2 : a, ny, py); };
-    if (f.use_Ox)
-        for (int k = tid; k < HY * HX; k += 256) sOx[k / HX][k % HX] = A.Ox[lin(g, hx(k % HX), hy(k / HX), z)];
     if (f.use_Oy)
         for (int k = tid; k < HY * FACE_TX; k += 256) {
             const int c = k % FACE_TX, xx = x0 + c < nx ? x0 + c : nx - 1;
@@ -1446,29 +1432,22 @@ __global__ __launch_bounds__(256) void k_faces(FaceArgs<R> A) {
         return d4(at(bmap(z - 3, nz, pz)), at(bmap(z - 2, nz, pz)), at(bmap(z - 1, nz, pz)), at(z),
                   at(bmap(z + 1, nz, pz)), at(bmap(z + 2, nz, pz)));
     };
-    auto col6 = [&](const R (*t)[HX], int c) -> double {  // rows y-3..y+2 of column c
-        return d4((double)t[ty][c], (double)t[ty + 1][c], (double)t[ty + 2][c], (double)t[ty + 3][c],
-                  (double)t[ty + 4][c], (double)t[ty + 5][c]);
-    };
     auto row6 = [&](const R* r) -> double {  // columns x-3..x+2 of a tile row
         return d4((double)r[tx], (double)r[tx + 1], (double)r[tx + 2], (double)r[tx + 3], (double)r[tx + 4],
                   (double)r[tx + 5]);
     };
     double bx = binit[0], by = binit[1], bz = binit[2];
-    if (f.use_Ox || f.use_Oz) {
-        double dOx = 0.0, dOz = 0.0;
-        if (f.use_Ox) dOx = col6(sOx, tx + 3);
-        if (f.use_Oz) dOz = dz_of(A.Oz);
-        bx = s.k1 * binit[0] + s.k3 * A.bp[i] - s.dtdy * dOx + s.dtdz * dOz;
+    const double none = 0.0;  // the differences along the axis of one cell
+    if (f.use_Oz) {
+        const double dOz = dz_of(A.Oz);
+        bx = s.k1 * binit[0] + s.k3 * A.bp[i] - s.dtdy * none + s.dtdz * dOz;
     }
-    if (f.use_Oy || f.use_Ox) {
-        double dOy = 0.0, dOx = 0.0;
-        if (f.use_Oy) dOy = dz_of(A.Oy);
-        if (f.use_Ox) dOx = row6(sOx[ty + 3]);
-        by = s.k1 * binit[1] + s.k3 * A.bp[g.ncell + i] - s.dtdz * dOy + s.dtdx * dOx;
+    if (f.use_Oy) {
+        const double dOy = dz_of(A.Oy);
+        by = s.k1 * binit[1] + s.k3 * A.bp[g.ncell + i] - s.dtdz * dOy + s.dtdx * none;
     }
     if (f.use_Oz || f.use_Oy) {
-        double dOz = 0.0, dOy = 0.0;
+        double dOz = none, dOy = none;
         if (f.use_Oz) dOz = row6(sOz[ty]);
         if (f.use_Oy)
             dOy = d4((double)sOy[ty][tx], (double)sOy[ty + 1][tx], (double)sOy[ty + 2][tx], (double)sOy[ty + 3][tx],

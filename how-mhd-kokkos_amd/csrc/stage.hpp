@@ -126,7 +126,7 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
     a.fixlist = c->fixlist;
     a.fixctl = c->fixctl;
     a.fixhost = c->fixhost;
-    const long long nx = c->g.n[0], ny = c->g.n[1], nz = c->g.n[2];
+    const long long nx = c->g.n[0], ny = c->g.n[1];
     const int order[3] = {1, 2, 0};
     constexpr bool packed = MODE != SW_ROUTED;
     unsigned nb = 0;
@@ -351,10 +351,9 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
         HCHECK(c, hipGetLastError());
     } else if (c->ctf.active) {
         EmfArgs<R> e;
-        e.fsy = (const R*)c->ct[0]; e.fsz = (const R*)c->ct[1];
-        e.gsx = (const R*)c->ct[2]; e.gsz = (const R*)c->ct[3];
+        e.fsz = (const R*)c->ct[1]; e.gsz = (const R*)c->ct[3];
         e.hsx = (const R*)c->ct[4]; e.hsy = (const R*)c->ct[5];
-        e.Ox2 = (R*)c->O2[0]; e.Oy2 = (R*)c->O2[1]; e.Oz2 = (R*)c->O2[2];
+        e.Oy2 = (R*)c->O2[1]; e.Oz2 = (R*)c->O2[2];
         e.g = c->g;
         e.f = c->ctf;
         {
@@ -363,8 +362,8 @@ int launch_stage(howmhd_gpu_ctx* c, int iw, double dt) {
         }
         HCHECK(c, hipGetLastError());
         SmoothArgs<R> m;
-        m.Ox2 = (const R*)c->O2[0]; m.Oy2 = (const R*)c->O2[1]; m.Oz2 = (const R*)c->O2[2];
-        m.Ox = (R*)c->O[0]; m.Oy = (R*)c->O[1]; m.Oz = (R*)c->O[2];
+        m.Oy2 = (const R*)c->O2[1]; m.Oz2 = (const R*)c->O2[2];
+        m.Oy = (R*)c->O[1]; m.Oz = (R*)c->O[2];
         m.g = c->g;
         m.f = c->ctf;
         {

@@ -120,3 +120,25 @@ def test_one_plane(n, bc, require_gpu):
 @pytest.mark.parametrize("bc", ["periodic", "open"])
 def test_one_axis(n, bc, require_gpu):
     _step_matches("mpi_smooth3d", n, bc, steps=2, one_nan=True)
+
+
+# arrays of a context in FP64, values a cell: q and faces of 5 stages, 7 fluxes an
+# axis, 6 CT terms; the EMF and the unsmoothed one of two-axis grids that k_plane
+# does not take.  Beside them, at most `more`: arrays of a few values a tile (88 B a
+# tile of the sweeps, which has 8 cells on a y-z grid: 2.8 values a cell), the
+# last interfaces, allocations rounded up to 2 MiB.
+@pytest.mark.parametrize("n,values,more", [((4096, 4000, 1), 40 + 15 + 14 + 6, 1.0),
+                                           ((16000000, 1, 1), 40 + 15 + 7 + 6, 1.0),
+                                           ((4096, 1, 4000), 40 + 15 + 14 + 6 + 2, 1.0),
+                                           ((1, 4096, 4000), 40 + 15 + 14 + 6 + 2, 3.5)])
+def test_context_memory(n, values, more, require_gpu):
+    torch = pytest.importorskip("torch")
+    params = H.gpu_params(H.parse(H.make_input(problem="mpi_smooth3d", nx=8, ny=8, nz=8, nt=1, tend=1.0)))
+    H.GpuSolver(params).close()  # what the process allocates once
+    params.nx, params.ny, params.nz = n
+    before = torch.cuda.mem_get_info()[0]
+    g = H.GpuSolver(params)
+    used = (before - torch.cuda.mem_get_info()[0]) / (8.0 * n[0] * n[1] * n[2])
+    g.close()
+    print(f"[launch rules] memory {n}: {used:.2f} values a cell", flush=True)
+    assert values <= used < values + more
