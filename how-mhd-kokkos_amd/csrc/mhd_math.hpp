@@ -64,10 +64,15 @@ __device__ __forceinline__ R div_by(R a, R b, R y) {
 // reciprocal, a function of b alone) and div_with.  So quotients that share a
 // denominator share its refinement and stay bit-for-bit the IEEE quotient.
 // The refinement here is one third-order step, r0 (1 + e + e^2) with
-// e = 1 - b r0 of 2^-24, instead of two Newton steps: three FMAs instead of
-// four, and the same 1/b but for cases within 2^-72 of a rounding boundary
-// (3.4e9 random and edge-case operands for each use: 1/t, 3/t, 6/t, alpha/S
-// and recip_rn, no difference from the IEEE quotient).
+// e = 1 - b r0 of at most 2^-24, instead of two Newton steps: three FMAs instead
+// of four.  Before its rounding the result is off by e^3, 2^-72 of 1/b, so it is
+// RN(1/b) except for the one b in some 2^18 whose 1/b lies that near to a
+// midpoint, where it can be the double on its other side.  div_with's remainder
+// step gives the IEEE quotient from RN(1/b) (Markstein's theorem).  From the
+// other double its value before rounding is off by 2^-52 ulp at most, so the
+// quotient can differ only where a/b lies that near to a midpoint, too: one pair
+// (a, b) in some 2^70.  (3.4e9 random and edge-case operands for each use, 1/t,
+// 3/t, 6/t, alpha/S and recip_rn, show no difference.)
 __device__ __forceinline__ double div_recip(double b) {
     const double r0 = __builtin_amdgcn_rcp(b);
     const double e = __builtin_fma(-b, r0, 1.0);
@@ -78,7 +83,12 @@ __device__ __forceinline__ double div_with(double a, double b, double r) {
     return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 // RN(1/b) for b in [2^-900, 2^900] (the division of 1 by b in these parts):
-// six instructions instead of the IEEE division's eleven.
+// six instructions instead of the IEEE division's eleven.  With r either double
+// next to 1/b and d = 1 - b r, exact, the step's r + r d is below 1/b by r d^2, less
+// than 2^-106 of it, and 2^-106 is the least distance of 1/b from a midpoint.
+// The one b whose step can tie is the all-ones significand from the double
+// below; the card's reciprocal gives it from the one above (checked for every
+// exponent).
 __device__ __forceinline__ double recip_rn(double b) {
     const double r = div_recip(b);
     return __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);

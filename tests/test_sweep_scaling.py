@@ -5,6 +5,7 @@
     quotient: random operands, multiples of the divisor, all-ones
     significands, operands next to the quotients' rounding boundaries, zeros, the
     smallest operands of the bound that the code states and those below it;
+  * the last step of the reciprocal, in exact rational arithmetic;
   * the WENO5 side on doubled arguments with four times eps: exactly twice the
     side on the arguments themselves, weights bit for bit (NumPy doubles),
     from 1e-140 to 1e45; a wrong eps fails.
@@ -76,6 +77,24 @@ def test_division_by_constant_smallest_operands(c):
         for x in 2.0 ** -e * (1.0 + rng.random(50)):
             got, exact = _two_step(float(x), c)[1], Fraction(float(x)) / c
             assert Fraction(np.nextafter(got, -np.inf)) < exact < Fraction(np.nextafter(got, np.inf))
+
+
+def test_reciprocal_step():
+    """The last step of recip_rn from either double next to 1/b: the correctly
+    rounded reciprocal, but for the all-ones significand from the double below."""
+    rng = np.random.default_rng(3)
+    ms = [int(m) for m in rng.integers(1 << 52, 1 << 53, 20000)]
+    ms += [(1 << 52) + k for k in range(1, 200)] + [(1 << 53) - k for k in range(1, 200)]
+    for m in ms:
+        b = m * 2.0 ** -52
+        exact = 1 / Fraction(b)
+        want = _rn(exact)
+        below = want if Fraction(want) < exact else float(np.nextafter(want, 0.0))
+        for r in (below, float(np.nextafter(below, 1.0))):
+            d = 1 - Fraction(b) * Fraction(r)
+            assert Fraction(_rn(d)) == d  # the remainder is a double
+            got = _rn(Fraction(r) + Fraction(r) * d)
+            assert (got == want) != (m == (1 << 53) - 1 and r == below), b.hex()
 
 
 def _side(a, b, c, d, eps):
