@@ -10,6 +10,7 @@
 #pragma once
 
 #include "howmhd_gpu.h"
+#include "helpers.hpp"
 #include "kernels.hpp"
 
 #include <hip/hip_runtime.h>
@@ -69,6 +70,7 @@ struct howmhd_gpu_ctx {
     size_t xfer_slot = 0;
     int xfer_n = 0;
     std::vector<hipEvent_t> xfer_ev;
+    howmhd::Helpers xfer_helpers;  // threads that copy beside the caller's
     // learned indicator: device weights, routing mode (0 off, 1 on with the
     // plain-WENO fallback, 2 on for every step), the routed sweeps' counter
     // words (per stage nwave words, four per tile of the x, y and z sweeps

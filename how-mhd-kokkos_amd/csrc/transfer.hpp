@@ -8,8 +8,9 @@
 // without ghosts.  Host threads move chunks between the caller's (pageable)
 // memory and their slots, filling the ghost layers with their images on the
 // way down, while the transpose kernel reads or writes the other slots of the
-// pinned memory over PCIe; on large grids each thread owns two slots, so that
-// its copy overlaps its kernel.
+// pinned memory over PCIe; on large grids there are two slots a thread, so that
+// its copy overlaps its kernel.  A thread that comes late finds less to do, or
+// nothing (helpers.hpp).
 //
 // Bound: PCIe (56 GB/s each way) for large grids, the first touch of the
 // caller's pages on the way down, the start of the threads and one chunk's
@@ -26,18 +27,16 @@
 #include <sched.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
 namespace howmhd {
 namespace {
 
-constexpr int kXferThreads = 8, kXferChunks = 2 * kXferThreads;
+constexpr int kXferThreads = 8, kXferChunks = 2 * kXferThreads, kXferSlots = 2 * kXferThreads;
 constexpr size_t kXferSlotMax = 1u << 18, kXferSlotMin = 1u << 15;  // values: 2 MiB, 256 KiB
 
 // Values per slot of a context of ncell cells: eight variables in 16 chunks,
@@ -51,7 +50,7 @@ inline size_t xfer_slot(size_t ncell, int nz) {
 // transfer nothing and halves the memory that create pins and the first
 // transfer touches (64^3: first upload 1.20 against 1.58 ms).
 inline int xfer_slots(size_t ncell, size_t slot) {
-    const size_t most = slot < kXferSlotMax ? kXferThreads : 2 * kXferThreads;
+    const size_t most = slot < kXferSlotMax ? kXferThreads : kXferSlots;
     return (int)std::min(most, (8 * ncell + slot - 1) / slot);
 }
 
@@ -148,16 +147,33 @@ int transfer(howmhd_gpu_ctx* c, double* ref, double* dev, int nvar) {
     const Geom& g = c->g;
     const size_t n6 = ((size_t)g.n[0] + 6) * ((size_t)g.n[1] + 6) * ((size_t)g.n[2] + 6);
     std::vector<Chunk> chunks;
-    std::vector<std::thread> pool;
-    std::atomic<size_t> next{0};
+    try {
+        chunks = xfer_chunks(g, nvar, c->xfer_slot);
+    } catch (const std::bad_alloc&) {
+        return fail(c, HOWMHD_ENOMEM, "host transfer: out of host memory");
+    }
+    // threads where they have a MiB of the caller's memory each, two chunks in flight for each
+    const size_t bytes = nvar * n6 * sizeof(double);
+    const int nw = (int)std::max<size_t>(1, std::min<size_t>({(size_t)cpu_share(), kXferThreads, chunks.size(), bytes >> 20,
+                                                              (size_t)c->xfer_n}));
+    const int most = 2 * nw;
+    // Under the mutex: the next chunk, the free slots (a bit each), the slots
+    // with a chunk in flight, oldest first, and the first error.  A thread is
+    // at one slot at a time; any thread may finish any chunk in flight.
     std::mutex mu;
+    size_t next = 0;
+    unsigned idle = (1u << c->xfer_n) - 1;
+    struct {
+        int slot;
+        size_t chunk;
+    } flight[kXferSlots];
+    int first = 0, flying = 0;
     hipError_t err = hipSuccess;
     const char* what = "";
     auto report = [&](hipError_t e, const char* w) {
         std::lock_guard<std::mutex> lk(mu);
         if (err == hipSuccess) { err = e; what = w; }
         (void)hipGetLastError();
-        next.store((size_t)-1 / 2);  // no further chunks
     };
     auto launch = [&](const Chunk& k, int slot) {
         const int ncol = k.nj * g.n[2];
@@ -176,45 +192,44 @@ int transfer(howmhd_gpu_ctx* c, double* ref, double* dev, int nvar) {
         if (e != hipSuccess) report(e, "hipEventSynchronize");
         return e == hipSuccess;
     };
-    // worker w of nw: slots w and w + nw (the second where there is one)
-    int nw = 1;
-    auto work = [&](int w) {
-        if (w > 0 && hipSetDevice(c->device) != hipSuccess) return report(hipErrorInvalidDevice, "hipSetDevice");
-        const int slots[2] = {w, w + nw};
-        const int ns = w + nw < c->xfer_n ? 2 : 1;
-        size_t held[2] = {(size_t)-1, (size_t)-1};  // chunk in flight in each slot
-        auto drain = [&](int s) {
-            if (held[s] == (size_t)-1) return true;
-            if (!arrived(slots[s])) return false;
-            if (!UP) unpack(g, c->xfer + (size_t)slots[s] * c->xfer_slot, chunks[held[s]], ref);
-            held[s] = (size_t)-1;
-            return true;
-        };
-        int s = 0;
-        for (size_t k; (k = next.fetch_add(1)) < chunks.size(); s = (s + 1) % ns) {
-            if (!drain(s)) return;
-            if (UP) pack(g, ref, chunks[k], c->xfer + (size_t)slots[s] * c->xfer_slot);
-            if (!launch(chunks[k], slots[s])) return;
-            held[s] = k;
+    auto work = [&](bool helper) {
+        if (helper && hipSetDevice(c->device) != hipSuccess) return report(hipErrorInvalidDevice, "hipSetDevice");
+        for (;;) {
+            int slot;
+            size_t k;
+            bool fill;
+            {
+                std::lock_guard<std::mutex> lk(mu);
+                const bool more = next < chunks.size();
+                fill = more && idle != 0 && flying < most;
+                if (err != hipSuccess) return;
+                if (fill) {
+                    slot = __builtin_ctz(idle);
+                    idle &= idle - 1;
+                    k = next++;
+                } else if (flying > 0 && (more || !UP)) {  // (up, the stream's end ends the last ones)
+                    slot = flight[first].slot;
+                    k = flight[first].chunk;
+                    first = (first + 1) % kXferSlots;
+                    --flying;
+                } else {
+                    return;  // no more threads than slots: what is left is in other threads' hands
+                }
+            }
+            if (fill) {
+                if (UP) pack(g, ref, chunks[k], c->xfer + (size_t)slot * c->xfer_slot);
+                if (!launch(chunks[k], slot)) return;
+                std::lock_guard<std::mutex> lk(mu);
+                flight[(first + flying++) % kXferSlots] = {slot, k};
+            } else {
+                if (!arrived(slot)) return;
+                if (!UP) unpack(g, c->xfer + (size_t)slot * c->xfer_slot, chunks[k], ref);
+                std::lock_guard<std::mutex> lk(mu);
+                idle |= 1u << slot;
+            }
         }
-        for (int t = 0; t < ns; ++t, s = (s + 1) % ns)
-            if (!drain(s)) return;
     };
-    try {
-        chunks = xfer_chunks(g, nvar, c->xfer_slot);
-        // threads where they have a MiB of the caller's memory each
-        const size_t bytes = nvar * n6 * sizeof(double);
-        nw = (int)std::max<size_t>(1, std::min<size_t>({(size_t)cpu_share(), kXferThreads, chunks.size(), bytes >> 20,
-                                                        (size_t)c->xfer_n}));
-        pool.reserve(nw);
-        for (int w = 1; w < nw; ++w) pool.emplace_back(work, w);
-    } catch (const std::system_error&) {
-        // no further threads: the chunks go to those there are
-    } catch (const std::bad_alloc&) {
-        if (chunks.empty()) return fail(c, HOWMHD_ENOMEM, "host transfer: out of host memory");
-    }
-    work(0);
-    for (auto& t : pool) t.join();
+    c->xfer_helpers.run(nw - 1, work);
     if (err != hipSuccess) {
         (void)hipStreamSynchronize(c->stream);
         return fail(c, HOWMHD_EHIP, std::string("host transfer: ") + what + ": " + hipGetErrorString(err));

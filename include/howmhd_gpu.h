@@ -117,8 +117,10 @@ HOWMHD_API int howmhd_gpu_destroy(howmhd_gpu_ctx* ctx);
  * (src/problem.cpp:39-59); this is the device hand-over of that array.
  * Host transfers (this call, upload_faces and the downloads) move the active
  * cells in chunks through the context's pinned host memory (at most 32 MiB);
- * up to eight host threads, joined before the call returns, copy between it
- * and the caller's memory while the layout change runs on the device.
+ * up to eight host threads (the caller's and helpers) copy between it and the
+ * caller's memory while the layout change runs on the device.  A helper that has
+ * got no processor when the transfer is done is not waited for: it leaves later
+ * without touching the caller's memory (howmhd_gpu_destroy waits for it).
  * Synchronises. */
 HOWMHD_API int howmhd_gpu_upload_q0(howmhd_gpu_ctx* ctx, const double* q0);
 
