@@ -313,7 +313,10 @@ class GpuSolver:
         self._check(self.lib.howmhd_gpu_set_timing(self.h, int(on)), "set_timing")
 
     def timing(self) -> dict:
-        """{kernel: (total ms, launches)} of the launches timed since set_timing(True)."""
+        """{kernel: (total ms, launches)} of the launches timed since set_timing(True).
+
+        On x-y planes everything after the sweeps is booked as "combine"; the sweeps
+        run one axis at a time while timing is on (howmhd_gpu.h)."""
         t = Timing()
         self._check(self.lib.howmhd_gpu_get_timing(self.h, C.byref(t)), "get_timing")
         return {k: (t.ms[i], t.launches[i]) for i, k in enumerate(KERNELS)}

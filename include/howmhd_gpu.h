@@ -88,7 +88,13 @@ typedef struct howmhd_diag {
 } howmhd_diag;
 
 /* Per-kernel device time of the launches issued while timing was on,
- * measured with HIP events on the context's stream. */
+ * measured with HIP events on the context's stream.  On x-y planes (nz == 1, nx
+ * and ny above 1) the EMF build, its smoothing, the face update and the stage
+ * combination are one launch, booked as HOWMHD_K_COMBINE: EMF2, EMF and FACES
+ * stay 0.  EMF2 is a launch of its own on x-z and y-z grids alone, and grids of
+ * one axis have no EMF and no face launch.  The sweeps of a stage, one launch
+ * otherwise, run one axis at a time while timing is on, so on grids that leave
+ * the device idle the entries add up to more than a step takes without it. */
 enum {
     HOWMHD_K_SWEEP_X = 0, HOWMHD_K_SWEEP_Y, HOWMHD_K_SWEEP_Z, HOWMHD_K_EMF2, HOWMHD_K_EMF,
     HOWMHD_K_FACES, HOWMHD_K_COMBINE, HOWMHD_K_CFL, HOWMHD_K_COUNT
