@@ -29,6 +29,8 @@ def _run(tmp_path, mode, rounds, *flags):
         pytest.skip("sanitizer runtime not available: " + build.stderr[-300:])
     assert build.returncode == 0, build.stderr[-3000:]
     r = subprocess.run([str(exe), mode, str(rounds)], capture_output=True, text=True, timeout=60)
+    if "FATAL: ThreadSanitizer" in r.stderr:  # (a memory layout it does not know)
+        pytest.skip(r.stderr[-300:])
     assert r.returncode == 0 and "WRONG" not in r.stdout, r.stdout[-2000:] + r.stderr[-3000:]
 
 
