@@ -235,7 +235,7 @@ struct SweepAxis {
     // y and z: a plane's tiles, then the blocks along the axis, then the next
     // plane's, so that tiles that share halos along the axis run close in time
     LaunchDiv by_chunk, by_blocks;
-    unsigned first;     // first block of the launch on this axis
+    int first;          // first block on this axis, from the launch's first
     int march;          // consecutive tiles along the axis per block
     long long tile0;    // first tile slot of the axis (queue, statistics)
 };
@@ -276,10 +276,9 @@ struct SweepArgs {
     unsigned* fixctl;
     unsigned* fixhost;
     // the axes of the sweeps in the order of their blocks: y, z, x (an axis
-    // without blocks starts where the next one does), and the first block of
-    // this launch (launch_parts)
+    // without blocks starts where the next one does; one that an earlier launch
+    // began, before block 0, launch_parts)
     SweepAxis<R> ax[3];
-    unsigned block0;
 };
 
 // dF layout per direction: component-major, interface index t = 0..n along the
@@ -974,10 +973,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             A.fixctl[1] = 0u;
         }
     } else {
-        const unsigned b = A.block0 + blockIdx.x;
+        const int b = (int)blockIdx.x;
         if (b >= A.ax[2].first) {
             int bx, by;
-            xcd_row_tiles(b - A.ax[2].first, A.ax[2], bx, by);
+            xcd_row_tiles((unsigned)(b - A.ax[2].first), A.ax[2], bx, by);
             sweep_tiles<R, ALONG_X, MODE, EX, DM, REDO>(A, A.ax[2], raw, bx, by, 1);
         } else {
             // The y and z sweeps are one code (strides) where it marches:
@@ -985,7 +984,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sweep_waves
             // axis: their constants then come straight from the kernel
             // arguments (routed FP32 y/z sweeps at 256^3 444/459 -> 429/445 us).
             auto across = [&](const SweepAxis<R>& X) {
-                const unsigned L = b - X.first, r = div(L, X.by_chunk), hi = div(r, X.by_blocks);
+                const unsigned L = (unsigned)(b - X.first), r = div(L, X.by_chunk), hi = div(r, X.by_blocks);
                 const unsigned bx = hi * X.by_chunk.d + (L - r * X.by_chunk.d), by = r - hi * X.by_blocks.d;
                 if (bx >= X.gx) return;  // the last chunk is short
                 sweep_tiles<R, ACROSS_X, MODE, EX, DM, REDO>(A, X, raw, (int)bx, (int)by * X.march, X.march);
@@ -1019,7 +1018,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
     auto tile = [&](auto tsc, const SweepAxis<R>& X) {
         constexpr int TS = decltype(tsc)::value;
         using T = SweepTile<TS>;
-        const unsigned L = blockIdx.x - X.first, rr = div(L, X.by_gx);
+        const unsigned L = blockIdx.x - (unsigned)X.first, rr = div(L, X.by_gx);
         const int bx = (int)(L - rr * X.gx), by = (int)rr;
         const TileLds<R, TS> lds = tile_lds<R, TS>(raw);
         const int tid = threadIdx.x, l = tid & 63, pass = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1074,8 +1073,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HOWMHD_SWEE
             }
         }
     };
-    if (blockIdx.x >= A.ax[2].first) tile(std::integral_constant<int, ALONG_X_64>{}, A.ax[2]);
-    else tile(std::integral_constant<int, ACROSS_X_64>{}, A.ax[blockIdx.x >= A.ax[1].first ? 1 : 0]);
+    const int b = (int)blockIdx.x;
+    if (b >= A.ax[2].first) tile(std::integral_constant<int, ALONG_X_64>{}, A.ax[2]);
+    else tile(std::integral_constant<int, ACROSS_X_64>{}, A.ax[b >= A.ax[1].first ? 1 : 0]);
 }
 
 template <typename R>

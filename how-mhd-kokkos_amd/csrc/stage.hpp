@@ -74,14 +74,16 @@ inline int march_planes(const dim3& tiles, int nz, int most) {
 // 2^32 threads along x, which 1-D launches of 256 reach at 2^24 blocks: routed
 // tiles are not packed, so a plane of 1 x 8192 x 8192 cells has as many.  (A
 // multiple of 8 keeps the launch's blocks on the XCDs that the tile order means.)
+// A later launch counts its blocks from 0 again and finds the axes' first blocks
+// below them: a block number to add was one more wait at the start of every
+// block (routed FP32 steps of 512^2 248.3 -> 249.4 us).
 constexpr unsigned kLaunchBlocks = 1u << 23;
 template <typename R, typename F>
-void launch_parts(SweepArgs<R>& a, unsigned blocks, const F& launch) {
-    for (unsigned done = 0; done < blocks;) {
-        const unsigned n = std::min(blocks - done, kLaunchBlocks);
-        a.block0 = done;
-        launch(n);
-        done += n;
+void launch_parts(const SweepArgs<R>& a, unsigned blocks, const F& launch) {
+    SweepArgs<R> part = a;
+    for (unsigned done = 0; done < blocks; done += kLaunchBlocks) {
+        for (int k = 0; k < 3; ++k) part.ax[k].first = a.ax[k].first - (int)done;
+        launch(part, std::min(blocks - done, kLaunchBlocks));
     }
 }
 
@@ -162,7 +164,7 @@ SweepArgs<R> sweep_args(howmhd_gpu_ctx* c, int iw, const double* qsrc, unsigned 
             x.by_w = launch_div(W);
             x.by_w5 = launch_div(W + 5);
         }
-        x.first = nb;
+        x.first = (int)nb;
         x.march = 1;
         x.tile0 = c->tile0[d];
         if (d != 0 && sweep_marches<R, MODE>() && !split)
@@ -214,15 +216,15 @@ void launch_sweep(howmhd_gpu_ctx* c, SweepArgs<R>& a, unsigned blocks) {
     const size_t lds = sweep_lds<R, MODE>(a);
     if constexpr (EX && MODE == SW_PLAIN) {
         if (a.ax[0].march == 1 && a.ax[1].march == 1) {
-            launch_parts(a, blocks, [&](unsigned nb) {
-                hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED, true>), dim3(nb), dim3(256), lds, c->stream, a);
+            launch_parts(a, blocks, [&](const SweepArgs<R>& p, unsigned nb) {
+                hipLaunchKernelGGL((k_sweep<R, MODE, EX, DIV_UNSCALED, true>), dim3(nb), dim3(256), lds, c->stream, p);
             });
             return;
         }
     }
     constexpr int DM = EX ? DIV_UNSCALED : DIV_IEEE;
-    launch_parts(a, blocks, [&](unsigned nb) {
-        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DM>), dim3(nb), dim3(256), lds, c->stream, a);
+    launch_parts(a, blocks, [&](const SweepArgs<R>& p, unsigned nb) {
+        hipLaunchKernelGGL((k_sweep<R, MODE, EX, DM>), dim3(nb), dim3(256), lds, c->stream, p);
     });
     if constexpr (EX && MODE != SW_COLLECT) {
         if (blocks) launch_recompute<R, MODE>(c, a);

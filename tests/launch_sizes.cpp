@@ -31,37 +31,37 @@ void record(const char* name, dim3 grid, dim3 block, const A&... args);
 namespace howmhd {
 
 struct Axis {
-    unsigned gx, gy, first, chunk, blocks;
-    int march;
+    unsigned gx, gy, chunk, blocks;
+    int first, march;
 };
 struct Launch {
     std::string name;
     dim3 grid, block;
-    unsigned long long first;
+    unsigned long long first;   // of the launch, from the sweeps' first block
+    std::vector<Axis> axes;     // y, z, x of the sweeps
 };
 static std::vector<Launch> launches;
 // (the reference-rounding form's IEEE-division launch takes its tiles from a queue)
 static bool is_sweep(const Launch& l) {
     return l.name.find("k_sweep") != std::string::npos && !(HOWMHD_EXACT && l.name.find("DIV_IEEE") != std::string::npos);
 }
-static std::vector<Axis> axes;  // y, z, x of the sweeps
 
 template <typename A>
 unsigned long long first_block(const A&, ...) { return 0; }
 template <typename A>
-auto first_block(const A& a, int) -> decltype((unsigned long long)a.block0) { return a.block0; }
+auto first_block(const A& a, int) -> decltype((void)a.ax, 0ull) { return (unsigned long long)-(long long)a.ax[0].first; }
 
 template <typename A>
 void note_axes(const A&, ...) {}
 template <typename A>
 auto note_axes(const A& a, int) -> decltype((void)a.ax) {
-    axes.clear();
-    for (const auto& x : a.ax) axes.push_back({x.gx, x.gy, x.first, x.by_chunk.d, x.by_blocks.d, x.march});
+    for (const auto& x : a.ax)
+        launches.back().axes.push_back({x.gx, x.gy, x.by_chunk.d, x.by_blocks.d, (int)x.first, x.march});
 }
 
 template <typename... A>
 void record(const char* name, dim3 grid, dim3 block, const A&... args) {
-    launches.push_back({name, grid, block, 0});
+    launches.push_back({name, grid, block, 0, {}});
     ((launches.back().first = first_block(args, 0)), ...);
     (note_axes(args, 0), ...);
 }
@@ -70,14 +70,16 @@ void record(const char* name, dim3 grid, dim3 block, const A&... args) {
 static void cover(bool split, const int* n) {
     const int dir[3] = {1, 2, 0};
     std::vector<unsigned char> seen[3];
-    for (int k = 0; k < 3; ++k) seen[k].assign(n[dir[k]] > 1 ? (size_t)axes[k].gx * axes[k].gy : 0, 0);
     for (const Launch& l : launches) {
         if (!is_sweep(l)) continue;
+        const std::vector<Axis>& axes = l.axes;
+        for (int k = 0; k < 3; ++k)
+            if (n[dir[k]] > 1) seen[k].resize((size_t)axes[k].gx * axes[k].gy);
         for (unsigned i = 0; i < l.grid.x; ++i) {
-            const unsigned b = (unsigned)(l.first + i);
+            const int b = (int)i;
             const int k = b >= axes[2].first ? 2 : b >= axes[1].first ? 1 : 0;
             const Axis& x = axes[k];
-            const unsigned L = b - x.first;
+            const unsigned L = (unsigned)(b - x.first);
             auto mark = [&](unsigned bx, unsigned by) {
                 if (bx < x.gx && by < x.gy) seen[k][bx + (size_t)x.gx * by]++;
             };
